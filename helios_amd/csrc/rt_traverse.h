@@ -1,0 +1,1058 @@
+// rt_traverse.h -- BVH traversal and launch helpers shared by the wavefront-persistent ray kernels.
+//
+//   trace_closest   stack traversal of the 64-byte BVH2 (both child boxes per node), LDS stack,
+//                   closest hit with the reference acceptance rule (t > tmin, skip the origin
+//                   primitive; R/shaders/common/bvh_traversal.glsl:68-170) and a canonical tie rule
+//                   (equal t -> lower primitive index) instead of traversal order.
+//   trace_any       occlusion query: any accepted hit with t <= tmax ends the traversal.  The direct
+//                   pass only needs "occluded or not"; with the nearest periodic face as tmax this
+//                   reproduces the reference decision (closest hit vs periodic face) exactly.
+//   k_direct        direct rays (R/shaders/direct_raygen.comp:323-731): one wave per (job, primitive),
+//                   d*d stratified samples, occlusion trace with periodic wrap, compensated sums of
+//                   ray strength split by lit face.
+//   k_diffuse       diffuse/scatter rays (R/shaders/diffuse_raygen.comp:330-560): one wave per
+//                   (pass, primitive), both faces, writes one hit word per ray.
+//   k_gather_*      per-primitive compensated reduction of gathered radiation_out / sky flux over a
+//                   hit table (diffuse_raygen.comp:562-652), deterministic (no atomics).
+//   k_cast          CollisionDetection::castRaysSoA (CD/src/CollisionDetection_RayTracing.cpp:551-680,
+//                   980-1080): one thread per ray, CD predicates, face-forwarded normal.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include <cfloat>
+#include <string>
+
+#include "rt_internal.h"
+
+// 4-wide tree for diffuse rays (1) or the binary tree (0); children of a 4-wide node fully sorted by entry
+// distance (1) or only the nearest taken first (0).  On the 1 M-primitive orchard the binary tree is faster
+// (916 ms per series of 5 passes against 956 sorted and 1021 nearest-first): the 4-wide step needs 112 B of
+// node per lane and more registers (6 instead of 7 waves per SIMD) for ~40 % fewer steps.
+#ifndef RT_DIFFUSE_BVH4
+#define RT_DIFFUSE_BVH4 0
+#endif
+#ifndef RT_DIFFUSE_QBVH4
+#define RT_DIFFUSE_QBVH4 1
+#endif
+#ifndef RT_CAST_QBVH4
+#define RT_CAST_QBVH4 1
+#endif
+#ifndef RT_Q4_EAGER
+#define RT_Q4_EAGER 1
+#endif
+// BVH4 pushes without branches into a spare LDS row per lane (the per-lane stacks then hold LSTK + 1 rows)
+#ifndef RT_PUSH_SPARE
+#define RT_PUSH_SPARE 1
+#endif
+#ifndef RT_BVH4_SORT
+#define RT_BVH4_SORT 1
+#endif
+// 8-bit node steps check the step budget and the link without a branch (the kernel reports a failed lane
+// when it finishes) and test the stack bound only on the pushes that can exceed it: 626 -> 611 ms for the
+// orchard's five diffuse passes
+#ifndef RT_Q4_LATE_ERR
+#define RT_Q4_LATE_ERR 1
+#endif
+#define RT_BUDGET_BAD 0xFFFFFFFFu
+// Diffuse rays take the 8-bit node step with the pop read issued beside the node load and no branch on the
+// hit-child count (611 -> 600 ms for the orchard's five passes); castRays keep the branching step, which is
+// faster for their long rays (3,112 against 2,700 Mrays/s)
+#ifndef RT_Q4_FLAT_DIFFUSE
+#define RT_Q4_FLAT_DIFFUSE 1
+#endif
+
+namespace rt {
+
+__device__ __forceinline__ float min3f(float a, float b, float c) { return fminf(fminf(a, b), c); }
+__device__ __forceinline__ float max3f(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
+
+// traversal work counters (node fetches, primitive tests) of one lane.  The counter type also carries the
+// traversal's flags MK: bit 0 = honour texture masks (off compiles the mask tests away for scenes without
+// masks, keeping the leaf code and its register use as small as before masks existed), bit 1 = watertight
+// intersection predicates instead of the reference's (rt_set_predicates).
+template <int MK>
+struct TCntT {
+    uint32_t nodes, prims;
+    static constexpr bool mask = (MK & RT_FL_MASK) != 0;
+    static constexpr bool wt = (MK & RT_FL_WT) != 0;
+    static constexpr int flags = MK;
+};
+// the same interface with every update compiled away (timed kernels)
+struct NopCounter {
+    __device__ __forceinline__ NopCounter operator++(int) { return *this; }
+    __device__ __forceinline__ NopCounter &operator+=(uint32_t) { return *this; }
+};
+template <int MK>
+struct NoCntT {
+    NopCounter nodes, prims;
+    static constexpr bool mask = (MK & RT_FL_MASK) != 0;
+    static constexpr bool wt = (MK & RT_FL_WT) != 0;
+    static constexpr int flags = MK;
+};
+using TCnt = TCntT<RT_FL_MASK>;
+using NoCnt = NoCntT<RT_FL_MASK>;
+template <bool COUNT, int MK>
+using Cnt = typename std::conditional<COUNT, TCntT<MK>, NoCntT<MK>>::type;
+
+struct RayPre {
+    float ix, iy, iz, ox, oy, oz;
+};
+
+__device__ __forceinline__ RayPre ray_pre(v3f o, v3f d) {
+    RayPre r;
+    r.ix = fabsf(d.x) > 1e-30f ? 1.0f / d.x : 1e30f;
+    r.iy = fabsf(d.y) > 1e-30f ? 1.0f / d.y : 1e30f;
+    r.iz = fabsf(d.z) > 1e-30f ? 1.0f / d.z : 1e30f;
+    r.ox = o.x * r.ix;
+    r.oy = o.y * r.iy;
+    r.oz = o.z * r.iz;
+    return r;
+}
+
+// BVH nodes and primitive records do not change while a trace kernel runs: loading them through the
+// constant address space lets the compiler use scalar loads when the index is wave-uniform (the
+// packet traversal) and ordinary vector loads otherwise.
+__device__ __forceinline__ float4 ldc(const float4 *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(4))) const float cfloat_t;
+    const cfloat_t *q = (const cfloat_t *)(const float *)p;
+    return make_float4(q[0], q[1], q[2], q[3]);
+#else
+    return *p;
+#endif
+}
+
+// wave-uniform copy of a pointer (lets the compiler keep it, and addresses built from uniform
+// indices, in scalar registers)
+template <typename T>
+__device__ __forceinline__ T *uptr(T *p) {
+    uint64_t v = (uint64_t)p;
+    uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (T *)(((uint64_t)hi << 32) | lo);
+}
+
+// Load of a value at a wave-uniform address through the constant address space (scalar load).
+template <typename T>
+__device__ __forceinline__ T ldu(const T *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(4))) const T cT;
+    return *(const cT *)p;
+#else
+    return *p;
+#endif
+}
+
+// Intersect the primitive whose record is at r (recs: the scene's record array, which mask descriptors count
+// from); returns its index and the hit.
+template <bool CD, int MK = RT_FL_MASK>
+__device__ __forceinline__ bool leaf_hit_at(const float4 *r, const float4 *recs, v3f o, v3f d, uint32_t skip,
+                                            uint32_t &id, float &t) {
+    float4 r0 = ldc(r);
+    uint32_t tag = __float_as_uint(r0.w);
+    id = tag & RT_ID_BITS;
+    bool patch = (tag & RT_PATCH_BIT) != 0;
+    const bool masked = (MK & RT_FL_MASK) && !CD && (tag & RT_MASK_BIT) != 0;
+    float4 r1 = ldc(r + 1), r2 = ldc(r + 2);
+    // a voxel is a box that castRays hits (CollisionDetection_RayTracing.cpp:1625-1711) and the radiation
+    // traversal never does (bvh_traversal.glsl:118-140 tests patches, tiles and triangles only)
+    if (CD && (tag & RT_VOXEL_BIT)) return voxel_hit_cd(r0, r1, o, d, t) && id != skip;
+    float4 r3 = (patch || masked) ? ldc(r + 3) : make_float4(0.f, 0.f, 0.f, 0.f);
+    float ua, ub;
+    bool hit = isect_rec_uv<CD, (MK & RT_FL_WT) != 0>(r0, r1, r2, r3, patch, o, d, t, ua, ub) && id != skip &&
+               (CD || !(tag & RT_VOXEL_BIT));
+    // texture mask (bvh_traversal.glsl:143-148): a transparent texel lets the ray pass
+    if (masked && hit) hit = mask_hit_opaque(recs, __float_as_uint(r3.w), patch, ua, ub, r1.w, r2.w);
+    return hit;
+}
+
+// leaf_hit_at() for the primitive in leaf slot k
+template <bool CD, int MK = RT_FL_MASK>
+__device__ __forceinline__ bool leaf_hit_p(const float4 *recs, uint32_t k, v3f o, v3f d, uint32_t skip, uint32_t &id,
+                                           float &t) {
+    return leaf_hit_at<CD, MK>(recs + (size_t)k * 4, recs, o, d, skip, id, t);
+}
+
+template <bool CD, int MK = RT_FL_MASK>
+__device__ __forceinline__ bool leaf_hit(const DevScene &sc, uint32_t k, v3f o, v3f d, uint32_t skip, uint32_t &id,
+                                         float &t) {
+    return leaf_hit_p<CD, MK>(sc.rec, k, o, d, skip, id, t);
+}
+
+template <bool CD, int MK = RT_FL_MASK>
+__device__ __forceinline__ void test_leaf(const float4 *recs, uint32_t k, v3f o, v3f d, float tmin, uint32_t skip,
+                                          float &best_t, uint32_t &best, uint32_t &best_slot) {
+    uint32_t id;
+    float t;
+    // castRays takes a patch or triangle beyond 1e-6 and a voxel at 1e-6 or beyond
+    // (CD/src/CollisionDetection_RayTracing.cpp:1562, 1595, 1681)
+    if (leaf_hit_p<CD, MK>(recs, k, o, d, skip, id, t) &&
+        (t > tmin || (CD && t == tmin && (__float_as_uint(ldc(recs + (size_t)k * 4).w) & RT_VOXEL_BIT)))) {
+        if (t < best_t || (t == best_t && best != RT_MISS && id < best)) {
+            best_t = t;
+            best = id;
+            best_slot = k;
+        }
+    }
+}
+
+// slab tests of both children of node ni against [.., tlim]
+struct NodeTest {
+    float tn0, tn1;
+    uint32_t c0, c1;
+    bool h0, h1;
+};
+
+__device__ __forceinline__ NodeTest node_test_p(const float4 *nodes, uint32_t ni, const RayPre &rp, float tlim);
+
+__device__ __forceinline__ NodeTest node_test(const DevScene &sc, uint32_t ni, const RayPre &rp, float tlim) {
+    return node_test_p(sc.node, ni, rp, tlim);
+}
+
+__device__ __forceinline__ NodeTest node_test_p(const float4 *nodes, uint32_t ni, const RayPre &rp, float tlim) {
+    const float4 *nd = nodes + (size_t)ni * 4;
+    float4 n0 = ldc(nd), n1 = ldc(nd + 1), n2 = ldc(nd + 2), n3 = ldc(nd + 3);
+    float ax = fmaf(n0.x, rp.ix, -rp.ox), bx = fmaf(n0.y, rp.ix, -rp.ox);
+    float ay = fmaf(n0.z, rp.iy, -rp.oy), by = fmaf(n0.w, rp.iy, -rp.oy);
+    float az = fmaf(n1.x, rp.iz, -rp.oz), bz = fmaf(n1.y, rp.iz, -rp.oz);
+    float tn0 = max3f(fminf(ax, bx), fminf(ay, by), fminf(az, bz));
+    float tf0 = min3f(fmaxf(ax, bx), fmaxf(ay, by), fmaxf(az, bz));
+    float cx = fmaf(n1.z, rp.ix, -rp.ox), dx = fmaf(n1.w, rp.ix, -rp.ox);
+    float cy = fmaf(n2.x, rp.iy, -rp.oy), dy = fmaf(n2.y, rp.iy, -rp.oy);
+    float cz = fmaf(n2.z, rp.iz, -rp.oz), dz = fmaf(n2.w, rp.iz, -rp.oz);
+    float tn1 = max3f(fminf(cx, dx), fminf(cy, dy), fminf(cz, dz));
+    float tf1 = min3f(fmaxf(cx, dx), fmaxf(cy, dy), fmaxf(cz, dz));
+    NodeTest r;
+    r.tn0 = tn0;
+    r.tn1 = tn1;
+    // tn <= tf && tf >= 0 && tn <= tlim, as one comparison (tlim >= 0; NaN only ever widens the test)
+    r.h0 = fmaxf(tn0, 0.f) <= fminf(tf0, tlim);
+    r.h1 = fmaxf(tn1, 0.f) <= fminf(tf1, tlim);
+    r.c0 = __float_as_uint(n3.x);
+    r.c1 = __float_as_uint(n3.y);
+    return r;
+}
+
+// Closest accepted hit (t > tmin, t < tstart, ties -> lower primitive index).
+template <bool CD, int STK, typename C>
+__device__ uint32_t trace_closest(const DevScene &sc, v3f o, v3f d, float tmin, uint32_t skip, float tstart,
+                                  float &t_out, uint32_t &slot_out, uint32_t *stk, uint32_t stride, int *err,
+                                  C &cnt) {
+    float best_t = tstart;
+    uint32_t best = RT_MISS, best_slot = RT_MISS;
+    // scene fields in registers: the stack stores below go through a generic pointer, and the compiler
+    // would otherwise reload them from the descriptor on every step
+    const float4 *nodes = sc.node, *recs = sc.rec;
+    const uint32_t nleaf = sc.nleaf;
+    if (nleaf <= 1) {
+        if (nleaf == 1) { cnt.prims++; test_leaf<CD, C::flags>(recs, 0, o, d, tmin, skip, best_t, best, best_slot); }
+        t_out = best_t;
+        slot_out = best_slot;
+        return best;
+    }
+    RayPre rp = ray_pre(o, d);
+    uint32_t ni = 0;
+    int sp = 0;
+    // every internal node is entered at most once per trace; the cap only guards malformed trees
+    uint32_t budget = nleaf + 8;
+    while (true) {
+        if (budget-- == 0 || ni >= nleaf - 1) {
+            atomicOr(err, 2);
+            break;
+        }
+        cnt.nodes++;
+        NodeTest nt = node_test_p(nodes, ni, rp, best_t);
+        bool l0 = (nt.c0 & RT_LEAF_BIT) != 0, l1 = (nt.c1 & RT_LEAF_BIT) != 0;
+        if (nt.h0 && l0) { cnt.prims++; test_leaf<CD, C::flags>(recs, nt.c0 & ~RT_LEAF_BIT, o, d, tmin, skip, best_t, best, best_slot); }
+        if (nt.h1 && l1) { cnt.prims++; test_leaf<CD, C::flags>(recs, nt.c1 & ~RT_LEAF_BIT, o, d, tmin, skip, best_t, best, best_slot); }
+        bool g0 = nt.h0 && !l0, g1 = nt.h1 && !l1;
+        if (g0 && g1) {
+            bool first0 = nt.tn0 <= nt.tn1;
+            if (sp >= STK) {
+                atomicOr(err, 1);
+                break;
+            }
+            stk[(uint32_t)sp * stride] = first0 ? nt.c1 : nt.c0;
+            sp++;
+            ni = first0 ? nt.c0 : nt.c1;
+        } else if (g0) {
+            ni = nt.c0;
+        } else if (g1) {
+            ni = nt.c1;
+        } else {
+            if (sp == 0) break;
+            sp--;
+            ni = stk[(uint32_t)sp * stride];
+        }
+    }
+    t_out = best_t;
+    slot_out = best_slot;
+    return best;
+}
+
+// Any accepted radiation-predicate hit with tmin < t <= tmax?
+template <int STK, typename C>
+__device__ bool trace_any(const DevScene &sc, v3f o, v3f d, float tmin, uint32_t skip, float tmax, uint32_t *stk,
+                          uint32_t stride, int *err, C &cnt) {
+    uint32_t id;
+    float t;
+    const float4 *nodes = sc.node, *recs = sc.rec;
+    const uint32_t nleaf = sc.nleaf;
+    if (nleaf <= 1) {
+        if (nleaf == 1) {
+            cnt.prims++;
+            return leaf_hit_p<false, C::flags>(recs, 0, o, d, skip, id, t) && t > tmin && t <= tmax;
+        }
+        return false;
+    }
+    RayPre rp = ray_pre(o, d);
+    uint32_t ni = 0;
+    int sp = 0;
+    uint32_t budget = nleaf + 8;
+    while (true) {
+        if (budget-- == 0 || ni >= nleaf - 1) {
+            atomicOr(err, 2);
+            return false;
+        }
+        cnt.nodes++;
+        NodeTest nt = node_test_p(nodes, ni, rp, tmax);
+        bool l0 = (nt.c0 & RT_LEAF_BIT) != 0, l1 = (nt.c1 & RT_LEAF_BIT) != 0;
+        if (nt.h0 && l0) {
+            cnt.prims++;
+            if (leaf_hit_p<false, C::flags>(recs, nt.c0 & ~RT_LEAF_BIT, o, d, skip, id, t) && t > tmin && t <= tmax) return true;
+        }
+        if (nt.h1 && l1) {
+            cnt.prims++;
+            if (leaf_hit_p<false, C::flags>(recs, nt.c1 & ~RT_LEAF_BIT, o, d, skip, id, t) && t > tmin && t <= tmax) return true;
+        }
+        bool g0 = nt.h0 && !l0, g1 = nt.h1 && !l1;
+        if (g0 && g1) {
+            bool first0 = nt.tn0 <= nt.tn1;
+            if (sp >= STK) {
+                atomicOr(err, 1);
+                return false;
+            }
+            stk[(uint32_t)sp * stride] = first0 ? nt.c1 : nt.c0;
+            sp++;
+            ni = first0 ? nt.c0 : nt.c1;
+        } else if (g0) {
+            ni = nt.c0;
+        } else if (g1) {
+            ni = nt.c1;
+        } else {
+            if (sp == 0) return false;
+            sp--;
+            ni = stk[(uint32_t)sp * stride];
+        }
+    }
+}
+
+// Wave-coherent any-hit query: the 64 lanes (rays of one primitive towards one source, hence nearly
+// parallel and close together) walk the BVH together.  The node index and the stack are wave-uniform
+// (node fetched once per wave through scalar loads, stack in a per-wave LDS column); every lane tests
+// the child boxes and primitives itself and stops searching at its first accepted hit.  A lane reaches
+// every node whose box chain it intersects, so its answer equals the per-lane traversal's.
+template <int STK, typename C>
+__device__ bool packet_any(const DevScene &sc, v3f o, v3f d, float tmin, uint32_t skip, float tmax, bool active,
+                           uint32_t *wstk, int *err, C &cnt) {
+    bool act = active, found = false;
+    uint32_t id;
+    float t;
+    if (sc.nleaf <= 1) {
+        if (sc.nleaf == 1 && act) {
+            cnt.prims++;
+            found = leaf_hit<false, C::flags>(sc, 0, o, d, skip, id, t) && t > tmin && t <= tmax;
+        }
+        return found;
+    }
+    RayPre rp = ray_pre(o, d);
+    const float4 *nodes = uptr(sc.node), *recs = uptr(sc.rec);
+    const uint32_t nleaf = __builtin_amdgcn_readfirstlane(sc.nleaf);
+    uint32_t ni = 0;
+    uint32_t sp = 0;
+    uint32_t budget = nleaf + 8;
+    while (__ballot(act) != 0) {
+        ni = __builtin_amdgcn_readfirstlane(ni);
+        if (budget-- == 0 || ni >= nleaf - 1) {
+            atomicOr(err, 2);
+            break;
+        }
+        if (act) cnt.nodes++;  // per-ray visits (one fetch serves the whole wave)
+        NodeTest nt = node_test_p(nodes, ni, rp, tmax);
+        uint32_t c0 = __builtin_amdgcn_readfirstlane(nt.c0), c1 = __builtin_amdgcn_readfirstlane(nt.c1);
+        nt.c0 = c0;
+        nt.c1 = c1;
+        bool l0 = (nt.c0 & RT_LEAF_BIT) != 0, l1 = (nt.c1 & RT_LEAF_BIT) != 0;
+        bool h0 = act && nt.h0, h1 = act && nt.h1;
+        if (l0 && h0) {
+            cnt.prims++;
+            if (leaf_hit_p<false, C::flags>(recs, nt.c0 & ~RT_LEAF_BIT, o, d, skip, id, t) && t > tmin && t <= tmax) {
+                found = true;
+                act = false;
+            }
+        }
+        if (l1 && h1 && act) {
+            cnt.prims++;
+            if (leaf_hit_p<false, C::flags>(recs, nt.c1 & ~RT_LEAF_BIT, o, d, skip, id, t) && t > tmin && t <= tmax) {
+                found = true;
+                act = false;
+            }
+        }
+        bool g0 = !l0 && __ballot(h0 && act) != 0;
+        bool g1 = !l1 && __ballot(h1 && act) != 0;
+        if (g0 && g1) {
+            // nearer child first, as seen by the wave's first still-searching lane
+            uint64_t m = __ballot(act && nt.tn0 <= nt.tn1);
+            uint64_t a = __ballot(act);
+            bool first0 = (m & (a & (~a + 1))) != 0;
+            if (sp >= STK) {
+                atomicOr(err, 1);
+                break;
+            }
+            wstk[sp] = first0 ? nt.c1 : nt.c0;  // same value from every lane
+            sp++;
+            ni = first0 ? nt.c0 : nt.c1;
+        } else if (g0) {
+            ni = nt.c0;
+        } else if (g1) {
+            ni = nt.c1;
+        } else {
+            if (sp == 0) break;
+            sp--;
+            ni = wstk[sp];
+        }
+    }
+    return found;
+}
+
+// Slab test of one child box of a BVH4 node.
+__device__ __forceinline__ void slab4(float lx, float hx, float ly, float hy, float lz, float hz, const RayPre &rp,
+                                      float &tn, float &tf) {
+    float ax = fmaf(lx, rp.ix, -rp.ox), bx = fmaf(hx, rp.ix, -rp.ox);
+    float ay = fmaf(ly, rp.iy, -rp.oy), by = fmaf(hy, rp.iy, -rp.oy);
+    float az = fmaf(lz, rp.iz, -rp.oz), bz = fmaf(hz, rp.iz, -rp.oz);
+    tn = max3f(fminf(ax, bx), fminf(ay, by), fminf(az, bz));
+    tf = min3f(fmaxf(ax, bx), fmaxf(ay, by), fmaxf(az, bz));
+}
+
+// Ascending compare-exchange of two (key, link) pairs held in scalar registers.
+__device__ __forceinline__ void cswap(float &ka, uint32_t &la, float &kb, uint32_t &lb) {
+    bool sw = kb < ka;
+    float k = sw ? kb : ka;
+    uint32_t l = sw ? lb : la;
+    kb = sw ? ka : kb;
+    lb = sw ? la : lb;
+    ka = k;
+    la = l;
+}
+
+// packet_any() on the BVH4: one 128-byte node per step (two scalar loads), four child boxes tested by every
+// lane.  Leaf children are tested by the lanes whose box test passed; internal children hit by any still
+// searching lane are visited nearest-first as seen by the wave's first searching lane (a sorting network on
+// at most four scalar keys), the others pushed on the per-wave LDS stack.  A lane still reaches every node
+// whose box chain it intersects, so each lane's answer equals the single-ray traversal's.
+#define RT_WSTK4 128
+template <typename C>
+__device__ bool packet_any4(const DevScene &sc, v3f o, v3f d, float tmin, uint32_t skip, float tmax, bool active,
+                            uint32_t *wstk, int *err, C &cnt) {
+    bool act = active, found = false;
+    uint32_t id;
+    float t;
+    if (sc.nleaf <= 1) {
+        if (sc.nleaf == 1 && act) {
+            cnt.prims++;
+            found = leaf_hit<false, C::flags>(sc, 0, o, d, skip, id, t) && t > tmin && t <= tmax;
+        }
+        return found;
+    }
+    RayPre rp = ray_pre(o, d);
+    const float4 *nodes = uptr(sc.node4), *recs = uptr(sc.rec);
+    const uint32_t nn4 = __builtin_amdgcn_readfirstlane(sc.nnode4);
+    uint32_t ni = 0, sp = 0;
+    uint32_t budget = nn4 + 8;
+    while (__ballot(act) != 0) {
+        ni = __builtin_amdgcn_readfirstlane(ni);
+        if (budget-- == 0 || ni >= nn4) {
+            atomicOr(err, 2);
+            break;
+        }
+        if (act) cnt.nodes++;
+        const float4 *nd = nodes + (size_t)ni * 8;
+        const float4 lx = ldc(nd), hx = ldc(nd + 1), ly = ldc(nd + 2), hy = ldc(nd + 3);
+        const float4 lz = ldc(nd + 4), hz = ldc(nd + 5), lk = ldc(nd + 6);
+        uint32_t lnk[4];
+        lnk[0] = __builtin_amdgcn_readfirstlane(__float_as_uint(lk.x));
+        lnk[1] = __builtin_amdgcn_readfirstlane(__float_as_uint(lk.y));
+        lnk[2] = __builtin_amdgcn_readfirstlane(__float_as_uint(lk.z));
+        lnk[3] = __builtin_amdgcn_readfirstlane(__float_as_uint(lk.w));
+        float tn[4], tf[4];
+        slab4(lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, rp, tn[0], tf[0]);
+        slab4(lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, rp, tn[1], tf[1]);
+        slab4(lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, rp, tn[2], tf[2]);
+        slab4(lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, rp, tn[3], tf[3]);
+        bool h[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) h[k] = fmaxf(tn[k], 0.f) <= fminf(tf[k], tmax);  // unused slots never pass
+        // leaf children: a wave-uniform branch per leaf, the test itself predicated per lane
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (lnk[k] & RT_LEAF_BIT) {
+                const bool want = h[k] && act;
+                if (__ballot(want) != 0) {
+                    cnt.prims += want ? 1u : 0u;
+                    const bool hit = leaf_hit_p<false, C::flags>(recs, lnk[k] & ~RT_LEAF_BIT, o, d, skip, id, t) && t > tmin &&
+                                     t <= tmax;
+                    const bool take = want && hit;
+                    found = found || take;
+                    act = act && !take;
+                }
+            }
+        }
+        const uint64_t am = __ballot(act);
+        if (am == 0) break;
+        const uint32_t leader = (uint32_t)__builtin_ctzll(am);
+        // internal children some searching lane hits, keyed by the leader's entry distance
+        float key[4];
+        uint32_t lk4[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            bool inner = !(lnk[k] & RT_LEAF_BIT);
+            bool any = inner && __ballot(h[k] && act) != 0;
+            const int kk = __builtin_amdgcn_readlane(__float_as_int(h[k] ? tn[k] : 3.0e38f), (int)leader);
+            key[k] = any ? __int_as_float(kk) : INFINITY;
+            lk4[k] = any ? lnk[k] : 0xFFFFFFFFu;
+        }
+        cswap(key[0], lk4[0], key[1], lk4[1]);
+        cswap(key[2], lk4[2], key[3], lk4[3]);
+        cswap(key[0], lk4[0], key[2], lk4[2]);
+        cswap(key[1], lk4[1], key[3], lk4[3]);
+        cswap(key[1], lk4[1], key[2], lk4[2]);
+        const uint32_t m = (lk4[0] != 0xFFFFFFFFu) + (lk4[1] != 0xFFFFFFFFu) + (lk4[2] != 0xFFFFFFFFu) +
+                           (lk4[3] != 0xFFFFFFFFu);
+        if (m == 0) {
+            if (sp == 0) break;
+            sp--;
+            ni = wstk[sp];
+        } else {
+            if (sp + m - 1 > RT_WSTK4) {
+                atomicOr(err, 1);
+                break;
+            }
+            if (m >= 4) wstk[sp++] = lk4[3];
+            if (m >= 3) wstk[sp++] = lk4[2];
+            if (m >= 2) wstk[sp++] = lk4[1];
+            ni = lk4[0];
+        }
+    }
+    return found;
+}
+
+// R/shaders/common/periodic_boundary.glsl:28-59
+__device__ __forceinline__ float isect_bbox_face(const BBoxFace &f, v3f o, v3f d) {
+    v3f n = mk3(f.n[0], f.n[1], f.n[2]);
+    v3f v0 = mk3(f.v0[0], f.v0[1], f.v0[2]);
+    float denom = dot3(d, n);
+    if (fabsf(denom) < 1e-8f) return -1.0f;
+    float t = rdiv(dot3(sub3(v0, o), n), denom);
+    if (t <= 1e-5f || t > 1e8f) return -1.0f;
+    v3f p = add3(o, mul3(d, t));
+    v3f dd = sub3(p, v0);
+    float da = dot3(dd, mk3(f.a[0], f.a[1], f.a[2]));
+    float db = dot3(dd, mk3(f.b[0], f.b[1], f.b[2]));
+    if (da > 0.0f && da < f.aa && db > 0.0f && db < f.bb) return t;
+    return -1.0f;
+}
+
+// nearest periodic face strictly below tlim (periodic_boundary.glsl:84-92); returns its t or -1
+__device__ __forceinline__ float nearest_face(const DevScene &sc, v3f o, v3f d, float tlim) {
+    float bt = tlim;
+    int cf = -1;
+    for (uint32_t f = 0; f < sc.nbbox; f++) {
+        float t = isect_bbox_face(sc.bbox[f], o, d);
+        if (t > 0.0f && t < bt) { bt = t; cf = (int)f; }
+    }
+    return cf < 0 ? -1.0f : bt;
+}
+
+// wrapped origin for a face hit at distance bt (periodic_boundary.glsl:94-111)
+__device__ __forceinline__ v3f wrap_at(const DevScene &sc, v3f o, v3f d, float bt) {
+    v3f hp = add3(o, mul3(d, bt));
+    const float eps = 1e-5f;
+    float wx = sc.dom[1] - sc.dom[0], wy = sc.dom[3] - sc.dom[2];
+    v3f w = hp;
+    if (sc.px && fabsf(hp.x - sc.dom[0]) <= eps) w.x += wx - eps;
+    else if (sc.px && fabsf(hp.x - sc.dom[1]) <= eps) w.x -= wx - eps;
+    else if (sc.py && fabsf(hp.y - sc.dom[2]) <= eps) w.y += wy - eps;
+    else if (sc.py && fabsf(hp.y - sc.dom[3]) <= eps) w.y -= wy - eps;
+    return w;
+}
+
+// Closest-hit trace with up to 32 periodic wraps (diffuse_raygen.comp:498-560 without translucent
+// covers).  Returns the last traversal result.
+template <int STK, typename C>
+__device__ __forceinline__ uint32_t trace_loop(const DevScene &sc, v3f o, v3f d, float tmin, uint32_t skip,
+                                               bool &exhausted, uint32_t *stk, uint32_t stride, int *err, C &cnt) {
+    uint32_t hit = RT_MISS;
+    v3f cur = o;
+    exhausted = true;
+    for (int step = 0; step < 32; ++step) {
+        float t;
+        uint32_t slot;
+        hit = trace_closest<false, STK>(sc, cur, d, tmin, skip, 1e30f, t, slot, stk, stride, err, cnt);
+        if (sc.nbbox) {
+            float bt = nearest_face(sc, cur, d, t);
+            if (bt > 0.f) { cur = wrap_at(sc, cur, d, bt); continue; }
+        }
+        exhausted = false;
+        break;
+    }
+    return hit;
+}
+
+// Occlusion towards a collimated source with periodic wraps (direct_raygen.comp:603-672 without
+// translucent covers).  The reference wraps when the nearest periodic face is strictly closer than
+// the closest hit, and is occluded otherwise if anything was hit; "some hit with t <= t_face" is the
+// same decision, so an any-hit query suffices.  32 wraps without resolution count as unoccluded.
+template <int STK, typename C>
+__device__ __forceinline__ bool occluded(const DevScene &sc, v3f o, v3f d, float tmin, uint32_t skip, uint32_t *stk,
+                                         uint32_t stride, int *err, C &cnt) {
+    v3f cur = o;
+    for (int step = 0; step < 32; ++step) {
+        float tf = sc.nbbox ? nearest_face(sc, cur, d, 1e30f) : -1.0f;
+        float tmax = tf > 0.f ? tf : 1e30f;
+        if (trace_any<STK>(sc, cur, d, tmin, skip, tmax, stk, stride, err, cnt)) return true;
+        if (tf <= 0.f) return false;
+        cur = wrap_at(sc, cur, d, tf);
+    }
+    return false;
+}
+
+// occluded() for a whole wave with packet_any4() (packet_any() when the scene has no usable BVH4); each
+// lane keeps its own wrap state.
+template <int STK, typename C>
+__device__ __forceinline__ bool packet_occluded(const DevScene &sc, v3f o, v3f d, float tmin, uint32_t skip,
+                                                bool active, uint32_t *wstk, uint32_t *wstk4, int *err, C &cnt) {
+    v3f cur = o;
+    bool need = active, occl = false;
+    for (int step = 0; step < 32; ++step) {
+        if (__ballot(need) == 0) break;
+        float tf = (need && sc.nbbox) ? nearest_face(sc, cur, d, 1e30f) : -1.0f;
+        float tmax = tf > 0.f ? tf : 1e30f;
+        bool f = sc.node4 ? packet_any4(sc, cur, d, tmin, skip, tmax, need, wstk4, err, cnt)
+                          : packet_any<STK>(sc, cur, d, tmin, skip, tmax, need, wstk, err, cnt);
+        if (need) {
+            if (f) { occl = true; need = false; }
+            else if (tf <= 0.f) need = false;
+            else cur = wrap_at(sc, cur, d, tf);
+        }
+    }
+    return occl;
+}
+
+// Next work item of this wave.  No lane-divergent branch around the fetch: every lane issues the
+// atomic (lane 0 adds 1, the others 0) and lane 0's old value is broadcast as a scalar.  A
+// `if (lane == 0) atomicAdd` + shuffle lets the compiler split the persistent loop into a lane-0
+// loop and a lanes-1..63 loop that re-processes item 0 forever.
+__device__ __forceinline__ uint32_t wave_item(uint32_t *counter, uint32_t chunk) {
+    uint32_t lane = threadIdx.x & 63;
+    uint32_t item = atomicAdd(counter, lane == 0 ? chunk : 0u);
+    return __builtin_amdgcn_readfirstlane(item);
+}
+
+template <typename J>
+__device__ __forceinline__ uint32_t find_job(const J *jobs, uint32_t njobs, uint32_t item) {
+    uint32_t lo = 0, hi = njobs;  // last job with item_begin <= item
+    while (hi - lo > 1) {
+        uint32_t mid = (lo + hi) >> 1;
+        if (jobs[mid].item_begin <= item) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+    for (int off = 32; off >= 1; off >>= 1) v += (uint32_t)__shfl_xor((int)v, off, 64);
+    return v;
+}
+
+// Sum of k rays of strength s, each added once: k s is exact in double (k < 2^24), then rounded to float.
+__device__ __forceinline__ float lit_sum(uint32_t k, float s) { return (float)((double)k * (double)s); }
+
+__device__ __forceinline__ void wave_reduce(ksum &k) {
+    for (int off = 32; off >= 1; off >>= 1) {
+        float os = __shfl_xor(k.s, off, 64);
+        float oc = __shfl_xor(k.c, off, 64);
+        k.merge(os, oc);
+    }
+}
+
+__device__ __forceinline__ bool traced_type(uint32_t t) { return t == 0 || t == 1 || t == 3; }
+
+template <int MK>
+__device__ __forceinline__ void add_stats(unsigned long long *, const NoCntT<MK> &, uint32_t) {}
+template <int MK>
+__device__ __forceinline__ void add_stats(unsigned long long *stats, const TCntT<MK> &c, uint32_t rays) {
+    if (stats) {
+        atomicAdd(&stats[0], (unsigned long long)c.nodes);
+        atomicAdd(&stats[1], (unsigned long long)c.prims);
+        atomicAdd(&stats[2], (unsigned long long)rays);
+    }
+}
+
+// lanes still traversing below which a wave hands out new rays; lanes waiting at a leaf that start a leaf phase;
+// stack entries of the resumable traversals kept in LDS (the rest in private memory)
+#ifndef RT_REFILL_BELOW
+#define RT_REFILL_BELOW 48
+#endif
+#ifndef RT_LEAF_BATCH
+#define RT_LEAF_BATCH 16
+#endif
+#ifndef RT_DIFFUSE_LDS_STACK
+#define RT_DIFFUSE_LDS_STACK 16
+#endif
+
+// Resumable closest-hit traversal state of one lane (BVH2), for kernels that refill finished lanes.
+struct LaneRay {
+    v3f o, d;
+    RayPre rp;
+    float best_t;
+    uint32_t best, ni, budget;
+    int sp;
+};
+
+__device__ __forceinline__ void lane_start(LaneRay &L, uint32_t nleaf) {
+    L.rp = ray_pre(L.o, L.d);
+    L.best_t = 1e30f;
+    L.best = RT_MISS;
+    L.ni = 0;
+    L.sp = 0;
+    L.budget = nleaf + 8;
+}
+
+// Starts the closest-hit trace of L.o, L.d; returns false when it is already complete (a scene with at
+// most one traced primitive needs no node steps), as trace_closest() with tstart = 1e30.
+template <typename C>
+__device__ __forceinline__ bool lane_begin(LaneRay &L, const float4 *recs, uint32_t nleaf, float tmin, uint32_t skip,
+                                           C &cnt) {
+    lane_start(L, nleaf);
+    if (nleaf > 1) return true;
+    uint32_t slot_unused;
+    if (nleaf == 1) { cnt.prims++; test_leaf<false, C::flags>(recs, 0, L.o, L.d, tmin, skip, L.best_t, L.best, slot_unused); }
+    return false;
+}
+
+// LDS pointer: accesses compile to ds_read/ds_write (a generic pointer chosen between LDS and private
+// memory would compile to slower flat accesses that also wait on vector memory)
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+#else
+typedef uint32_t lds_u32;
+#endif
+
+// Traversal entries are inner nodes or leaves (RT_LEAF_BIT).  The stack holds its first LSTK entries in
+// LDS (stk, lane stride `stride`) and the rest, up to STK, in the lane's private array ovf (deep stacks
+// are rare; LDS per wave bounds the occupancy).  lane_pop() returns true when the stack is empty.
+template <int STK, int LSTK>
+__device__ __forceinline__ bool lane_pop(LaneRay &L, const lds_u32 *stk, const uint32_t *ovf, uint32_t stride) {
+    if (L.sp == 0) return true;
+    L.sp--;
+    if (LSTK >= STK || L.sp < LSTK) L.ni = stk[(uint32_t)L.sp * stride];
+    else L.ni = ovf[L.sp - LSTK];
+    return false;
+}
+
+// Visit the inner node L.ni: both child boxes against [0, best_t]; the nearer hit child (inner or leaf)
+// becomes the next entry and the farther one is pushed.  Returns true when the traversal has ended.
+template <int STK, int LSTK, typename C>
+__device__ __forceinline__ bool lane_node(const float4 *nodes, uint32_t nleaf, LaneRay &L, lds_u32 *stk, uint32_t *ovf,
+                                          uint32_t stride, int *err, C &cnt) {
+    if (L.budget-- == 0 || L.ni >= nleaf - 1) {
+        atomicOr(err, 2);
+        return true;
+    }
+    cnt.nodes++;
+    NodeTest nt = node_test_p(nodes, L.ni, L.rp, L.best_t);
+    if (nt.h0 && nt.h1) {
+        bool first0 = nt.tn0 <= nt.tn1;
+        if (L.sp >= STK) {
+            atomicOr(err, 1);
+            return true;
+        }
+        const uint32_t far = first0 ? nt.c1 : nt.c0;
+        if (LSTK >= STK || L.sp < LSTK) stk[(uint32_t)L.sp * stride] = far;
+        else ovf[L.sp - LSTK] = far;
+        L.sp++;
+        L.ni = first0 ? nt.c0 : nt.c1;
+    } else if (nt.h0) {
+        L.ni = nt.c0;
+    } else if (nt.h1) {
+        L.ni = nt.c1;
+    } else {
+        return lane_pop<STK, LSTK>(L, stk, ovf, stride);
+    }
+    return false;
+}
+
+// The hit children of a BVH4 visit (key = entry distance, +inf = missed): the nearest becomes the next
+// entry and the others are pushed (farthest first with RT_BVH4_SORT, else in slot order); the stack empty
+// after no hit ends the traversal (returns true), as does a stack overflow (error bit 1).
+template <int STK, int LSTK>
+__device__ __forceinline__ bool node4_order(LaneRay &L, float *key, uint32_t *lnk, uint32_t nhit, lds_u32 *stk,
+                                            uint32_t *ovf, uint32_t stride, int *err) {
+    if (nhit == 0) return lane_pop<STK, LSTK>(L, stk, ovf, stride);
+#if RT_BVH4_SORT
+    // ascending sort of the four (key, link) pairs; missed children (key +inf) end up last
+    cswap(key[0], lnk[0], key[1], lnk[1]);
+    cswap(key[2], lnk[2], key[3], lnk[3]);
+    cswap(key[0], lnk[0], key[2], lnk[2]);
+    cswap(key[1], lnk[1], key[3], lnk[3]);
+    cswap(key[1], lnk[1], key[2], lnk[2]);
+#if !RT_Q4_LATE_ERR
+    if ((uint32_t)L.sp + nhit - 1 > (uint32_t)STK) {
+        atomicOr(err, 1);
+        return true;
+    }
+#endif
+#if RT_PUSH_SPARE
+    // (with the stack bound tested after this path, the path needs sp + 3 <= LSTK even when LSTK >= STK)
+    if ((!RT_Q4_LATE_ERR && LSTK >= STK) || (uint32_t)L.sp + 3u <= (uint32_t)LSTK) {
+        // every slot a push may use is in LDS: three stores without branches, those beyond the pushed
+        // children aimed at the lane's spare row (index LSTK, which nothing reads); child k < nhit goes to
+        // slot sp + nhit - 1 - k, so the farthest lies deepest and child 1 on top
+#pragma unroll
+        for (int k = 3; k >= 1; k--) {
+            const uint32_t at = (uint32_t)k < nhit ? (uint32_t)L.sp + nhit - 1u - (uint32_t)k : (uint32_t)LSTK;
+            stk[at * stride] = lnk[k];
+        }
+        L.sp += (int)nhit - 1;
+        L.ni = lnk[0];
+        return false;
+    }
+#endif
+#if RT_Q4_LATE_ERR
+    // (the branch-free pushes above cannot overflow: sp + 3 <= LSTK <= STK)
+    if ((uint32_t)L.sp + nhit - 1 > (uint32_t)STK) {
+        atomicOr(err, 1);
+        return true;
+    }
+#endif
+#pragma unroll
+    for (int k = 3; k >= 1; k--) {
+        if ((uint32_t)k < nhit) {
+            if (LSTK >= STK || L.sp < LSTK) stk[(uint32_t)L.sp * stride] = lnk[k];
+            else ovf[L.sp - LSTK] = lnk[k];
+            L.sp++;
+        }
+    }
+    L.ni = lnk[0];
+    return false;
+#else
+    // the nearest hit child next; the other hit children pushed in slot order
+    int m = 0;
+    float km = key[0];
+#pragma unroll
+    for (int k = 1; k < 4; k++)
+        if (key[k] < km) { km = key[k]; m = k; }
+    if ((uint32_t)L.sp + nhit - 1 > (uint32_t)STK) {
+        atomicOr(err, 1);
+        return true;
+    }
+    uint32_t next = lnk[0];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        if (k == m) next = lnk[k];
+        else if (key[k] < INFINITY) {
+            if (LSTK >= STK || L.sp < LSTK) stk[(uint32_t)L.sp * stride] = lnk[k];
+            else ovf[L.sp - LSTK] = lnk[k];
+            L.sp++;
+        }
+    }
+    L.ni = next;
+    return false;
+#endif
+}
+
+// Visit the BVH4 node L.ni: four child boxes against [0, best_t]; the hit children (inner nodes or leaves)
+// in ascending entry distance -- the nearest becomes the next entry, the others are pushed farthest first.
+// Unused slots are +inf point boxes that never pass the test.  Returns true when the traversal has ended.
+template <int STK, int LSTK, typename C>
+__device__ __forceinline__ bool lane_node4(const float4 *nodes4, uint32_t nn4, LaneRay &L, lds_u32 *stk, uint32_t *ovf,
+                                           uint32_t stride, int *err, C &cnt) {
+    if (L.budget-- == 0 || L.ni >= nn4) {
+        atomicOr(err, 2);
+        return true;
+    }
+    cnt.nodes++;
+    const float4 *nd = nodes4 + (size_t)L.ni * 8;
+    const float4 lx = ldc(nd), hx = ldc(nd + 1), ly = ldc(nd + 2), hy = ldc(nd + 3);
+    const float4 lz = ldc(nd + 4), hz = ldc(nd + 5), lk = ldc(nd + 6);
+    float tn[4], tf[4];
+    slab4(lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, L.rp, tn[0], tf[0]);
+    slab4(lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, L.rp, tn[1], tf[1]);
+    slab4(lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, L.rp, tn[2], tf[2]);
+    slab4(lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, L.rp, tn[3], tf[3]);
+    float key[4];
+    uint32_t lnk[4] = {__float_as_uint(lk.x), __float_as_uint(lk.y), __float_as_uint(lk.z), __float_as_uint(lk.w)};
+    uint32_t nhit = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const bool h = fmaxf(tn[k], 0.f) <= fminf(tf[k], L.best_t);
+        key[k] = h ? tn[k] : INFINITY;
+        nhit += h ? 1u : 0u;
+    }
+    return node4_order<STK, LSTK>(L, key, lnk, nhit, stk, ovf, stride, err);
+}
+
+// Visit the 8-bit BVH4 node L.ni (64 B: see k_q4 in rt_scene.hip).  A child bound q decodes in t-space as
+// (o + q 2^e - ray origin) / dir = q (2^e / dir) + (o - ray origin) / dir: one convert and one fma per bound
+// after a multiply and an fma per axis.  The decoded boxes contain the float boxes, and the t rounding is a
+// few ulps of the scene scale, far inside the leaf boxes' padding, so no ray a float box passes is culled
+// and the hits are those of the float trees.
+__device__ __forceinline__ float qbyte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xFFu); }
+
+template <int STK, int LSTK, bool FLAT, typename C>
+__device__ __forceinline__ bool lane_node4q(const float4 *q4, uint32_t nn4, LaneRay &L, lds_u32 *stk, uint32_t *ovf,
+                                            uint32_t stride, int *err, C &cnt) {
+#if RT_Q4_LATE_ERR
+    // a spent step budget or a link outside the tree ends the trace without a branch: the read goes to
+    // node 0 and the budget becomes RT_BUDGET_BAD, which the kernel reports when the lane finishes
+    const bool bad = L.budget == 0u || L.ni >= nn4;
+    L.budget = bad ? RT_BUDGET_BAD : L.budget - 1u;
+    const uint32_t ni = bad ? 0u : L.ni;
+#else
+    if (L.budget-- == 0 || L.ni >= nn4) {
+        atomicOr(err, 2);
+        return true;
+    }
+    const uint32_t ni = L.ni;
+    constexpr bool bad = false;
+#endif
+    cnt.nodes++;
+    const float4 *nd = q4 + (size_t)ni * 4;
+    const float4 f0 = ldc(nd), f1 = ldc(nd + 1), f2 = ldc(nd + 2), f3 = ldc(nd + 3);
+    // FLAT: the entry a pop would take is read now, so its latency hides under the node's (a lane whose
+    // stack top is not in LDS reads its spare row and takes the general path below)
+    const uint32_t sp0 = (uint32_t)L.sp;
+    uint32_t popv = 0u;
+    if (FLAT) popv = stk[((sp0 != 0u && sp0 <= (uint32_t)LSTK) ? sp0 - 1u : (uint32_t)LSTK) * stride];
+    const uint32_t meta = __float_as_uint(f0.w);
+    const uint32_t nch = meta >> 24;
+    // 2^e as a float from the biased exponent byte (e + 127 in [1, 254])
+    const float sx = __uint_as_float((meta & 0xFFu) << 23), sy = __uint_as_float(((meta >> 8) & 0xFFu) << 23),
+                sz = __uint_as_float(((meta >> 16) & 0xFFu) << 23);
+    const float Ax = sx * L.rp.ix, Ay = sy * L.rp.iy, Az = sz * L.rp.iz;
+    const float Bx = fmaf(f0.x, L.rp.ix, -L.rp.ox), By = fmaf(f0.y, L.rp.iy, -L.rp.oy),
+                Bz = fmaf(f0.z, L.rp.iz, -L.rp.oz);
+#if RT_Q4_EAGER
+    // keep the link words' load beside the box words' (the compiler would otherwise sink it into the
+    // branch that pushes, a second dependent round trip per step)
+    asm volatile("" ::"v"(f2.z), "v"(f2.w), "v"(f3.x), "v"(f3.y));
+#endif
+    const uint32_t wlx = __float_as_uint(f1.x), whx = __float_as_uint(f1.y), wly = __float_as_uint(f1.z),
+                   why = __float_as_uint(f1.w), wlz = __float_as_uint(f2.x), whz = __float_as_uint(f2.y);
+    float key[4];
+    uint32_t lnk[4] = {__float_as_uint(f2.z), __float_as_uint(f2.w), __float_as_uint(f3.x), __float_as_uint(f3.y)};
+    uint32_t nhit = 0;
+    // per axis, the bound word nearer the origin: the lower bounds when the direction is positive (A > 0:
+    // t rises with q), else the upper ones.  t(near) = min(t(lo), t(hi)) exactly, so the entry and exit
+    // distances equal the min/max form's with one select per axis instead of a min and a max per child.
+    const bool sx_pos = L.rp.ix >= 0.f, sy_pos = L.rp.iy >= 0.f, sz_pos = L.rp.iz >= 0.f;
+    const uint32_t nwx = sx_pos ? wlx : whx, fwx = sx_pos ? whx : wlx;
+    const uint32_t nwy = sy_pos ? wly : why, fwy = sy_pos ? why : wly;
+    const uint32_t nwz = sz_pos ? wlz : whz, fwz = sz_pos ? whz : wlz;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float tn = max3f(fmaf(qbyte(nwx, k), Ax, Bx), fmaf(qbyte(nwy, k), Ay, By), fmaf(qbyte(nwz, k), Az, Bz));
+        const float tf = min3f(fmaf(qbyte(fwx, k), Ax, Bx), fmaf(qbyte(fwy, k), Ay, By), fmaf(qbyte(fwz, k), Az, Bz));
+        const bool h = (uint32_t)k < nch && fmaxf(tn, 0.f) <= fminf(tf, L.best_t);
+        key[k] = h ? tn : INFINITY;
+        nhit += h ? 1u : 0u;
+    }
+    if (FLAT && sp0 + 3u <= (uint32_t)LSTK) {
+        // no branch on the number of hit children: the sorted children are pushed into the rows above the
+        // stack top (those beyond the hit children into the spare row), and the next entry is the nearest
+        // hit child or, with none, the popped entry; the pushes write rows >= sp0, never the one popped
+        cswap(key[0], lnk[0], key[1], lnk[1]);
+        cswap(key[2], lnk[2], key[3], lnk[3]);
+        cswap(key[0], lnk[0], key[2], lnk[2]);
+        cswap(key[1], lnk[1], key[3], lnk[3]);
+        cswap(key[1], lnk[1], key[2], lnk[2]);
+#pragma unroll
+        for (int k = 3; k >= 1; k--) {
+            const uint32_t at = (uint32_t)k < nhit ? sp0 + nhit - 1u - (uint32_t)k : (uint32_t)LSTK;
+            stk[at * stride] = lnk[k];
+        }
+        L.ni = nhit != 0u ? lnk[0] : popv;
+        L.sp = (int)(nhit != 0u ? sp0 + nhit - 1u : (sp0 != 0u ? sp0 - 1u : 0u));
+        return (nhit == 0u && sp0 == 0u) || bad;
+    }
+#if RT_Q4_LATE_ERR
+    return node4_order<STK, LSTK>(L, key, lnk, nhit, stk, ovf, stride, err) || bad;
+#else
+    return node4_order<STK, LSTK>(L, key, lnk, nhit, stk, ovf, stride, err);
+#endif
+}
+
+// Test the leaf entry L.ni (closest accepted hit, ties to the lower primitive index), then pop.
+template <int STK, int LSTK, typename C>
+__device__ __forceinline__ bool lane_leaf(const float4 *recs, LaneRay &L, float tmin, uint32_t skip,
+                                          const lds_u32 *stk, const uint32_t *ovf, uint32_t stride, C &cnt) {
+    cnt.prims++;
+    uint32_t slot_unused;
+    test_leaf<false, C::flags>(recs, L.ni & ~RT_LEAF_BIT, L.o, L.d, tmin, skip, L.best_t, L.best, slot_unused);
+    return lane_pop<STK, LSTK>(L, stk, ovf, stride);
+}
+
+// The result does not depend on the visiting order: a primitive hit at t <= the final closest t lies in
+// boxes whose entry distance is <= t <= every intermediate best_t, so no step culls it, and the tie rule
+// is order-free.  The entries visited equal trace_closest()'s up to that order.
+
+static __global__ void k_zero_u64(unsigned long long *p) { *p = 0ull; }
+
+static __global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
+
+// ------------------------------------------------------------------------------------------------
+// launchers
+// ------------------------------------------------------------------------------------------------
+static inline uint32_t grid_for(const LaunchCfg &cfg, int ncu, uint32_t total, uint32_t wpb) {
+    uint64_t g = (uint64_t)cfg.blocks_per_cu * (uint64_t)ncu;
+    uint64_t per_block = (uint64_t)wpb * std::max(cfg.chunk, 1u);
+    uint64_t need = (total + per_block - 1) / per_block;
+    if (g > need) g = need;
+    if (g < 1) g = 1;
+    return (uint32_t)g;
+}
+
+#define LCHECK()                                                                        \
+    do {                                                                                \
+        hipError_t e_ = hipGetLastError();                                              \
+        if (e_ != hipSuccess) {                                                         \
+            set_error(std::string("kernel launch failed: ") + hipGetErrorString(e_));    \
+            return -1;                                                                  \
+        }                                                                               \
+    } while (0)
+
+// LDS stack depth chosen from the BVH depth: 32 entries (32 KB per 256-lane block, 5 blocks per CU)
+// when the tree allows it, else 64.
+#define PICK_STK(depth, CALL32, CALL64) \
+    do {                                 \
+        if ((depth) + 1 <= 32) { CALL32; } else { CALL64; } \
+    } while (0)
+
+// Runs f(std::integral_constant<int, FL>) for the traversal flags fl (RT_FL_*): one kernel instance per flag set.
+template <typename F>
+static void with_flags(int fl, F &&f) {
+    switch (fl & (RT_FL_MASK | RT_FL_WT)) {
+        case 0: f(std::integral_constant<int, 0>{}); break;
+        case RT_FL_MASK: f(std::integral_constant<int, RT_FL_MASK>{}); break;
+        case RT_FL_WT: f(std::integral_constant<int, RT_FL_WT>{}); break;
+        default: f(std::integral_constant<int, RT_FL_MASK | RT_FL_WT>{}); break;
+    }
+}
+// the counting variants always compile the mask tests in (a scene without masks skips them at run time)
+static inline int counting_flags(int fl) { return (fl & RT_FL_WT) | RT_FL_MASK; }
+
+}  // namespace rt
