@@ -183,7 +183,7 @@ int rt_cast_rays_soa_device(rt_ctx *ctx, const rt_scene *scene, const float *o, 
     hipEvent_t a = nullptr, b = nullptr;
     if (ctx->sx.timing) { CKR(hipEventCreate(&a)); CKR(hipEventCreate(&b)); CKR(hipEventRecord(a, st)); }
     if (launch_cast(scene->s.d, scene->s.h.depth, n, o, d, max_dist, t, nrm, uuid, counter, err, ctx->sx.stat_ptr(2),
-                    ctx->sx.ncu, st, ctx->sx.watertight))
+                    ctx->sx.ncu, st, scene_flags(scene->s, ctx->sx)))
         return -1;
     if (b) CKR(hipEventRecord(b, st));
     int herr = 0;
@@ -348,7 +348,7 @@ int rt_lidar_cast_rays_noalloc(rt_ctx *ctx, const rt_scene *scene, const float *
     // castRaysSoA with the miss distance as the maximum distance (LiDAR.cpp:577-579); hits write hit_t
     // directly, misses leave it for the conversion
     if (launch_cast(scene->s.d, scene->s.h.depth, n, d_origins, d_dirs, miss_t, d_hit_t, nrm, uuid, counter, err,
-                    nullptr, ctx->sx.ncu, st, ctx->sx.watertight))
+                    nullptr, ctx->sx.ncu, st, scene_flags(scene->s, ctx->sx)))
         return -1;
     k_lidar_convert<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(n, d_dirs, nrm, uuid, miss_t, d_hit_t, d_hit_fnorm,
                                                                  d_hit_id);

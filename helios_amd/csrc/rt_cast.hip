@@ -16,29 +16,169 @@ __device__ __forceinline__ bool lane_leaf_cd(const float4 *recs, LaneRay &L, uin
     return lane_pop<STK, LSTK>(L, stk, ovf, stride);
 }
 
-// Next 64-ray chunk of a wave (wave-uniform 64-bit work counter).
-__device__ __forceinline__ unsigned long long wave_chunk64(unsigned long long *counter) {
+// Next chunk of rays of a wave (wave-uniform 64-bit work counter).
+__device__ __forceinline__ unsigned long long wave_chunk64(unsigned long long *counter, uint32_t chunk) {
     const uint32_t lane = threadIdx.x & 63;
-    unsigned long long f = atomicAdd(counter, lane == 0 ? 64ull : 0ull);
+    unsigned long long f = atomicAdd(counter, lane == 0 ? (unsigned long long)chunk : 0ull);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)f);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(f >> 32));
     return ((unsigned long long)hi << 32) | lo;
 }
 
-// castRaysSoA (CD/src/CollisionDetection_RayTracing.cpp:551-680, 980-1080): closest hit of each ray with
-// the CD predicates.  Persistent waves take 64-ray chunks from a counter and keep 64 rays in flight: a lane
-// whose trace ends writes its result and takes the chunk's next ray; traversal runs in node and leaf phases
-// as k_diffuse's.  Each ray is traced exactly as on its own.
-template <int STK, bool COUNT, int MK>
+// Result of a cast ray: the hit's UUID, distance and normal; a miss leaves distance and normal untouched.
+// rr: the hit's record (read on a hit only).
+__device__ __forceinline__ void cast_result(unsigned long long my_r, uint32_t h, float best_t, const float4 *rr, v3f o, v3f d,
+                                            const uint32_t *uuid, float *T, float *N, uint32_t *U) {
+    if (h == RT_MISS) {
+        U[my_r] = RT_MISS;
+        return;
+    }
+    U[my_r] = uuid[h];
+    T[my_r] = best_t;
+    const float4 r0 = rr[0], r1 = rr[1], r2 = rr[2], r3 = rr[3];
+    const uint32_t tag = __float_as_uint(r0.w);
+    const bool patch = (tag & RT_PATCH_BIT) != 0;
+    // CD/src/CollisionDetection_RayTracing.cpp:1572-1585: normal of cross(v1-v0, v2-v0), facing
+    // the origin; a voxel's is the outward normal of the face hit (1685-1711), not turned
+    v3f nn;
+    bool ok;
+    if (tag & RT_VOXEL_BIT) {
+        nn = voxel_normal_cd(r0, r1, add3(o, mul3(d, best_t)));
+        ok = false;
+    } else if (patch) {
+        nn = mk3(r3.x, r3.y, r3.z);
+        v3f raw = cross3(mk3(r1.x, r1.y, r1.z), add3(mk3(r1.x, r1.y, r1.z), mk3(r2.x, r2.y, r2.z)));
+        ok = rsqrt_cr(raw.x * raw.x + raw.y * raw.y + raw.z * raw.z) > 1e-8f;
+    } else {
+        nn = cross3(mk3(r1.x, r1.y, r1.z), mk3(r2.x, r2.y, r2.z));
+        float mag = rsqrt_cr(nn.x * nn.x + nn.y * nn.y + nn.z * nn.z);
+        ok = mag > 1e-8f;
+        if (ok) nn = mul3(nn, rdiv(1.0f, mag));
+    }
+    if (ok) {
+        v3f ip = add3(o, mul3(d, best_t));
+        v3f to = sub3(o, ip);
+        if (nn.x * to.x + nn.y * to.y + nn.z * to.z < 0) nn = mul3(nn, -1.0f);
+    } else if (!(tag & RT_VOXEL_BIT)) {
+        nn = nrm3(mk3(-d.x, -d.y, -d.z));
+    }
+    N[my_r * 3] = nn.x;
+    N[my_r * 3 + 1] = nn.y;
+    N[my_r * 3 + 2] = nn.z;
+}
+
 #ifndef RT_CAST_WAVES_PER_EU
 #define RT_CAST_WAVES_PER_EU 1
 #endif
-__global__ __launch_bounds__(256, COUNT ? 1 : RT_CAST_WAVES_PER_EU) void k_cast(const DevScene *__restrict__ scp, uint64_t n, const float *__restrict__ O,
+#ifndef RT_CAST_ROWS
+#define RT_CAST_ROWS 16
+#endif
+// castRaysSoA (CD/src/CollisionDetection_RayTracing.cpp:551-680, 980-1080): closest hit of each ray with
+// the CD predicates.  Persistent waves take chunks of rays from a counter and keep 64 rays in flight: a lane
+// whose trace ends writes its result and takes the chunk's next ray; traversal runs in node and leaf phases.
+// Each ray is traced exactly as on its own.  Over the block tree (blk_node_step).
+template <int WPB, int MK>
+__global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const DevScene *__restrict__ scp, uint64_t n, const float *__restrict__ O,
                                               const float *__restrict__ D, float maxd, float *__restrict__ T,
                                               float *__restrict__ N, uint32_t *__restrict__ U,
-                                              unsigned long long *counter, int *err, unsigned long long *stats) {
+                                              unsigned long long *counter, uint32_t chunk, int *err) {
+    constexpr int ROWS = RT_CAST_ROWS;
+    __shared__ uint32_t stk_all[ROWS * WPB * 64];
+    uint32_t ovf[RT_STACK - ROWS];
+    lds_u32 *stk = (lds_u32 *)stk_all + threadIdx.x;
+    const uint32_t stride = WPB * 64;
+    const DevScene &sc = *scp;
+    const float4 *recs = ldu(&sc.rec);
+    const char *blk = (const char *)ldu(&sc.blk);
+    const uint32_t *uuid = ldu(&sc.uuid);
+    const float tstart = maxd > 0.f ? maxd : FLT_MAX;
+    // a pass of the traversal loop takes at most one trace of each lane: more node steps than that mean a
+    // malformed tree
+    const uint32_t max_steps = (uint32_t)min(64ull * (ldu(&sc.nnode4) + 8ull), 0xFFFFFFFFull);
+    unsigned long long q_next = 0, q_end = 0, my_r = 0;
+    bool drained = false, busy = false;
+    BlkRay L;
+    L.o = L.d = mk3(0.f, 0.f, 0.f);
+    L.ix = L.iy = L.iz = L.ox = L.oy = L.oz = 0.f;
+    L.best_t = 0.f;
+    L.best = RT_MISS;
+    L.ni = RT_BLK_DONE;
+    L.sp = 1u;
+    uint32_t slot = 0u;
+    while (true) {
+        // finished lanes write their result
+        if (busy && L.ni == RT_BLK_DONE) {
+            cast_result(my_r, L.best, L.best_t, (const float4 *)(blk + (slot & ~63u)), L.o, L.d, uuid, T, N, U);
+            busy = false;
+        }
+        // idle lanes take the next rays of the wave's chunk
+        while (true) {
+            const uint64_t idle = __builtin_amdgcn_ballot_w64(!busy);
+            if (idle == 0) break;
+            if (q_next == q_end) {
+                if (drained) break;
+                const unsigned long long f = wave_chunk64(counter, chunk);
+                if (f >= n) { drained = true; break; }
+                q_next = f;
+                q_end = f + chunk < n ? f + chunk : n;
+            }
+            const uint32_t rank =
+                __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
+            const uint32_t left = (uint32_t)(q_end - q_next);
+            const uint32_t take = min((uint32_t)__popcll(idle), left);
+            if (!busy && rank < take) {
+                const unsigned long long r = q_next + rank;
+                L.o = mk3(O[r * 3], O[r * 3 + 1], O[r * 3 + 2]);
+                L.d = mk3(D[r * 3], D[r * 3 + 1], D[r * 3 + 2]);
+                // a cast ray may start far outside the scene, where an ulp of the reciprocal counts: divide
+                L.ix = fabsf(L.d.x) > 1e-18f ? 1.0f / L.d.x : copysignf(1e18f, L.d.x);
+                L.iy = fabsf(L.d.y) > 1e-18f ? 1.0f / L.d.y : copysignf(1e18f, L.d.y);
+                L.iz = fabsf(L.d.z) > 1e-18f ? 1.0f / L.d.z : copysignf(1e18f, L.d.z);
+                blk_start(L, stk);
+                L.best_t = tstart;
+                my_r = r;
+                busy = true;
+            }
+            q_next += take;
+        }
+        if (__builtin_amdgcn_ballot_w64(busy) == 0) break;  // queue empty and nothing in flight
+        const uint32_t floor_lanes = drained ? 1u : RT_REFILL_BELOW;
+        uint32_t steps = 0;
+        while (true) {
+            while (true) {
+                const bool inner = !(L.ni & RT_BLK_REC);
+                if (__builtin_amdgcn_ballot_w64(inner) == 0 ||
+                    (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(!inner && L.ni != RT_BLK_DONE)) >= RT_LEAF_BATCH)
+                    break;
+                if (++steps > max_steps) {
+                    atomicOr(err, 2);
+                    L.ni = RT_BLK_DONE;
+                    break;
+                }
+                if (inner) blk_node_step<ROWS>(blk, L, stk, ovf, stride);
+            }
+            while (true) {
+                const bool leaf = (L.ni & RT_BLK_REC) && L.ni != RT_BLK_DONE;
+                if (__builtin_amdgcn_ballot_w64(leaf) == 0) break;
+                if (leaf) {
+                    blk_leaf<true, MK>(blk, recs, L.ni, L, 1e-6f, RT_MISS, slot);
+                    L.ni = blk_pop<ROWS>(L, stk, ovf, stride);
+                }
+            }
+            if ((uint32_t)__popcll(__builtin_amdgcn_ballot_w64(L.ni != RT_BLK_DONE)) < floor_lanes) break;
+        }
+    }
+}
+
+// The same over the binary tree: the counting variant (COUNT), whose node visits are the canonical work measure,
+// and scenes without a block tree.
+template <int STK, bool COUNT, int MK>
+__global__ __launch_bounds__(256) void k_cast_bin(const DevScene *__restrict__ scp, uint64_t n, const float *__restrict__ O,
+                                                  const float *__restrict__ D, float maxd, float *__restrict__ T,
+                                                  float *__restrict__ N, uint32_t *__restrict__ U,
+                                                  unsigned long long *counter, int *err, unsigned long long *stats) {
     constexpr int LSTK = STK < RT_DIFFUSE_LDS_STACK ? STK : RT_DIFFUSE_LDS_STACK;
-    __shared__ uint32_t stk_all[(LSTK + 1) * 256];  // + the spare row of the branch-free BVH4 pushes
+    __shared__ uint32_t stk_all[LSTK * 256];
     uint32_t ovf[STK > LSTK ? RT_STACK - LSTK : 1];
     lds_u32 *stk = (lds_u32 *)stk_all + threadIdx.x;
     const uint32_t stride = 256;
@@ -47,11 +187,6 @@ __global__ __launch_bounds__(256, COUNT ? 1 : RT_CAST_WAVES_PER_EU) void k_cast(
     const uint32_t *uuid = ldu(&sc.uuid);
     const uint32_t nleaf = ldu(&sc.nleaf);
     const float tstart = maxd > 0.f ? maxd : FLT_MAX;
-    // the 8-bit 4-wide tree when present and its worst-case stack fits; the counting variant walks the
-    // binary tree, whose node visits are the canonical work measure
-    const float4 *q4 = ldu(&sc.qnode4);
-    const uint32_t nn4 = ldu(&sc.nnode4);
-    const bool useq = RT_CAST_QBVH4 && !COUNT && q4 != nullptr && 3u * ldu(&sc.depth4) + 1u <= (uint32_t)STK;
     Cnt<COUNT, MK> cnt{};
     uint32_t nray = 0;
     unsigned long long q_next = 0, q_end = 0, my_r = 0;
@@ -63,45 +198,7 @@ __global__ __launch_bounds__(256, COUNT ? 1 : RT_CAST_WAVES_PER_EU) void k_cast(
     while (true) {
         // finished lanes write their result
         if (busy && !trav) {
-            if (RT_Q4_LATE_ERR && L.budget == RT_BUDGET_BAD) atomicOr(err, 2);
-            const uint32_t h = L.best;
-            if (h == RT_MISS) {
-                U[my_r] = RT_MISS;
-            } else {
-                U[my_r] = uuid[h];
-                T[my_r] = L.best_t;
-                const float4 *rr = recs + (size_t)slot * 4;
-                const float4 r0 = rr[0], r1 = rr[1], r2 = rr[2], r3 = rr[3];
-                const uint32_t tag = __float_as_uint(r0.w);
-                const bool patch = (tag & RT_PATCH_BIT) != 0;
-                // CD/src/CollisionDetection_RayTracing.cpp:1572-1585: normal of cross(v1-v0, v2-v0), facing
-                // the origin; a voxel's is the outward normal of the face hit (1685-1711), not turned
-                v3f nn;
-                bool ok;
-                if (tag & RT_VOXEL_BIT) {
-                    nn = voxel_normal_cd(r0, r1, add3(L.o, mul3(L.d, L.best_t)));
-                    ok = false;
-                } else if (patch) {
-                    nn = mk3(r3.x, r3.y, r3.z);
-                    v3f raw = cross3(mk3(r1.x, r1.y, r1.z), add3(mk3(r1.x, r1.y, r1.z), mk3(r2.x, r2.y, r2.z)));
-                    ok = rsqrt_cr(raw.x * raw.x + raw.y * raw.y + raw.z * raw.z) > 1e-8f;
-                } else {
-                    nn = cross3(mk3(r1.x, r1.y, r1.z), mk3(r2.x, r2.y, r2.z));
-                    float mag = rsqrt_cr(nn.x * nn.x + nn.y * nn.y + nn.z * nn.z);
-                    ok = mag > 1e-8f;
-                    if (ok) nn = mul3(nn, rdiv(1.0f, mag));
-                }
-                if (ok) {
-                    v3f ip = add3(L.o, mul3(L.d, L.best_t));
-                    v3f to = sub3(L.o, ip);
-                    if (nn.x * to.x + nn.y * to.y + nn.z * to.z < 0) nn = mul3(nn, -1.0f);
-                } else if (!(tag & RT_VOXEL_BIT)) {
-                    nn = nrm3(mk3(-L.d.x, -L.d.y, -L.d.z));
-                }
-                N[my_r * 3] = nn.x;
-                N[my_r * 3 + 1] = nn.y;
-                N[my_r * 3 + 2] = nn.z;
-            }
+            cast_result(my_r, L.best, L.best_t, recs + (size_t)slot * 4, L.o, L.d, uuid, T, N, U);
             busy = false;
         }
         // idle lanes take the next rays of the wave's chunk
@@ -110,7 +207,7 @@ __global__ __launch_bounds__(256, COUNT ? 1 : RT_CAST_WAVES_PER_EU) void k_cast(
             if (idle == 0) break;
             if (q_next == q_end) {
                 if (drained) break;
-                const unsigned long long f = wave_chunk64(counter);
+                const unsigned long long f = wave_chunk64(counter, 64u);
                 if (f >= n) { drained = true; break; }
                 q_next = f;
                 q_end = f + 64 < n ? f + 64 : n;
@@ -141,8 +238,7 @@ __global__ __launch_bounds__(256, COUNT ? 1 : RT_CAST_WAVES_PER_EU) void k_cast(
                 const bool inner = trav && !(L.ni & RT_LEAF_BIT);
                 const uint64_t mi = __ballot(inner);
                 if (mi == 0 || (uint32_t)__popcll(__ballot(trav && !inner)) >= RT_LEAF_BATCH) break;
-                if (inner && (useq ? lane_node4q<STK, LSTK, false>(q4, nn4, L, stk, ovf, stride, err, cnt)
-                                   : lane_node<STK, LSTK>(nodes, nleaf, L, stk, ovf, stride, err, cnt)))
+                if (inner && lane_node<STK, LSTK>(nodes, nleaf, L, stk, ovf, stride, err, cnt))
                     trav = false;
             }
             while (true) {
@@ -615,7 +711,7 @@ int launch_camera(const CameraLaunch &c, uint32_t depth, bool labels, int *err, 
 
 int launch_cast(const DevScene *sc, uint32_t depth, uint64_t n, const float *o, const float *d, float maxd, float *t,
                 float *nrm, uint32_t *uuid, unsigned long long *counter, int *err, unsigned long long *stats,
-                int ncu, hipStream_t st, bool watertight) {
+                int ncu, hipStream_t st, int flags) {
     if (n == 0) return 0;
     if (depth + 1 > RT_STACK) {
         set_error("BVH depth " + std::to_string(depth) + " exceeds the traversal stack (" + std::to_string(RT_STACK) + ")");
@@ -623,16 +719,14 @@ int launch_cast(const DevScene *sc, uint32_t depth, uint64_t n, const float *o, 
     }
     k_zero_u64<<<1, 1, 0, st>>>(counter);
     const uint64_t chunks = (n + 63) / 64;
-    uint64_t g = std::min<uint64_t>((uint64_t)8 * ncu, (chunks + 3) / 4);
-    if (g < 1) g = 1;
+    const uint32_t g = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)8 * ncu, (chunks + 3) / 4));
     // castRays ignores texture masks (as CollisionDetection does); only the predicate flag applies
-    if (watertight) {
-        if (stats) k_cast<RT_STACK, true, RT_FL_WT><<<(uint32_t)g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, err, stats);
-        else k_cast<RT_STACK, false, RT_FL_WT><<<(uint32_t)g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, err, stats);
-    } else {
-        if (stats) k_cast<RT_STACK, true, 0><<<(uint32_t)g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, err, stats);
-        else k_cast<RT_STACK, false, 0><<<(uint32_t)g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, err, stats);
-    }
+    with_flags(flags & RT_FL_WT, [&](auto fl) {
+        constexpr int FL = decltype(fl)::value & RT_FL_WT;
+        if (stats) k_cast_bin<RT_STACK, true, FL><<<g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, err, stats);
+        else if (flags & RT_FL_BLK) k_cast<4, FL><<<g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, 64u, err);
+        else k_cast_bin<RT_STACK, false, FL><<<g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, err, nullptr);
+    });
     LCHECK();
     return 0;
 }

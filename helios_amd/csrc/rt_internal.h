@@ -95,7 +95,7 @@ int launch_camera(const CameraLaunch &c, uint32_t depth, bool labels, int *err, 
 // counter: device scratch for the work queue (zeroed by the launch)
 int launch_cast(const DevScene *sc, uint32_t depth, uint64_t n, const float *o, const float *d, float maxd, float *t,
                 float *nrm, uint32_t *uuid, unsigned long long *counter, int *err, unsigned long long *stats,
-                int ncu, hipStream_t st, bool watertight = false);
+                int ncu, hipStream_t st, int flags);
 int launch_debug_rays(const DevScene *sc, uint32_t P, uint32_t n, uint32_t seed, float *out, hipStream_t st);
 int launch_debug_trace(const DevScene *sc, uint32_t n, const float *rays, const uint32_t *skip, float tmin, int brute,
                        uint32_t *hit, float *t, int *err, hipStream_t st, int flags = 0);

@@ -442,15 +442,11 @@ __global__ void k_c4_write(uint32_t count, uint32_t level_base, uint32_t next_ba
     o[7] = make_float4(__uint_as_float((uint32_t)cnt), 0.f, 0.f, 0.f);
 }
 
-// 8-bit BVH4 nodes (64 B) from the float ones (128 B).  Per node: the union box of its children as the
+// Blocks (rt_types.h) from the float BVH4 nodes (128 B).  Per node: the union box of its children as the
 // origin o and a power-of-two step s_a = 2^e_a per axis with 255 s_a >= extent; a child bound is stored as
 // floor((lo - o) / s) and ceil((hi - o) / s), so the decoded box o + q s contains the float box exactly
 // (the differences and quotients are exact in double: floats differ by a double-exact amount, s is a power
-// of two).  Layout, as uint words:
-//   q0 = (o.x, o.y, o.z bits, e_x+127 | e_y+127 << 8 | e_z+127 << 16 | children << 24)
-//   q1 = (lo.x, hi.x, lo.y, hi.y), q2 = (lo.z, hi.z, link0, link1), q3 = (link2, link3, 0, 0)
-// where each bound word holds the four children's bytes, child k in bits 8k..8k+7.  Unused slots (k >=
-// children) are never tested.
+// of two).
 __device__ __forceinline__ int q_exponent(double ext) {
     // smallest e in [-126, 127] with 255 * 2^e >= ext
     if (!(ext > 0.0)) return -126;
@@ -459,39 +455,69 @@ __device__ __forceinline__ int q_exponent(double ext) {
     return x < -126 ? -126 : (x > 127 ? 127 : x);
 }
 
-__global__ void k_q4(uint32_t nn4, const float4 *__restrict__ node4, uint4 *__restrict__ q4, int *__restrict__ bad) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nn4) return;
+// base[t]: block of node t's first child
+__device__ __forceinline__ void blk_node(uint32_t t, const float4 *__restrict__ node4, const uint32_t *__restrict__ base,
+                                         uint4 *__restrict__ dst, int *bad) {
     const float4 *o = node4 + (size_t)t * 8;
     const uint32_t cnt = __float_as_uint(o[7].x);
-    float lo[3][4], hi[3][4];
+    uint32_t org[3], ex[3], wl[3], wh[3];
     for (int a = 0; a < 3; a++) {
         const float4 l = o[2 * a], h = o[2 * a + 1];
-        lo[a][0] = l.x; lo[a][1] = l.y; lo[a][2] = l.z; lo[a][3] = l.w;
-        hi[a][0] = h.x; hi[a][1] = h.y; hi[a][2] = h.z; hi[a][3] = h.w;
-    }
-    uint32_t org[3], meta = cnt << 24, wl[3] = {0u, 0u, 0u}, wh[3] = {0u, 0u, 0u};
-    for (int a = 0; a < 3; a++) {
+        const float lo[4] = {l.x, l.y, l.z, l.w}, hi[4] = {h.x, h.y, h.z, h.w};
         float u0 = INFINITY, u1 = -INFINITY;
-        for (uint32_t k = 0; k < cnt; k++) { u0 = fminf(u0, lo[a][k]); u1 = fmaxf(u1, hi[a][k]); }
+        for (uint32_t k = 0; k < 4; k++)
+            if (k < cnt) { u0 = fminf(u0, lo[k]); u1 = fmaxf(u1, hi[k]); }
         const int e = q_exponent((double)u1 - (double)u0);
         const double s = ldexp(1.0, e);
-        for (uint32_t k = 0; k < cnt; k++) {
-            const double ql = floor(((double)lo[a][k] - (double)u0) / s);
-            const double qh = ceil(((double)hi[a][k] - (double)u0) / s);
-            if (!(ql >= 0.0 && qh <= 255.0 && ql <= qh)) atomicOr(bad, 1);
+        wl[a] = wh[a] = 0u;
+        for (uint32_t k = 0; k < 4; k++) {
+            double ql = 255.0, qh = 0.0;  // unused child: an empty box
+            if (k < cnt) {
+                ql = floor(((double)lo[k] - (double)u0) / s);
+                qh = ceil(((double)hi[k] - (double)u0) / s);
+                if (!(ql >= 0.0 && qh <= 255.0 && ql <= qh)) atomicOr(bad, 1);
+            }
             wl[a] |= (uint32_t)fmin(fmax(ql, 0.0), 255.0) << (8 * k);
             wh[a] |= (uint32_t)fmin(fmax(qh, 0.0), 255.0) << (8 * k);
         }
         org[a] = __float_as_uint(u0);
-        meta |= (uint32_t)(e + 127) << (8 * a);
+        ex[a] = (uint32_t)(e + 127);
     }
-    const float4 lk = o[6];
-    uint4 *q = q4 + (size_t)t * 4;
-    q[0] = make_uint4(org[0], org[1], org[2], meta);
-    q[1] = make_uint4(wl[0], wh[0], wl[1], wh[1]);
-    q[2] = make_uint4(wl[2], wh[2], __float_as_uint(lk.x), __float_as_uint(lk.y));
-    q[3] = make_uint4(__float_as_uint(lk.z), __float_as_uint(lk.w), 0u, 0u);
+    const float4 lk4 = o[6];
+    const uint32_t lk[4] = {__float_as_uint(lk4.x), __float_as_uint(lk4.y), __float_as_uint(lk4.z),
+                            __float_as_uint(lk4.w)};
+    uint32_t code = 0u;
+    for (uint32_t k = 0; k < 4; k++) {
+        const uint32_t c = k < cnt ? k : 0u;
+        code |= ((c << 6) | ((lk[c] & RT_LEAF_BIT) ? RT_BLK_REC : 0u)) << (8 * k);
+    }
+    dst[0] = make_uint4(org[0], org[1], org[2], (ex[0] << 23) | (ex[1] << 15) | (ex[2] << 7));
+    dst[1] = make_uint4(wl[0], wh[0], wl[1], wh[1]);
+    dst[2] = make_uint4(wl[2], wh[2], code, 64u * base[t]);
+    dst[3] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+__global__ void k_blk_count(uint32_t nn4, const float4 *__restrict__ node4, uint32_t *__restrict__ cnt) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nn4) cnt[t] = __float_as_uint(node4[(size_t)t * 8 + 7].x);
+}
+
+// one thread per (node, child slot); thread 0 also writes the root
+__global__ void k_blocks(uint32_t nn4, const float4 *__restrict__ node4, const float4 *__restrict__ rec,
+                         const uint32_t *__restrict__ base, uint4 *__restrict__ blk, int *__restrict__ bad) {
+    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = g >> 2, k = g & 3u;
+    if (t >= nn4) return;
+    if (g == 0) blk_node(0u, node4, base, blk, bad);
+    if (k >= __float_as_uint(node4[(size_t)t * 8 + 7].x)) return;
+    const uint32_t lk = __float_as_uint(((const float *)(node4 + (size_t)t * 8 + 6))[k]);
+    uint4 *dst = blk + ((size_t)base[t] + k) * 4;
+    if (lk & RT_LEAF_BIT) {
+        const uint4 *r = (const uint4 *)rec + (size_t)(lk & ~RT_LEAF_BIT) * 4;
+        for (int q = 0; q < 4; q++) dst[q] = r[q];
+    } else {
+        blk_node(lk, node4, base, dst, bad);
+    }
 }
 
 // node layout: (c0.lo.x, c0.hi.x, c0.lo.y, c0.hi.y), (c0.lo.z, c0.hi.z, c1.lo.x, c1.hi.x),
@@ -652,6 +678,35 @@ static int build_bvh4(uint32_t n, const uint32_t *child, const float *lbox, cons
     return 0;
 }
 
+// bytes of the block tree of nn4 nodes over nleaf records and of the build's check word
+static size_t blk_bytes(uint32_t nn4, uint32_t nleaf) { return 64 * ((size_t)nn4 + nleaf) + 64; }
+
+static int write_blocks(uint32_t nn4, uint32_t nleaf, const float4 *node4, const float4 *rec, uint4 *blk, hipStream_t st) {
+    int *bad = (int *)(blk + 4 * ((size_t)nn4 + nleaf));
+    uint32_t *cnt;
+    CK(hipMalloc(&cnt, sizeof(uint32_t) * 2 * (size_t)nn4));
+    uint32_t *base = cnt + nn4;
+    size_t tmp_bytes = 0;
+    // child blocks follow the root's
+    CK(hipcub::DeviceScan::ExclusiveScan(nullptr, tmp_bytes, cnt, base, hipcub::Sum(), 1u, (int)nn4, st));
+    void *tmp;
+    CK(hipMalloc(&tmp, tmp_bytes + 16));
+    CK(hipMemsetAsync(bad, 0, sizeof(int), st));
+    k_blk_count<<<blocks(nn4, 256), 256, 0, st>>>(nn4, node4, cnt);
+    CK(hipcub::DeviceScan::ExclusiveScan(tmp, tmp_bytes, cnt, base, hipcub::Sum(), 1u, (int)nn4, st));
+    k_blocks<<<blocks((size_t)nn4 * 4, 256), 256, 0, st>>>(nn4, node4, rec, base, blk, bad);
+    CK(hipGetLastError());
+    int hbad = 0;
+    CK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, st));
+    CK(hipStreamSynchronize(st));
+    CK(hipFree(cnt)); CK(hipFree(tmp));
+    if (hbad) {
+        set_error("block tree: a child box lies outside its node's 8-bit grid");
+        return -1;
+    }
+    return 0;
+}
+
 int validate_geometry(uint64_t P, const uint32_t *types, const char *who) {
     if (P > RT_MAX_PRIMS) {
         set_error(std::string(who) + ": " + std::to_string(P) + " primitives (at most 2^29)");
@@ -744,7 +799,8 @@ int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, cons
     S.h.smax = 0.f;
     for (int a = 0; a < 3; a++) S.h.smax = fmaxf(S.h.smax, fmaxf(fabsf(vmin[a]), fabsf(vmax[a])));
 
-    float4 *rec = nullptr, *node = nullptr, *node4 = nullptr, *qnode4 = nullptr;
+    float4 *rec = nullptr, *node = nullptr, *node4 = nullptr;
+    uint4 *blk = nullptr;
     uint32_t depth = 0, nnode4 = 0, depth4 = 0;
     if (nleaf > 0) {
         float *lbox;
@@ -787,17 +843,10 @@ int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, cons
             CK(hipMalloc(&node4, sizeof(float4) * 8 * (size_t)(nleaf - 1)));
             S.own.push_back(node4);
             if (build_bvh4(nleaf, child, lbox, ibox, node4, nnode4, depth4, st)) return -1;
-            CK(hipMalloc(&qnode4, sizeof(uint4) * 4 * (size_t)nnode4 + sizeof(int)));
-            S.own.push_back(qnode4);
-            int *qbad = (int *)((uint4 *)qnode4 + 4 * (size_t)nnode4);
-            CK(hipMemsetAsync(qbad, 0, sizeof(int), st));
-            k_q4<<<blocks(nnode4, 256), 256, 0, st>>>(nnode4, node4, (uint4 *)qnode4, qbad);
-            int hbad = 0;
-            CK(hipMemcpyAsync(&hbad, qbad, sizeof(int), hipMemcpyDeviceToHost, st));
-            CK(hipStreamSynchronize(st));
-            if (hbad) {
-                set_error("8-bit BVH4 node quantisation failed (a child box outside its node's grid)");
-                return -1;
+            if ((uint64_t)nnode4 + nleaf <= RT_BLK_MAX) {
+                CK(hipMalloc(&blk, blk_bytes(nnode4, nleaf)));
+                S.own.push_back(blk);
+                if (write_blocks(nnode4, nleaf, node4, rec, blk, st)) return -1;
             }
             CK(hipFree(child)); CK(hipFree(ibox));
         } else {
@@ -823,7 +872,7 @@ int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, cons
     S.h.order = vals2;
     // a BVH4 traversal pushes at most 3 entries per level: use it only when that fits the wave stack (128)
     S.h.node4 = (node4 && 3 * depth4 + 1 <= 128) ? node4 : nullptr;
-    S.h.qnode4 = S.h.node4 ? qnode4 : nullptr;
+    S.h.blk = 3 * depth4 + 1 <= RT_STACK ? blk : nullptr;
     S.h.nnode4 = nnode4;
     S.h.depth4 = depth4;
     S.h.nleaf = nleaf;
@@ -833,7 +882,7 @@ int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, cons
     CK(hipMemcpyAsync(S.d, &S.h, sizeof(DevScene), hipMemcpyHostToDevice, st));
     CK(hipStreamSynchronize(st));
     S.bytes = (size_t)P * (64 + 4 * 4 + 16 * 2) + (size_t)nleaf * 64 + (nleaf > 1 ? (size_t)(nleaf - 1) * 64 : 0) +
-              (size_t)(nleaf > 1 ? nleaf - 1 : 0) * 128 + (size_t)nnode4 * 64;
+              (size_t)(nleaf > 1 ? nleaf - 1 : 0) * 128 + (blk ? blk_bytes(nnode4, nleaf) : 0);
     return 0;
 }
 
@@ -934,6 +983,8 @@ int scene_set_masks(Scene &S, uint32_t nmasks, const uint8_t *texels, const uint
     if (dm) S.own.push_back(dm);
     S.h.rec = R;
     S.h.mdesc = dm;
+    // the block tree holds copies of the records
+    if (S.h.blk && write_blocks(S.h.nnode4, nleaf, S.h.node4, R, const_cast<uint4 *>(S.h.blk), st)) return -1;
     CK(hipMemcpyAsync(S.d, &S.h, sizeof(DevScene), hipMemcpyHostToDevice, st));
     CK(hipStreamSynchronize(st));
     return 0;

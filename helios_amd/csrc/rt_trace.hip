@@ -6,34 +6,30 @@ namespace rt {
 // ------------------------------------------------------------------------------------------------
 // diffuse / scattering rays -> hit words
 // ------------------------------------------------------------------------------------------------
-// A wave keeps 64 rays in flight.  Rays of one primitive are handed to idle lanes in ray order; a lane
-// whose traversal ends writes its hit word and takes the primitive's next ray, and the wave opens the
-// next primitive of the work queue when the current one has no rays left.  The traversal loop runs until
-// fewer than RT_REFILL_BELOW lanes are still traversing (all of them once the queue is empty), so lanes do
-// not idle for the longest ray of a fixed group of 64.  Every ray is traced exactly as a plain
-// per-ray trace_loop() would trace it; only the assignment of rays to lanes and steps differs.
-// The traversal stack keeps its first RT_DIFFUSE_LDS_STACK entries in LDS and deeper ones in private
-// memory: 4 KB of LDS per wave leaves the register file (about 70 VGPRs) as the occupancy limit.
-// Diffuse lanes park the first leaf they reach and keep stepping (585 against 598 ms for the orchard's five
-// passes)
-#ifndef RT_LEAF_DEFER
-#define RT_LEAF_DEFER 1
-#endif
-#define RT_DEFER_END 0xFFFFFFFFu
-// With parked leaves, the leaf phase tests one leaf per waiting lane and returns to the node phase (lanes
-// that reach further leaves park them there), and starts once 8 lanes wait: 589 -> 554 ms for the
-// orchard's five passes (batches of 2-24 lanes swept; the full leaf phase with 16 lanes was the 589)
-#ifndef RT_LEAF_ONE_ROUND
-#define RT_LEAF_ONE_ROUND 1
-#endif
+// A wave keeps 64 rays in flight; a lane whose traversal ends writes its hit word and takes another ray, and
+// the wave opens the next primitive of the work queue when the current one has no rays left, so lanes do not
+// idle for the longest ray of a fixed group of 64.  Every ray is traced exactly as a plain per-ray
+// trace_loop() would trace it; only the assignment of rays to lanes and steps differs.
+//
+// k_diffuse walks the block tree.  It is bound by the issue of VALU instructions (see
+// blk_node_step()), so everything else keeps as many lanes as it can in each instruction:
+// - Rays are generated up to 64 at a time with every lane active, into the wave's LDS queue (local sample point
+//   and world direction, 20 B a ray): the hashing, square roots and divisions of a ray (about 1,500 cycles a
+//   wave) ran for the 19 lanes being refilled on average when each refill generated its own rays.  A
+//   primitive's rays are split into equal batches (450 rays: 8 of 56 or 57).
+// - A lane that reaches a record parks it and goes on with its next link, so it keeps taking node steps; it
+//   waits only at a second record or with no links left.  Once RT_LEAF_BATCH_PARKED lanes wait, every parked
+//   record is tested, one per lane, and the node phase goes on.
+// LDS per wave: RT_BLK_ROWS stack rows and the queue's five, 5 KB, which 32 waves fill the CU's 160 KB with.
 #ifndef RT_LEAF_BATCH_PARKED
 #define RT_LEAF_BATCH_PARKED 8
 #endif
-// Waves per SIMD the compiler must fit the timed diffuse kernel into (the default launch shape, 16 two-wave
-// workgroups per CU, runs 8 per SIMD): on the orchard 8 waves with a few spills beat 5 waves without (622
-// against 726 ms per diurnal series).  With texture masks, 8 as well (the homogeneous-canopy benchmark's
-// diffuse runBand 0.67 s at 5 waves, 0.56 s at 8); with watertight predicates, 6 (one plain orchard solve
-// 804 ms at 8, 732 ms at 6: the larger leaf test spills more); the counting variants keep their registers.
+#ifndef RT_BLK_REFILL
+#define RT_BLK_REFILL 48
+#endif
+#define RT_BLK_ROWS 15
+// Waves per SIMD the compiler must fit the kernel into (the default launch shape, 16 two-wave workgroups per CU,
+// runs 8 per SIMD).  Watertight predicates: 6 (their larger leaf test would spill at 8).
 #ifndef RT_DIFFUSE_WAVES_PER_EU
 #define RT_DIFFUSE_WAVES_PER_EU 8
 #endif
@@ -43,15 +39,218 @@ namespace rt {
 #ifndef RT_DIFFUSE_WAVES_PER_EU_MASKED
 #define RT_DIFFUSE_WAVES_PER_EU_MASKED 8
 #endif
+// rr / n and rr % n of a ray number rr < n * n: a multiply by ceil(2^32 / n) is exact while n^3 < 2^32
+__device__ __forceinline__ void ray_cell(uint32_t rr, uint32_t n, uint32_t inv, uint32_t &lx, uint32_t &ly) {
+    ly = n - 2u < 1598u ? __umulhi(rr, inv) : rr / n;
+    lx = rr - ly * n;
+}
+
+template <int WPB, int MK>
+__global__ __launch_bounds__(WPB * 64, (MK & RT_FL_MASK) ? RT_DIFFUSE_WAVES_PER_EU_MASKED
+                                       : (MK & RT_FL_WT) ? RT_DIFFUSE_WAVES_PER_EU_WT
+                                                         : RT_DIFFUSE_WAVES_PER_EU)
+void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *counter, uint32_t chunk, int *err) {
+    constexpr int ROWS = RT_BLK_ROWS;
+    __shared__ uint32_t stk_all[ROWS * WPB * 64];
+    __shared__ float queue_all[5 * WPB * 64];
+    // stack rows beyond the LDS part, in private memory
+    uint32_t ovf[RT_STACK - ROWS];
+    lds_u32 *stk = (lds_u32 *)stk_all + threadIdx.x;
+    const uint32_t stride = WPB * 64;
+    const uint32_t lane = threadIdx.x & 63;
+    // the wave's queue: entry e of component c at queue[c * 64 + e]
+    lds_f32 *queue = (lds_f32 *)queue_all + (threadIdx.x >> 6) * 320u;
+    // job and scene (wave-uniform, scalar loads)
+    const DevScene &sc = *ldu(&job->sc);
+    const float4 *recs = ldu(&sc.rec), *nrm = ldu(&sc.nrm), *frame = ldu(&sc.frame);
+    const char *blk = (const char *)ldu(&sc.blk);
+    const float *T = ldu(&sc.T);
+    const uint32_t *type = ldu(&sc.type);
+    const uint32_t *mdesc = ldu(&sc.mdesc);
+    const uint32_t nbbox = ldu(&sc.nbbox);
+    const uint32_t n = ldu(&job->n), nn = n * n, seed = ldu(&job->seed);
+    const uint32_t inv = n > 1u ? (uint32_t)((0x100000000ull + n - 1u) / n) : 0u;
+    const uint32_t faces = ldu(&job->faces) ? ldu(&job->faces) : 3u;
+    const uint32_t item_begin = ldu(&job->item_begin);
+    const uint32_t *order = ldu(&job->order);
+    uint32_t *hits = ldu(&job->hits);
+    // a pass of the traversal loop takes at most one trace of each lane: more node steps than that mean a
+    // malformed tree
+    const uint32_t max_steps = (uint32_t)min(64ull * (ldu(&sc.nnode4) + 8ull), 0xFFFFFFFFull);
+    // work queue, open primitive and its ray queue (wave-uniform); the primitive's frame and transform are
+    // reloaded (scalar) whenever rays are generated or taken, so they hold no registers across the traversal
+    uint32_t it = 0, it_end = 0;
+    bool drained = false;
+    uint32_t op_i = 0, op_next = 0, op_cnt = 0, op_base = 0, op_m = RT_MISS;
+    uint32_t q_next = 0, q_cnt = 0, q_ray = 0;
+    bool patch = false, flip = false;
+    // lane state: busy = holds a ray (its trace has ended when L.ni is RT_BLK_DONE and no record is parked)
+    bool busy = false;
+    BlkRay L;
+    L.o = L.d = mk3(0.f, 0.f, 0.f);
+    L.ix = L.iy = L.iz = L.ox = L.oy = L.oz = 0.f;
+    L.best_t = 0.f;
+    L.best = RT_MISS;
+    L.ni = RT_BLK_DONE;
+    L.sp = 1u;
+    uint32_t my_i = 0, my_r = 0, wraps = 0;
+    uint32_t pend = 0u;  // link of the parked record, 0 = none
+    while (true) {
+        // finish lanes whose traversal ended: periodic wrap (as trace_loop: at most 32 traces), else write
+        if (busy && L.ni == RT_BLK_DONE) {
+            bool done = true;
+            if (nbbox) {
+                float bt = nearest_face_u(sc, nbbox, L.o, L.d, L.best_t);
+                if (bt > 0.f && wraps < 31) {
+                    L.o = wrap_at(sc, L.o, L.d, bt);
+                    wraps++;
+                    blk_start(L, stk);
+                    done = false;
+                }
+            }
+            if (done) {
+                uint32_t word = RT_MISS;
+                if (L.best != RT_MISS) {
+                    float4 hn = nrm[L.best];
+                    bool hit_top = dot3(mk3(hn.x, hn.y, hn.z), L.d) < 0.0f;
+                    word = L.best | (hit_top ? 0u : RT_HIT_BOTTOM);
+                }
+                hits[(size_t)my_i * 2 * nn + my_r] = word;
+                busy = false;
+            }
+        }
+        // refill idle lanes
+        while (true) {
+            const uint64_t idle = __builtin_amdgcn_ballot_w64(!busy);
+            if (idle == 0) break;
+            if (q_next == q_cnt) {
+                if (op_next == op_cnt) {
+                    // open the next primitive of the work queue
+                    if (it == it_end) {
+                        if (drained) break;
+                        it = wave_item(counter, chunk);
+                        if (it >= total) { drained = true; it = it_end = 0; break; }
+                        it_end = min(it + chunk, total);
+                    }
+                    uint32_t i = it - item_begin;
+                    if (order) i = ldu(order + i);
+                    i = __builtin_amdgcn_readfirstlane(i);
+                    it++;
+                    uint32_t *w = hits + (size_t)i * 2 * nn;
+                    const uint32_t ty = ldu(type + i);
+                    if (!traced_type(ty)) {
+                        for (uint32_t r = lane; r < 2 * nn; r += 64) w[r] = RT_NOT_LAUNCHED;
+                        continue;
+                    }
+                    const uint32_t tw = __float_as_uint(ldu(&nrm[i].w));
+                    const bool s0 = (faces & 1u) != 0, s1 = ((faces >> 1) & 1u) != 0 && tw != 0;
+                    if (!s0) for (uint32_t r = lane; r < nn; r += 64) w[r] = RT_NOT_LAUNCHED;
+                    if (!s1) for (uint32_t r = nn + lane; r < 2 * nn; r += 64) w[r] = RT_NOT_LAUNCHED;
+                    op_i = i;
+                    op_m = (MK && mdesc) ? ldu(mdesc + i) : RT_MISS;
+                    op_next = 0;
+                    op_cnt = ((s0 ? 1u : 0u) + (s1 ? 1u : 0u)) * nn;
+                    op_base = s0 ? 0u : nn;
+                    patch = ty == 0 || ty == 3;
+                    flip = tw == 1;
+                    continue;
+                }
+                // generate the next batch of the open primitive's rays
+                const uint32_t left = op_cnt - op_next, batches = (left + 63u) >> 6;
+                q_cnt = (left + batches - 1u) / batches;
+                q_next = 0;
+                q_ray = op_base + op_next;
+                op_next += q_cnt;
+                if (lane < q_cnt) {
+                    const uint32_t r = q_ray + lane;
+                    const uint32_t slot = r >= nn ? 1u : 0u;  // slot 0 = top launch (face 1), slot 1 = bottom (face 0)
+                    uint32_t lx, ly;
+                    ray_cell(r - slot * nn, n, inv, lx, ly);
+                    float spx, spy;
+                    v3f dl;
+                    if (diffuse_sample_m(op_i, lx, ly, n, seed, patch, recs, op_m, spx, spy, dl)) {
+                        const float4 fr = ldu(frame + op_i);
+                        v3f dir = frame_rotate(dl, fr.x, fr.y, fr.z, fr.w);
+                        if (slot == 1 && flip) dir = mk3(-dir.x, -dir.y, -dir.z);
+                        queue[lane] = spx;
+                        queue[64 + lane] = spy;
+                        queue[128 + lane] = dir.x;
+                        queue[192 + lane] = dir.y;
+                        queue[256 + lane] = dir.z;
+                    } else {
+                        // origin on transparent texels: the ray is dropped (adds nothing to the gather); the lane
+                        // that takes this entry stays idle and takes another
+                        hits[(size_t)op_i * 2 * nn + r] = RT_NOT_LAUNCHED;
+                        queue[128 + lane] = 2.0f;
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();
+                continue;
+            }
+            const uint32_t rank =
+                __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
+            const uint32_t take = min((uint32_t)__popcll(idle), q_cnt - q_next);
+            if (!busy && rank < take) {
+                const uint32_t e = q_next + rank;
+                const float dx = queue[128 + e];
+                if (!MK || dx != 2.0f) {
+                    float tm[12];
+                    const float *Tp = T + (size_t)op_i * 16;
+#pragma unroll
+                    for (int q = 0; q < 12; q++) tm[q] = ldu(Tp + q);
+                    L.o = xform3(tm, queue[e], queue[64 + e], 0.0f);
+                    L.d = mk3(dx, queue[192 + e], queue[256 + e]);
+                    L.ix = blk_rcp(L.d.x);
+                    L.iy = blk_rcp(L.d.y);
+                    L.iz = blk_rcp(L.d.z);
+                    blk_start(L, stk);
+                    my_i = op_i;
+                    my_r = q_ray + e;
+                    wraps = 0;
+                    busy = true;
+                }
+            }
+            q_next += take;
+        }
+        if (__builtin_amdgcn_ballot_w64(busy) == 0) break;  // queue empty and nothing in flight
+        // traverse until fewer than RT_BLK_REFILL lanes (once the queue is empty: no lane) still do
+        const uint32_t floor_lanes = drained ? 1u : RT_BLK_REFILL;
+        uint32_t steps = 0;
+        while (true) {
+            while (true) {
+                if ((L.ni & RT_BLK_REC) && L.ni != RT_BLK_DONE && pend == 0u) {
+                    pend = L.ni;
+                    L.ni = blk_pop<ROWS>(L, stk, ovf, stride);
+                }
+                const bool inner = !(L.ni & RT_BLK_REC);
+                if (__builtin_amdgcn_ballot_w64(inner) == 0 ||
+                    (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(!inner && pend != 0u)) >= RT_LEAF_BATCH_PARKED)
+                    break;
+                if (++steps > max_steps) {
+                    atomicOr(err, 2);
+                    L.ni = RT_BLK_DONE;
+                    break;
+                }
+                if (inner) blk_node_step<ROWS>(blk, L, stk, ovf, stride);
+            }
+            if (pend != 0u) {
+                uint32_t slot_unused;
+                blk_leaf<false, MK>(blk, recs, pend, L, 1e-5f, my_i, slot_unused);
+                pend = 0u;
+            }
+            if ((uint32_t)__popcll(__builtin_amdgcn_ballot_w64(L.ni != RT_BLK_DONE)) < floor_lanes) break;
+        }
+    }
+}
+
+// The same over the binary tree: the counting variant (COUNT), whose node visits and primitive tests are the
+// canonical work measure, and scenes without a block tree.  Traversal alternates a node phase (inner-node
+// steps until RT_LEAF_BATCH lanes wait at a leaf) and a leaf phase.
 template <int WPB, int STK, bool COUNT, int MK>
-__global__ __launch_bounds__(WPB * 64, COUNT ? 1 : ((MK & RT_FL_MASK) ? RT_DIFFUSE_WAVES_PER_EU_MASKED
-                                                                    : (MK & RT_FL_WT) ? RT_DIFFUSE_WAVES_PER_EU_WT
-                                                                                      : RT_DIFFUSE_WAVES_PER_EU))
-void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total,
-                                                      uint32_t *counter, uint32_t chunk, int *err,
-                                                      unsigned long long *stats) {
+__global__ __launch_bounds__(WPB * 64) void k_diffuse_bin(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *counter,
+                                                           uint32_t chunk, int *err, unsigned long long *stats) {
     constexpr int LSTK = STK < RT_DIFFUSE_LDS_STACK ? STK : RT_DIFFUSE_LDS_STACK;
-    __shared__ uint32_t stk_all[(LSTK + 1) * WPB * 64];  // + the spare row of the branch-free BVH4 pushes
+    __shared__ uint32_t stk_all[LSTK * WPB * 64];
     // overflow entries: sized for the deepest stack (RT_STACK) so the array stays in private memory
     // instead of being promoted to registers, which would cost the occupancy the small LDS part buys
     uint32_t ovf[STK > LSTK ? RT_STACK - LSTK : 1];
@@ -63,14 +262,6 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total,
     // job and scene (wave-uniform, scalar loads)
     const DevScene &sc = *ldu(&job->sc);
     const float4 *nodes = ldu(&sc.node), *recs = ldu(&sc.rec), *nrm = ldu(&sc.nrm), *frame = ldu(&sc.frame);
-    // the 4-wide tree when it exists and its worst-case stack fits (3 pushes per level); the counting
-    // variant walks the binary tree, whose node visits are the canonical work measure
-    const float4 *nodes4 = ldu(&sc.node4);
-    const uint32_t nn4 = ldu(&sc.nnode4);
-    const bool use4 = RT_DIFFUSE_BVH4 && !COUNT && nodes4 != nullptr && 3u * ldu(&sc.depth4) + 1u <= (uint32_t)STK;
-    // the 8-bit 4-wide tree (64 B per node): half the node fetches of the binary tree per ray
-    const float4 *q4 = ldu(&sc.qnode4);
-    const bool useq = RT_DIFFUSE_QBVH4 && !COUNT && q4 != nullptr && 3u * ldu(&sc.depth4) + 1u <= (uint32_t)STK;
     const float *T = ldu(&sc.T);
     const uint32_t *type = ldu(&sc.type);
     const uint32_t *mdesc = ldu(&sc.mdesc);
@@ -92,12 +283,10 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total,
     L.o = L.d = mk3(0.f, 0.f, 0.f);
     lane_start(L, nleaf);
     uint32_t my_i = 0, my_r = 0, wraps = 0;
-    uint32_t pend = 0u;  // a parked leaf entry (RT_LEAF_DEFER), 0 = none
     while (true) {
         // finish lanes whose traversal ended: periodic wrap (as trace_loop: at most 32 traces), else write
         if (busy && !trav) {
             bool done = true;
-            if (RT_Q4_LATE_ERR && L.budget == RT_BUDGET_BAD) atomicOr(err, 2);
             if (nbbox) {
                 float bt = nearest_face(sc, L.o, L.d, L.best_t);
                 if (bt > 0.f && wraps < 31) {
@@ -192,58 +381,12 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total,
         // phase: the waiting lanes test their leaves together (the intersection code runs with many lanes
         // active instead of once per node step for the few lanes that reached a leaf)
         const uint32_t floor_lanes = drained ? 1u : RT_REFILL_BELOW;
-        if (RT_LEAF_DEFER && !COUNT) {
-        // A lane that reaches a leaf parks it (pend) and goes on with its next entry, so it keeps taking node
-        // steps; it waits only when it reaches a second leaf or runs out of entries (L.ni = RT_DEFER_END).  The
-        // leaf phase tests the parked leaves and the leaves lanes wait at, many lanes at a time, one leaf per
-        // lane per phase.  (The counting variant keeps the plain order, whose node visits are the canonical
-        // work measure.)
-        while (true) {
-            while (true) {
-                if (trav && pend == 0u && (L.ni & RT_LEAF_BIT) && L.ni != RT_DEFER_END) {
-                    pend = L.ni;
-                    if (lane_pop<STK, LSTK>(L, stk, ovf, stride)) L.ni = RT_DEFER_END;
-                }
-                const bool inner = trav && !(L.ni & RT_LEAF_BIT);
-                const uint64_t mi = __ballot(inner);
-                if (mi == 0 || (uint32_t)__popcll(__ballot(trav && !inner)) >= RT_LEAF_BATCH_PARKED) break;
-                if (inner && (useq   ? lane_node4q<STK, LSTK, RT_Q4_FLAT_DIFFUSE != 0>(q4, nn4, L, stk, ovf, stride, err, cnt)
-                              : use4 ? lane_node4<STK, LSTK>(nodes4, nn4, L, stk, ovf, stride, err, cnt)
-                                     : lane_node<STK, LSTK>(nodes, nleaf, L, stk, ovf, stride, err, cnt))) {
-                    if (pend != 0u) L.ni = RT_DEFER_END;
-                    else trav = false;
-                }
-            }
-            for (int round = 0; !RT_LEAF_ONE_ROUND || round < 1; round++) {
-                const bool atleaf = trav && (L.ni & RT_LEAF_BIT) && L.ni != RT_DEFER_END;
-                const bool work = trav && (pend != 0u || atleaf);
-                if (__ballot(work) == 0) break;
-                if (work) {
-                    uint32_t slot_unused;
-                    cnt.prims++;
-                    if (pend != 0u) {
-                        test_leaf<false, MK>(recs, pend & ~RT_LEAF_BIT, L.o, L.d, 1e-5f, my_i,
-                                                              L.best_t, L.best, slot_unused);
-                        pend = 0u;
-                    } else {
-                        test_leaf<false, MK>(recs, L.ni & ~RT_LEAF_BIT, L.o, L.d, 1e-5f, my_i,
-                                                              L.best_t, L.best, slot_unused);
-                        if (lane_pop<STK, LSTK>(L, stk, ovf, stride)) L.ni = RT_DEFER_END;
-                    }
-                }
-                if (trav && pend == 0u && L.ni == RT_DEFER_END) trav = false;
-            }
-            if ((uint32_t)__popcll(__ballot(trav)) < floor_lanes) break;
-        }
-        } else {
         while (true) {
             while (true) {
                 const bool inner = trav && !(L.ni & RT_LEAF_BIT);
                 const uint64_t mi = __ballot(inner);
                 if (mi == 0 || (uint32_t)__popcll(__ballot(trav && !inner)) >= RT_LEAF_BATCH) break;
-                if (inner && (useq   ? lane_node4q<STK, LSTK, RT_Q4_FLAT_DIFFUSE != 0>(q4, nn4, L, stk, ovf, stride, err, cnt)
-                              : use4 ? lane_node4<STK, LSTK>(nodes4, nn4, L, stk, ovf, stride, err, cnt)
-                                     : lane_node<STK, LSTK>(nodes, nleaf, L, stk, ovf, stride, err, cnt)))
+                if (inner && lane_node<STK, LSTK>(nodes, nleaf, L, stk, ovf, stride, err, cnt))
                     trav = false;
             }
             while (true) {
@@ -252,7 +395,6 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total,
                 if (leaf && lane_leaf<STK, LSTK>(recs, L, 1e-5f, my_i, stk, ovf, stride, cnt)) trav = false;
             }
             if ((uint32_t)__popcll(__ballot(trav)) < floor_lanes) break;
-        }
         }
     }
     add_stats(stats, cnt, nray);
@@ -497,8 +639,6 @@ __global__ __launch_bounds__(256, RT_GATHER_WAVES_PER_EU) void k_gather_chan(con
 int launch_diffuse(const DiffuseJob *job, uint32_t total, uint32_t depth, uint32_t *counter, int *err,
                    unsigned long long *stats, const LaunchCfg &cfg, int ncu, hipStream_t st, int flags) {
     if (total == 0) return 0;
-    // the stack's first RT_DIFFUSE_LDS_STACK entries live in LDS and the rest in private memory, so its
-    // full depth (RT_STACK) costs no occupancy: one stack size serves the binary and the 4-wide tree
     if (depth + 1 > RT_STACK) {
         set_error("BVH depth " + std::to_string(depth) + " exceeds the traversal stack (" + std::to_string(RT_STACK) + ")");
         return -1;
@@ -510,17 +650,21 @@ int launch_diffuse(const DiffuseJob *job, uint32_t total, uint32_t depth, uint32
     if (stats) {
         // counting variant: 4 waves per block
         with_flags(counting_flags(flags), [&](auto fl) {
-            k_diffuse<4, RT_STACK, true, decltype(fl)::value><<<g, 256, 0, st>>>(job, total, counter, ch, err, stats);
+            k_diffuse_bin<4, RT_STACK, true, decltype(fl)::value><<<g, 256, 0, st>>>(job, total, counter, ch, err, stats);
         });
         LCHECK();
         return 0;
     }
     with_flags(flags, [&](auto fl) {
         constexpr int FL = decltype(fl)::value;
+        if (!(flags & RT_FL_BLK)) {
+            k_diffuse_bin<2, RT_STACK, false, FL><<<grid_for(cfg, ncu, total, 2), 128, 0, st>>>(job, total, counter, ch, err, stats);
+            return;
+        }
         switch (wpb) {
-            case 1: k_diffuse<1, RT_STACK, false, FL><<<g, 64, 0, st>>>(job, total, counter, ch, err, stats); break;
-            case 2: k_diffuse<2, RT_STACK, false, FL><<<g, 128, 0, st>>>(job, total, counter, ch, err, stats); break;
-            default: k_diffuse<4, RT_STACK, false, FL><<<g, 256, 0, st>>>(job, total, counter, ch, err, stats); break;
+            case 1: k_diffuse<1, FL><<<g, 64, 0, st>>>(job, total, counter, ch, err); break;
+            case 2: k_diffuse<2, FL><<<g, 128, 0, st>>>(job, total, counter, ch, err); break;
+            default: k_diffuse<4, FL><<<g, 256, 0, st>>>(job, total, counter, ch, err); break;
         }
     });
     LCHECK();

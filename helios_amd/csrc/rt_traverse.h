@@ -28,43 +28,6 @@
 
 #include "rt_internal.h"
 
-// 4-wide tree for diffuse rays (1) or the binary tree (0); children of a 4-wide node fully sorted by entry
-// distance (1) or only the nearest taken first (0).  On the 1 M-primitive orchard the binary tree is faster
-// (916 ms per series of 5 passes against 956 sorted and 1021 nearest-first): the 4-wide step needs 112 B of
-// node per lane and more registers (6 instead of 7 waves per SIMD) for ~40 % fewer steps.
-#ifndef RT_DIFFUSE_BVH4
-#define RT_DIFFUSE_BVH4 0
-#endif
-#ifndef RT_DIFFUSE_QBVH4
-#define RT_DIFFUSE_QBVH4 1
-#endif
-#ifndef RT_CAST_QBVH4
-#define RT_CAST_QBVH4 1
-#endif
-#ifndef RT_Q4_EAGER
-#define RT_Q4_EAGER 1
-#endif
-// BVH4 pushes without branches into a spare LDS row per lane (the per-lane stacks then hold LSTK + 1 rows)
-#ifndef RT_PUSH_SPARE
-#define RT_PUSH_SPARE 1
-#endif
-#ifndef RT_BVH4_SORT
-#define RT_BVH4_SORT 1
-#endif
-// 8-bit node steps check the step budget and the link without a branch (the kernel reports a failed lane
-// when it finishes) and test the stack bound only on the pushes that can exceed it: 626 -> 611 ms for the
-// orchard's five diffuse passes
-#ifndef RT_Q4_LATE_ERR
-#define RT_Q4_LATE_ERR 1
-#endif
-#define RT_BUDGET_BAD 0xFFFFFFFFu
-// Diffuse rays take the 8-bit node step with the pop read issued beside the node load and no branch on the
-// hit-child count (611 -> 600 ms for the orchard's five passes); castRays keep the branching step, which is
-// faster for their long rays (3,112 against 2,700 Mrays/s)
-#ifndef RT_Q4_FLAT_DIFFUSE
-#define RT_Q4_FLAT_DIFFUSE 1
-#endif
-
 namespace rt {
 
 __device__ __forceinline__ float min3f(float a, float b, float c) { return fminf(fminf(a, b), c); }
@@ -578,6 +541,22 @@ __device__ __forceinline__ float nearest_face(const DevScene &sc, v3f o, v3f d, 
     return cf < 0 ? -1.0f : bt;
 }
 
+// The same with the faces read through scalar loads (sc wave-uniform, its faces do not change)
+__device__ __forceinline__ float nearest_face_u(const DevScene &sc, uint32_t nbbox, v3f o, v3f d, float tlim) {
+    float bt = tlim;
+    bool any = false;
+    for (uint32_t f = 0; f < nbbox; f++) {
+        BBoxFace F;
+        const float *src = (const float *)&sc.bbox[f];
+        float *dst = (float *)&F;
+#pragma unroll
+        for (int k = 0; k < (int)(sizeof(BBoxFace) / 4); k++) dst[k] = ldu(src + k);
+        const float t = isect_bbox_face(F, o, d);
+        if (t > 0.0f && t < bt) { bt = t; any = true; }
+    }
+    return any ? bt : -1.0f;
+}
+
 // wrapped origin for a face hit at distance bt (periodic_boundary.glsl:94-111)
 __device__ __forceinline__ v3f wrap_at(const DevScene &sc, v3f o, v3f d, float bt) {
     v3f hp = add3(o, mul3(d, bt));
@@ -748,8 +727,10 @@ __device__ __forceinline__ bool lane_begin(LaneRay &L, const float4 *recs, uint3
 // memory would compile to slower flat accesses that also wait on vector memory)
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
+typedef __attribute__((address_space(3))) float lds_f32;
 #else
 typedef uint32_t lds_u32;
+typedef float lds_f32;
 #endif
 
 // Traversal entries are inner nodes or leaves (RT_LEAF_BIT).  The stack holds its first LSTK entries in
@@ -796,206 +777,6 @@ __device__ __forceinline__ bool lane_node(const float4 *nodes, uint32_t nleaf, L
     return false;
 }
 
-// The hit children of a BVH4 visit (key = entry distance, +inf = missed): the nearest becomes the next
-// entry and the others are pushed (farthest first with RT_BVH4_SORT, else in slot order); the stack empty
-// after no hit ends the traversal (returns true), as does a stack overflow (error bit 1).
-template <int STK, int LSTK>
-__device__ __forceinline__ bool node4_order(LaneRay &L, float *key, uint32_t *lnk, uint32_t nhit, lds_u32 *stk,
-                                            uint32_t *ovf, uint32_t stride, int *err) {
-    if (nhit == 0) return lane_pop<STK, LSTK>(L, stk, ovf, stride);
-#if RT_BVH4_SORT
-    // ascending sort of the four (key, link) pairs; missed children (key +inf) end up last
-    cswap(key[0], lnk[0], key[1], lnk[1]);
-    cswap(key[2], lnk[2], key[3], lnk[3]);
-    cswap(key[0], lnk[0], key[2], lnk[2]);
-    cswap(key[1], lnk[1], key[3], lnk[3]);
-    cswap(key[1], lnk[1], key[2], lnk[2]);
-#if !RT_Q4_LATE_ERR
-    if ((uint32_t)L.sp + nhit - 1 > (uint32_t)STK) {
-        atomicOr(err, 1);
-        return true;
-    }
-#endif
-#if RT_PUSH_SPARE
-    // (with the stack bound tested after this path, the path needs sp + 3 <= LSTK even when LSTK >= STK)
-    if ((!RT_Q4_LATE_ERR && LSTK >= STK) || (uint32_t)L.sp + 3u <= (uint32_t)LSTK) {
-        // every slot a push may use is in LDS: three stores without branches, those beyond the pushed
-        // children aimed at the lane's spare row (index LSTK, which nothing reads); child k < nhit goes to
-        // slot sp + nhit - 1 - k, so the farthest lies deepest and child 1 on top
-#pragma unroll
-        for (int k = 3; k >= 1; k--) {
-            const uint32_t at = (uint32_t)k < nhit ? (uint32_t)L.sp + nhit - 1u - (uint32_t)k : (uint32_t)LSTK;
-            stk[at * stride] = lnk[k];
-        }
-        L.sp += (int)nhit - 1;
-        L.ni = lnk[0];
-        return false;
-    }
-#endif
-#if RT_Q4_LATE_ERR
-    // (the branch-free pushes above cannot overflow: sp + 3 <= LSTK <= STK)
-    if ((uint32_t)L.sp + nhit - 1 > (uint32_t)STK) {
-        atomicOr(err, 1);
-        return true;
-    }
-#endif
-#pragma unroll
-    for (int k = 3; k >= 1; k--) {
-        if ((uint32_t)k < nhit) {
-            if (LSTK >= STK || L.sp < LSTK) stk[(uint32_t)L.sp * stride] = lnk[k];
-            else ovf[L.sp - LSTK] = lnk[k];
-            L.sp++;
-        }
-    }
-    L.ni = lnk[0];
-    return false;
-#else
-    // the nearest hit child next; the other hit children pushed in slot order
-    int m = 0;
-    float km = key[0];
-#pragma unroll
-    for (int k = 1; k < 4; k++)
-        if (key[k] < km) { km = key[k]; m = k; }
-    if ((uint32_t)L.sp + nhit - 1 > (uint32_t)STK) {
-        atomicOr(err, 1);
-        return true;
-    }
-    uint32_t next = lnk[0];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        if (k == m) next = lnk[k];
-        else if (key[k] < INFINITY) {
-            if (LSTK >= STK || L.sp < LSTK) stk[(uint32_t)L.sp * stride] = lnk[k];
-            else ovf[L.sp - LSTK] = lnk[k];
-            L.sp++;
-        }
-    }
-    L.ni = next;
-    return false;
-#endif
-}
-
-// Visit the BVH4 node L.ni: four child boxes against [0, best_t]; the hit children (inner nodes or leaves)
-// in ascending entry distance -- the nearest becomes the next entry, the others are pushed farthest first.
-// Unused slots are +inf point boxes that never pass the test.  Returns true when the traversal has ended.
-template <int STK, int LSTK, typename C>
-__device__ __forceinline__ bool lane_node4(const float4 *nodes4, uint32_t nn4, LaneRay &L, lds_u32 *stk, uint32_t *ovf,
-                                           uint32_t stride, int *err, C &cnt) {
-    if (L.budget-- == 0 || L.ni >= nn4) {
-        atomicOr(err, 2);
-        return true;
-    }
-    cnt.nodes++;
-    const float4 *nd = nodes4 + (size_t)L.ni * 8;
-    const float4 lx = ldc(nd), hx = ldc(nd + 1), ly = ldc(nd + 2), hy = ldc(nd + 3);
-    const float4 lz = ldc(nd + 4), hz = ldc(nd + 5), lk = ldc(nd + 6);
-    float tn[4], tf[4];
-    slab4(lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, L.rp, tn[0], tf[0]);
-    slab4(lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, L.rp, tn[1], tf[1]);
-    slab4(lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, L.rp, tn[2], tf[2]);
-    slab4(lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, L.rp, tn[3], tf[3]);
-    float key[4];
-    uint32_t lnk[4] = {__float_as_uint(lk.x), __float_as_uint(lk.y), __float_as_uint(lk.z), __float_as_uint(lk.w)};
-    uint32_t nhit = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const bool h = fmaxf(tn[k], 0.f) <= fminf(tf[k], L.best_t);
-        key[k] = h ? tn[k] : INFINITY;
-        nhit += h ? 1u : 0u;
-    }
-    return node4_order<STK, LSTK>(L, key, lnk, nhit, stk, ovf, stride, err);
-}
-
-// Visit the 8-bit BVH4 node L.ni (64 B: see k_q4 in rt_scene.hip).  A child bound q decodes in t-space as
-// (o + q 2^e - ray origin) / dir = q (2^e / dir) + (o - ray origin) / dir: one convert and one fma per bound
-// after a multiply and an fma per axis.  The decoded boxes contain the float boxes, and the t rounding is a
-// few ulps of the scene scale, far inside the leaf boxes' padding, so no ray a float box passes is culled
-// and the hits are those of the float trees.
-__device__ __forceinline__ float qbyte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xFFu); }
-
-template <int STK, int LSTK, bool FLAT, typename C>
-__device__ __forceinline__ bool lane_node4q(const float4 *q4, uint32_t nn4, LaneRay &L, lds_u32 *stk, uint32_t *ovf,
-                                            uint32_t stride, int *err, C &cnt) {
-#if RT_Q4_LATE_ERR
-    // a spent step budget or a link outside the tree ends the trace without a branch: the read goes to
-    // node 0 and the budget becomes RT_BUDGET_BAD, which the kernel reports when the lane finishes
-    const bool bad = L.budget == 0u || L.ni >= nn4;
-    L.budget = bad ? RT_BUDGET_BAD : L.budget - 1u;
-    const uint32_t ni = bad ? 0u : L.ni;
-#else
-    if (L.budget-- == 0 || L.ni >= nn4) {
-        atomicOr(err, 2);
-        return true;
-    }
-    const uint32_t ni = L.ni;
-    constexpr bool bad = false;
-#endif
-    cnt.nodes++;
-    const float4 *nd = q4 + (size_t)ni * 4;
-    const float4 f0 = ldc(nd), f1 = ldc(nd + 1), f2 = ldc(nd + 2), f3 = ldc(nd + 3);
-    // FLAT: the entry a pop would take is read now, so its latency hides under the node's (a lane whose
-    // stack top is not in LDS reads its spare row and takes the general path below)
-    const uint32_t sp0 = (uint32_t)L.sp;
-    uint32_t popv = 0u;
-    if (FLAT) popv = stk[((sp0 != 0u && sp0 <= (uint32_t)LSTK) ? sp0 - 1u : (uint32_t)LSTK) * stride];
-    const uint32_t meta = __float_as_uint(f0.w);
-    const uint32_t nch = meta >> 24;
-    // 2^e as a float from the biased exponent byte (e + 127 in [1, 254])
-    const float sx = __uint_as_float((meta & 0xFFu) << 23), sy = __uint_as_float(((meta >> 8) & 0xFFu) << 23),
-                sz = __uint_as_float(((meta >> 16) & 0xFFu) << 23);
-    const float Ax = sx * L.rp.ix, Ay = sy * L.rp.iy, Az = sz * L.rp.iz;
-    const float Bx = fmaf(f0.x, L.rp.ix, -L.rp.ox), By = fmaf(f0.y, L.rp.iy, -L.rp.oy),
-                Bz = fmaf(f0.z, L.rp.iz, -L.rp.oz);
-#if RT_Q4_EAGER
-    // keep the link words' load beside the box words' (the compiler would otherwise sink it into the
-    // branch that pushes, a second dependent round trip per step)
-    asm volatile("" ::"v"(f2.z), "v"(f2.w), "v"(f3.x), "v"(f3.y));
-#endif
-    const uint32_t wlx = __float_as_uint(f1.x), whx = __float_as_uint(f1.y), wly = __float_as_uint(f1.z),
-                   why = __float_as_uint(f1.w), wlz = __float_as_uint(f2.x), whz = __float_as_uint(f2.y);
-    float key[4];
-    uint32_t lnk[4] = {__float_as_uint(f2.z), __float_as_uint(f2.w), __float_as_uint(f3.x), __float_as_uint(f3.y)};
-    uint32_t nhit = 0;
-    // per axis, the bound word nearer the origin: the lower bounds when the direction is positive (A > 0:
-    // t rises with q), else the upper ones.  t(near) = min(t(lo), t(hi)) exactly, so the entry and exit
-    // distances equal the min/max form's with one select per axis instead of a min and a max per child.
-    const bool sx_pos = L.rp.ix >= 0.f, sy_pos = L.rp.iy >= 0.f, sz_pos = L.rp.iz >= 0.f;
-    const uint32_t nwx = sx_pos ? wlx : whx, fwx = sx_pos ? whx : wlx;
-    const uint32_t nwy = sy_pos ? wly : why, fwy = sy_pos ? why : wly;
-    const uint32_t nwz = sz_pos ? wlz : whz, fwz = sz_pos ? whz : wlz;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float tn = max3f(fmaf(qbyte(nwx, k), Ax, Bx), fmaf(qbyte(nwy, k), Ay, By), fmaf(qbyte(nwz, k), Az, Bz));
-        const float tf = min3f(fmaf(qbyte(fwx, k), Ax, Bx), fmaf(qbyte(fwy, k), Ay, By), fmaf(qbyte(fwz, k), Az, Bz));
-        const bool h = (uint32_t)k < nch && fmaxf(tn, 0.f) <= fminf(tf, L.best_t);
-        key[k] = h ? tn : INFINITY;
-        nhit += h ? 1u : 0u;
-    }
-    if (FLAT && sp0 + 3u <= (uint32_t)LSTK) {
-        // no branch on the number of hit children: the sorted children are pushed into the rows above the
-        // stack top (those beyond the hit children into the spare row), and the next entry is the nearest
-        // hit child or, with none, the popped entry; the pushes write rows >= sp0, never the one popped
-        cswap(key[0], lnk[0], key[1], lnk[1]);
-        cswap(key[2], lnk[2], key[3], lnk[3]);
-        cswap(key[0], lnk[0], key[2], lnk[2]);
-        cswap(key[1], lnk[1], key[3], lnk[3]);
-        cswap(key[1], lnk[1], key[2], lnk[2]);
-#pragma unroll
-        for (int k = 3; k >= 1; k--) {
-            const uint32_t at = (uint32_t)k < nhit ? sp0 + nhit - 1u - (uint32_t)k : (uint32_t)LSTK;
-            stk[at * stride] = lnk[k];
-        }
-        L.ni = nhit != 0u ? lnk[0] : popv;
-        L.sp = (int)(nhit != 0u ? sp0 + nhit - 1u : (sp0 != 0u ? sp0 - 1u : 0u));
-        return (nhit == 0u && sp0 == 0u) || bad;
-    }
-#if RT_Q4_LATE_ERR
-    return node4_order<STK, LSTK>(L, key, lnk, nhit, stk, ovf, stride, err) || bad;
-#else
-    return node4_order<STK, LSTK>(L, key, lnk, nhit, stk, ovf, stride, err);
-#endif
-}
-
 // Test the leaf entry L.ni (closest accepted hit, ties to the lower primitive index), then pop.
 template <int STK, int LSTK, typename C>
 __device__ __forceinline__ bool lane_leaf(const float4 *recs, LaneRay &L, float tmin, uint32_t skip,
@@ -1004,6 +785,137 @@ __device__ __forceinline__ bool lane_leaf(const float4 *recs, LaneRay &L, float 
     uint32_t slot_unused;
     test_leaf<false, C::flags>(recs, L.ni & ~RT_LEAF_BIT, L.o, L.d, tmin, skip, L.best_t, L.best, slot_unused);
     return lane_pop<STK, LSTK>(L, stk, ovf, stride);
+}
+
+// ------------------------------------------------------------------------------------------------
+// block tree (rt_types.h): resumable per-lane traversal
+// ------------------------------------------------------------------------------------------------
+// One lane's ray: origin, direction, reciprocal direction and origin x reciprocal, closest hit so far, the
+// next link to visit (RT_BLK_DONE: none left) and the rows in use of the lane's stack.
+struct BlkRay {
+    v3f o, d;
+    float ix, iy, iz, ox, oy, oz;
+    float best_t;
+    uint32_t best, ni, sp;
+};
+
+// A lane's stack: row r of the wave's LDS array (lane stride 4 B, row stride 4 x `stride`), rows from ROWS on
+// in the lane's private array.  Row 0 holds RT_BLK_DONE, so taking the top entry of an empty stack ends the
+// trace without a test of its own.  The tree's depth bounds the rows (3 per level): the launchers choose
+// this traversal only when they fit RT_STACK.
+template <int ROWS>
+__device__ __forceinline__ uint32_t blk_pop(BlkRay &L, const lds_u32 *stk, const uint32_t *ovf, uint32_t stride) {
+    L.sp--;
+    return L.sp < (uint32_t)ROWS ? stk[L.sp * stride] : ovf[L.sp - ROWS];
+}
+
+// Reciprocal of a direction component for the box tests: any value within a few ulps does (a box is padded by
+// 4e-6 of the scene's extent); a component near 0 gives a slab +-1e18 times as far as the origin is from its
+// planes, beyond every hit.
+__device__ __forceinline__ float blk_rcp(float d) {
+    return copysignf(fminf(__builtin_amdgcn_rcpf(fabsf(d)), 1e18f), d);
+}
+
+__device__ __forceinline__ void blk_start(BlkRay &L, lds_u32 *stk) {
+    L.ox = L.o.x * L.ix;
+    L.oy = L.o.y * L.iy;
+    L.oz = L.o.z * L.iz;
+    L.best_t = 1e30f;
+    L.best = RT_MISS;
+    L.ni = 0u;
+    L.sp = 1u;
+    stk[0] = RT_BLK_DONE;
+}
+
+__device__ __forceinline__ float qbyte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xFFu); }
+__device__ __forceinline__ int max3i(int a, int b, int c) { return max(max(a, b), c); }
+__device__ __forceinline__ int med3i(int a, int b, int c) { return max(min(a, b), min(max(a, b), c)); }
+
+// Visit the node block L.ni: four child boxes against [0, best_t]; the hit children are pushed farthest first and
+// the nearest (or, with none hit, the stack's top entry) becomes the next link.
+//
+// The traversals are bound by the issue of VALU instructions (a wave's step takes about as many cycles as its
+// instructions need at 8 waves per SIMD), and fma, mul, add and bit operations take about half the cycles of
+// min/max, compares, selects, shifts and conversions here.  So: a child bound q decodes in t-space as
+// q (2^e / dir) + (o - ray origin) / dir, one convert and one fma; one select per axis picks the bound word
+// nearer the origin instead of a min and a max per child; each hit child is one 32-bit key, the bits of its
+// entry distance with the low byte replaced by its link code (v_perm), so the order of four children takes
+// eight min / med / max and no selects of links, and a link is base + (key & 0xC1); pushes need no branches:
+// the three farthest keys are stored above the stack's top whether they are hits or not (a key that is not
+// lies above the new top).  Keys of missed children are 0x80000000: the smallest as int, so last in the
+// descending order, and above every hit as unsigned, so never the nearest.
+template <int ROWS>
+__device__ __forceinline__ void blk_node_step(const char *blk, BlkRay &L, lds_u32 *stk, uint32_t *ovf, uint32_t stride) {
+    const uint4 *nd = (const uint4 *)(blk + L.ni);
+    const uint4 a = nd[0], b = nd[1], c = nd[2];
+    // the entry a pop would take, read beside the node
+    const uint32_t sp0 = L.sp;
+    uint32_t popv = stk[min(sp0 - 1u, (uint32_t)ROWS - 1u) * stride];
+    const float Ax = __uint_as_float(a.w & 0x7F800000u) * L.ix;
+    const float Ay = __uint_as_float((a.w << 8) & 0x7F800000u) * L.iy;
+    const float Az = __uint_as_float((a.w << 16) & 0x7F800000u) * L.iz;
+    const float Bx = fmaf(__uint_as_float(a.x), L.ix, -L.ox), By = fmaf(__uint_as_float(a.y), L.iy, -L.oy),
+                Bz = fmaf(__uint_as_float(a.z), L.iz, -L.oz);
+    const bool px = L.ix >= 0.f, py = L.iy >= 0.f, pz = L.iz >= 0.f;
+    const uint32_t nwx = px ? b.x : b.y, fwx = px ? b.y : b.x;
+    const uint32_t nwy = py ? b.z : b.w, fwy = py ? b.w : b.z;
+    const uint32_t nwz = pz ? c.x : c.y, fwz = pz ? c.y : c.x;
+    int key[4];
+    uint32_t n = sp0 - 1u;  // becomes the rows in use after the step
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float tn = fmaxf(max3f(fmaf(qbyte(nwx, k), Ax, Bx), fmaf(qbyte(nwy, k), Ay, By), fmaf(qbyte(nwz, k), Az, Bz)), 0.f);
+        const float tf = fminf(min3f(fmaf(qbyte(fwx, k), Ax, Bx), fmaf(qbyte(fwy, k), Ay, By), fmaf(qbyte(fwz, k), Az, Bz)), L.best_t);
+        const bool h = tn <= tf;
+        // bytes 3..1 of tn over byte k of the codes
+        const uint32_t kb = __builtin_amdgcn_perm(__float_as_uint(tn), c.z, 0x07060500u + (uint32_t)k);
+        key[k] = h ? (int)kb : (int)0x80000000u;
+        n += h ? 1u : 0u;
+    }
+    const int hi = max3i(key[0], key[1], key[2]), mid = med3i(key[0], key[1], key[2]),
+              lo = min(min(key[0], key[1]), key[2]);
+    const uint32_t e0 = (uint32_t)max(hi, key[3]), e1 = (uint32_t)med3i(hi, mid, key[3]), e2 = (uint32_t)med3i(mid, lo, key[3]);
+    const uint32_t nearest = min(min(min((uint32_t)key[0], (uint32_t)key[1]), (uint32_t)key[2]), (uint32_t)key[3]);
+    const uint32_t base = c.w;
+    if (sp0 + 3u <= (uint32_t)ROWS) {
+        lds_u32 *top = stk + sp0 * stride;
+        top[0] = base + (e0 & 0xC1u);
+        top[stride] = base + (e1 & 0xC1u);
+        top[2 * stride] = base + (e2 & 0xC1u);
+    } else {
+        // rows beyond the LDS part
+        const uint32_t e[3] = {e0, e1, e2};
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const uint32_t r = sp0 + (uint32_t)k;
+            if (r < n) {
+                if (r < (uint32_t)ROWS) stk[r * stride] = base + (e[k] & 0xC1u);
+                else ovf[r - ROWS] = base + (e[k] & 0xC1u);
+            }
+        }
+        if (sp0 > (uint32_t)ROWS) popv = ovf[sp0 - 1u - ROWS];
+    }
+    L.ni = (int)nearest >= 0 ? base + (nearest & 0xC1u) : popv;
+    L.sp = n;
+}
+
+// Closest-hit test of the record at link (ties to the lower primitive index)
+template <bool CD, int MK>
+__device__ __forceinline__ void blk_leaf(const char *blk, const float4 *recs, uint32_t link, BlkRay &L, float tmin,
+                                         uint32_t skip, uint32_t &slot) {
+    uint32_t id;
+    float t;
+    const float4 *r = (const float4 *)(blk + (link & ~63u));
+    // castRays takes a patch or triangle beyond 1e-6 and a voxel at 1e-6 or beyond
+    // (CD/src/CollisionDetection_RayTracing.cpp:1562, 1595, 1681)
+    if (leaf_hit_at<CD, MK>(r, recs, L.o, L.d, skip, id, t) &&
+        (t > tmin || (CD && t == tmin && (__float_as_uint(ldc(r).w) & RT_VOXEL_BIT)))) {
+        if (t < L.best_t || (t == L.best_t && L.best != RT_MISS && id < L.best)) {
+            L.best_t = t;
+            L.best = id;
+            slot = link;
+        }
+    }
 }
 
 // The result does not depend on the visiting order: a primitive hit at t <= the final closest t lies in

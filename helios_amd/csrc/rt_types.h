@@ -16,6 +16,8 @@
 #define RT_FL_WT 2
 // host-side launch flag (not a kernel template argument): every job of a direct launch has an occlusion grid
 #define RT_FL_GRIDS 4
+// host-side launch flag: the scene has a block tree whose traversal fits the stack
+#define RT_FL_BLK 8
 #define RT_NOT_LAUNCHED 0xFFFFFFFEu
 #define RT_HIT_BOTTOM 0x80000000u
 
@@ -49,8 +51,21 @@ struct DevScene {
     float smax;            // largest |coordinate| of any vertex (scale of FP32 rounding in the scene)
     const uint32_t *mdesc; // [P] mask descriptor index (float4 units from rec) per primitive, RT_MISS = none;
                            // null when no primitive has a texture mask
-    const float4 *qnode4;  // [nnode4][4] the BVH4 nodes with 8-bit child boxes (64 B per node), null = none
+    const uint4 *blk;      // block tree (below), null = none: the traversals then walk the binary tree
 };
+
+// Block tree: the BVH4 in 64-byte blocks, each a node with 8-bit child boxes or a primitive record.  The root is
+// block 0 and the two to four children of a node are consecutive blocks (nodes in breadth-first order).  A link
+// is the byte offset of a block, with bit 0 set for a record.  A node holds, as uint words:
+//   w0 = bits of o.x, o.y, o.z; e_x + 127 in bits 23-30, e_y + 127 in bits 15-22, e_z + 127 in bits 7-14
+//   w1 = lo.x, hi.x, lo.y, hi.y: byte k = child k's bound in units of 2^e from o
+//   w2 = lo.z, hi.z; byte k = (64 k | record bit) of child k; byte offset of the children
+// An unused child is an empty box (lower bound 255, upper bound 0) with child 0's code: a ray so far away that
+// the two bounds round to one distance would visit child 0 again, which changes no closest hit.
+// 32-bit byte offsets reach 2^26 blocks (about 45 million primitives); a larger scene has no block tree.
+#define RT_BLK_REC 1u
+#define RT_BLK_DONE 0xFFFFFFFFu
+#define RT_BLK_MAX 0x3FFFFFFull
 
 // Occlusion grid of one collimated-source direction: every traced primitive's padded projection onto the
 // plane perpendicular to the direction, binned into a uniform grid (CSR: start[cell] .. start[cell + 1]
