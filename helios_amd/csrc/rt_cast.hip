@@ -70,8 +70,9 @@ __device__ __forceinline__ void cast_result(unsigned long long my_r, uint32_t h,
 #ifndef RT_CAST_WAVES_PER_EU
 #define RT_CAST_WAVES_PER_EU 1
 #endif
+// stack rows in LDS: 20 KB a workgroup, which eight of them fill the CU's 160 KB with
 #ifndef RT_CAST_ROWS
-#define RT_CAST_ROWS 16
+#define RT_CAST_ROWS 20
 #endif
 // castRaysSoA (CD/src/CollisionDetection_RayTracing.cpp:551-680, 980-1080): closest hit of each ray with
 // the CD predicates.  Persistent waves take chunks of rays from a counter and keep 64 rays in flight: a lane
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
                                               unsigned long long *counter, uint32_t chunk, int *err) {
     constexpr int ROWS = RT_CAST_ROWS;
     __shared__ uint32_t stk_all[ROWS * WPB * 64];
-    uint32_t ovf[RT_STACK - ROWS];
+    uint32_t ovf[RT_BLK_OVF(ROWS)];
     lds_u32 *stk = (lds_u32 *)stk_all + threadIdx.x;
     const uint32_t stride = WPB * 64;
     const DevScene &sc = *scp;
@@ -99,7 +100,8 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
     bool drained = false, busy = false;
     BlkRay L;
     L.o = L.d = mk3(0.f, 0.f, 0.f);
-    L.ix = L.iy = L.iz = L.ox = L.oy = L.oz = 0.f;
+    blk_direction(L, 0.f, 0.f, 0.f);
+    L.ox = L.oy = L.oz = 0.f;
     L.best_t = 0.f;
     L.best = RT_MISS;
     L.ni = RT_BLK_DONE;
@@ -131,9 +133,9 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
                 L.o = mk3(O[r * 3], O[r * 3 + 1], O[r * 3 + 2]);
                 L.d = mk3(D[r * 3], D[r * 3 + 1], D[r * 3 + 2]);
                 // a cast ray may start far outside the scene, where an ulp of the reciprocal counts: divide
-                L.ix = fabsf(L.d.x) > 1e-18f ? 1.0f / L.d.x : copysignf(1e18f, L.d.x);
-                L.iy = fabsf(L.d.y) > 1e-18f ? 1.0f / L.d.y : copysignf(1e18f, L.d.y);
-                L.iz = fabsf(L.d.z) > 1e-18f ? 1.0f / L.d.z : copysignf(1e18f, L.d.z);
+                blk_direction(L, fabsf(L.d.x) > 1e-18f ? 1.0f / L.d.x : copysignf(1e18f, L.d.x),
+                              fabsf(L.d.y) > 1e-18f ? 1.0f / L.d.y : copysignf(1e18f, L.d.y),
+                              fabsf(L.d.z) > 1e-18f ? 1.0f / L.d.z : copysignf(1e18f, L.d.z));
                 blk_start(L, stk);
                 L.best_t = tstart;
                 my_r = r;
@@ -147,9 +149,8 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
         while (true) {
             while (true) {
                 const bool inner = !(L.ni & RT_BLK_REC);
-                if (__builtin_amdgcn_ballot_w64(inner) == 0 ||
-                    (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(!inner && L.ni != RT_BLK_DONE)) >= RT_LEAF_BATCH)
-                    break;
+                const uint64_t minner = __builtin_amdgcn_ballot_w64(inner);
+                if (minner == 0 || wave_popc(__builtin_amdgcn_ballot_w64(L.ni != RT_BLK_DONE) & ~minner) >= RT_LEAF_BATCH) break;
                 if (++steps > max_steps) {
                     atomicOr(err, 2);
                     L.ni = RT_BLK_DONE;
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
                     L.ni = blk_pop<ROWS>(L, stk, ovf, stride);
                 }
             }
-            if ((uint32_t)__popcll(__builtin_amdgcn_ballot_w64(L.ni != RT_BLK_DONE)) < floor_lanes) break;
+            if ((uint32_t)wave_popc(__builtin_amdgcn_ballot_w64(L.ni != RT_BLK_DONE)) < floor_lanes) break;
         }
     }
 }

@@ -443,16 +443,15 @@ __global__ void k_c4_write(uint32_t count, uint32_t level_base, uint32_t next_ba
 }
 
 // Blocks (rt_types.h) from the float BVH4 nodes (128 B).  Per node: the union box of its children as the
-// origin o and a power-of-two step s_a = 2^e_a per axis with 255 s_a >= extent; a child bound is stored as
-// floor((lo - o) / s) and ceil((hi - o) / s), so the decoded box o + q s contains the float box exactly
-// (the differences and quotients are exact in double: floats differ by a double-exact amount, s is a power
-// of two).
-__device__ __forceinline__ int q_exponent(double ext) {
-    // smallest e in [-126, 127] with 255 * 2^e >= ext
+// origin o and a step s_a per axis with 255 s_a >= extent; a child bound is stored as the last step at or below it
+// and the first at or above it, in double, so the decoded box o + q s contains the float box.
+// Smallest exponent e in [-126, 103] with 255 m 2^e >= ext (m in [1, 2))
+__device__ __forceinline__ int q_exponent(double ext, double m) {
     if (!(ext > 0.0)) return -126;
     int x;
-    (void)frexp(ext / 255.0, &x);  // ext / 255 = m 2^x with m in [0.5, 1): 2^x > ext / 255
-    return x < -126 ? -126 : (x > 127 ? 127 : x);
+    const double f = frexp(ext / (255.0 * m), &x);  // ext / (255 m) = f 2^x with f in [0.5, 1)
+    if (f == 0.5) x--;
+    return x < -126 ? -126 : (x > 103 ? 103 : x);
 }
 
 // base[t]: block of node t's first child
@@ -460,28 +459,34 @@ __device__ __forceinline__ void blk_node(uint32_t t, const float4 *__restrict__ 
                                          uint4 *__restrict__ dst, int *bad) {
     const float4 *o = node4 + (size_t)t * 8;
     const uint32_t cnt = __float_as_uint(o[7].x);
-    uint32_t org[3], ex[3], wl[3], wh[3];
-    for (int a = 0; a < 3; a++) {
+    uint32_t org[3], wl[3], wh[3], w = 0u;
+    // y, z, x: each step's mantissa holds what is in the word below its exponent
+    for (int q = 0; q < 3; q++) {
+        const int a = q == 0 ? 1 : (q == 1 ? 2 : 0);
         const float4 l = o[2 * a], h = o[2 * a + 1];
         const float lo[4] = {l.x, l.y, l.z, l.w}, hi[4] = {h.x, h.y, h.z, h.w};
         float u0 = INFINITY, u1 = -INFINITY;
         for (uint32_t k = 0; k < 4; k++)
             if (k < cnt) { u0 = fminf(u0, lo[k]); u1 = fmaxf(u1, hi[k]); }
-        const int e = q_exponent((double)u1 - (double)u0);
-        const double s = ldexp(1.0, e);
+        const uint32_t mant = q == 0 ? 0u : (q == 1 ? w << 15 : w);
+        const int e = q_exponent((double)u1 - (double)u0, (double)__uint_as_float(0x3F800000u | mant));
+        w |= (uint32_t)(e + 127 + 24) << (q == 0 ? 0 : (q == 1 ? 8 : 23));
+        const double s = (double)__uint_as_float(((uint32_t)(e + 127) << 23) | mant);
         wl[a] = wh[a] = 0u;
         for (uint32_t k = 0; k < 4; k++) {
             double ql = 255.0, qh = 0.0;  // unused child: an empty box
             if (k < cnt) {
-                ql = floor(((double)lo[k] - (double)u0) / s);
-                qh = ceil(((double)hi[k] - (double)u0) / s);
+                const double dl = (double)lo[k] - (double)u0, dh = (double)hi[k] - (double)u0;
+                ql = floor(dl / s);
+                qh = ceil(dh / s);
+                if (ql * s > dl) ql -= 1.0;  // (rounded quotients)
+                if (qh * s < dh) qh += 1.0;
                 if (!(ql >= 0.0 && qh <= 255.0 && ql <= qh)) atomicOr(bad, 1);
             }
             wl[a] |= (uint32_t)fmin(fmax(ql, 0.0), 255.0) << (8 * k);
             wh[a] |= (uint32_t)fmin(fmax(qh, 0.0), 255.0) << (8 * k);
         }
         org[a] = __float_as_uint(u0);
-        ex[a] = (uint32_t)(e + 127);
     }
     const float4 lk4 = o[6];
     const uint32_t lk[4] = {__float_as_uint(lk4.x), __float_as_uint(lk4.y), __float_as_uint(lk4.z),
@@ -491,7 +496,7 @@ __device__ __forceinline__ void blk_node(uint32_t t, const float4 *__restrict__ 
         const uint32_t c = k < cnt ? k : 0u;
         code |= ((c << 6) | ((lk[c] & RT_LEAF_BIT) ? RT_BLK_REC : 0u)) << (8 * k);
     }
-    dst[0] = make_uint4(org[0], org[1], org[2], (ex[0] << 23) | (ex[1] << 15) | (ex[2] << 7));
+    dst[0] = make_uint4(org[0], org[1], org[2], w);
     dst[1] = make_uint4(wl[0], wh[0], wl[1], wh[1]);
     dst[2] = make_uint4(wl[2], wh[2], code, 64u * base[t]);
     dst[3] = make_uint4(0u, 0u, 0u, 0u);

@@ -11,33 +11,44 @@ namespace rt {
 // idle for the longest ray of a fixed group of 64.  Every ray is traced exactly as a plain per-ray
 // trace_loop() would trace it; only the assignment of rays to lanes and steps differs.
 //
-// k_diffuse walks the block tree.  It is bound by the issue of VALU instructions (see
-// blk_node_step()), so everything else keeps as many lanes as it can in each instruction:
+// k_diffuse walks the block tree.  Two units of a CU bound it together (SQ and TCP counters, 86 ms a pass of the
+// 1,001,600-primitive orchard, 439 M rays): the vector ALU (one instruction per SIMD every 3.1 cycles where the mix
+// needs about 3.3) and the vL1D's address path (a load instruction whose lanes lie on different lines takes 43
+// cycles for 64 lanes whatever its width, 1.5 lanes a cycle: about 90 % of the pass).  So a node is three 16-byte
+// loads (rt_types.h), its step is short (blk_node_step()), and the rest keeps as many lanes as it can in each
+// instruction:
 // - Rays are generated up to 64 at a time with every lane active, into the wave's LDS queue (local sample point
 //   and world direction, 20 B a ray): the hashing, square roots and divisions of a ray (about 1,500 cycles a
 //   wave) ran for the 19 lanes being refilled on average when each refill generated its own rays.  A
 //   primitive's rays are split into equal batches (450 rays: 8 of 56 or 57).
 // - A lane that reaches a record parks it and goes on with its next link, so it keeps taking node steps; it
 //   waits only at a second record or with no links left.  Once RT_LEAF_BATCH_PARKED lanes wait, every parked
-//   record is tested, one per lane, and the node phase goes on.
-// LDS per wave: RT_BLK_ROWS stack rows and the queue's five, 5 KB, which 32 waves fill the CU's 160 KB with.
+//   record is tested, one per lane, and the node phase goes on (6 to 16 lanes swept: 8 best, 16 3 % slower).
+// - Refills start below RT_BLK_REFILL traversing lanes (40 to 58 swept: 48 best on all scenes).
+// A pass of that orchard took 110 ms over 64-byte nodes with explicit links, 87 ms so (the masked kernel on 140,000
+// texture-masked patches, 1,024 rays: 95 to 65 ms).  LDS per wave: RT_BLK_ROWS stack rows and the queue's five; 17 rows let 28 waves
+// share the CU's 160 KB, and 7 waves per SIMD need no spills.  More than 11 entries lie on one lane in 0.6 % of its
+// steps and so on some lane of a wave in a quarter of them; 17 rows against 15 with 8 waves: 427 and 431 ms for
+// the orchard's five passes, 21 rows with 6 waves 459, 26 with 5 waves 506.
 #ifndef RT_LEAF_BATCH_PARKED
 #define RT_LEAF_BATCH_PARKED 8
 #endif
 #ifndef RT_BLK_REFILL
 #define RT_BLK_REFILL 48
 #endif
-#define RT_BLK_ROWS 15
-// Waves per SIMD the compiler must fit the kernel into (the default launch shape, 16 two-wave workgroups per CU,
-// runs 8 per SIMD).  Watertight predicates: 6 (their larger leaf test would spill at 8).
+#ifndef RT_BLK_ROWS
+#define RT_BLK_ROWS 17
+#endif
+// Waves per SIMD the compiler must fit the kernel into.  Watertight predicates: 6 (their larger leaf test would
+// spill).
 #ifndef RT_DIFFUSE_WAVES_PER_EU
-#define RT_DIFFUSE_WAVES_PER_EU 8
+#define RT_DIFFUSE_WAVES_PER_EU 7
 #endif
 #ifndef RT_DIFFUSE_WAVES_PER_EU_WT
 #define RT_DIFFUSE_WAVES_PER_EU_WT 6
 #endif
 #ifndef RT_DIFFUSE_WAVES_PER_EU_MASKED
-#define RT_DIFFUSE_WAVES_PER_EU_MASKED 8
+#define RT_DIFFUSE_WAVES_PER_EU_MASKED 7
 #endif
 // rr / n and rr % n of a ray number rr < n * n: a multiply by ceil(2^32 / n) is exact while n^3 < 2^32
 __device__ __forceinline__ void ray_cell(uint32_t rr, uint32_t n, uint32_t inv, uint32_t &lx, uint32_t &ly) {
@@ -54,7 +65,7 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
     __shared__ uint32_t stk_all[ROWS * WPB * 64];
     __shared__ float queue_all[5 * WPB * 64];
     // stack rows beyond the LDS part, in private memory
-    uint32_t ovf[RT_STACK - ROWS];
+    uint32_t ovf[RT_BLK_OVF(ROWS)];
     lds_u32 *stk = (lds_u32 *)stk_all + threadIdx.x;
     const uint32_t stride = WPB * 64;
     const uint32_t lane = threadIdx.x & 63;
@@ -88,13 +99,15 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
     bool busy = false;
     BlkRay L;
     L.o = L.d = mk3(0.f, 0.f, 0.f);
-    L.ix = L.iy = L.iz = L.ox = L.oy = L.oz = 0.f;
+    blk_direction(L, 0.f, 0.f, 0.f);
+    L.ox = L.oy = L.oz = 0.f;
     L.best_t = 0.f;
     L.best = RT_MISS;
     L.ni = RT_BLK_DONE;
     L.sp = 1u;
     uint32_t my_i = 0, my_r = 0, wraps = 0;
-    uint32_t pend = 0u;  // link of the parked record, 0 = none
+    uint32_t pend = 0u;   // link of the parked record of the lanes in mpend
+    uint64_t mpend = 0u;  // lanes with a parked record (none outside the traversal loop)
     while (true) {
         // finish lanes whose traversal ended: periodic wrap (as trace_loop: at most 32 traces), else write
         if (busy && L.ni == RT_BLK_DONE) {
@@ -200,9 +213,7 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
                     for (int q = 0; q < 12; q++) tm[q] = ldu(Tp + q);
                     L.o = xform3(tm, queue[e], queue[64 + e], 0.0f);
                     L.d = mk3(dx, queue[192 + e], queue[256 + e]);
-                    L.ix = blk_rcp(L.d.x);
-                    L.iy = blk_rcp(L.d.y);
-                    L.iz = blk_rcp(L.d.z);
+                    blk_direction(L, blk_rcp(L.d.x), blk_rcp(L.d.y), blk_rcp(L.d.z));
                     blk_start(L, stk);
                     my_i = op_i;
                     my_r = q_ray + e;
@@ -218,14 +229,16 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
         uint32_t steps = 0;
         while (true) {
             while (true) {
-                if ((L.ni & RT_BLK_REC) && L.ni != RT_BLK_DONE && pend == 0u) {
+                const uint64_t mpark = __builtin_amdgcn_ballot_w64((L.ni & RT_BLK_REC) != 0u) &
+                                       ~__builtin_amdgcn_ballot_w64(L.ni == RT_BLK_DONE) & ~mpend;
+                mpend |= mpark;
+                if (__builtin_amdgcn_inverse_ballot_w64(mpark)) {
                     pend = L.ni;
                     L.ni = blk_pop<ROWS>(L, stk, ovf, stride);
                 }
                 const bool inner = !(L.ni & RT_BLK_REC);
-                if (__builtin_amdgcn_ballot_w64(inner) == 0 ||
-                    (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(!inner && pend != 0u)) >= RT_LEAF_BATCH_PARKED)
-                    break;
+                const uint64_t minner = __builtin_amdgcn_ballot_w64(inner);
+                if (minner == 0 || wave_popc(mpend & ~minner) >= RT_LEAF_BATCH_PARKED) break;
                 if (++steps > max_steps) {
                     atomicOr(err, 2);
                     L.ni = RT_BLK_DONE;
@@ -233,12 +246,12 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
                 }
                 if (inner) blk_node_step<ROWS>(blk, L, stk, ovf, stride);
             }
-            if (pend != 0u) {
+            if (__builtin_amdgcn_inverse_ballot_w64(mpend)) {
                 uint32_t slot_unused;
                 blk_leaf<false, MK>(blk, recs, pend, L, 1e-5f, my_i, slot_unused);
-                pend = 0u;
             }
-            if ((uint32_t)__popcll(__builtin_amdgcn_ballot_w64(L.ni != RT_BLK_DONE)) < floor_lanes) break;
+            mpend = 0;
+            if ((uint32_t)wave_popc(__builtin_amdgcn_ballot_w64(L.ni != RT_BLK_DONE)) < floor_lanes) break;
         }
     }
 }

@@ -795,18 +795,22 @@ __device__ __forceinline__ bool lane_leaf(const float4 *recs, LaneRay &L, float 
 struct BlkRay {
     v3f o, d;
     float ix, iy, iz, ox, oy, oz;
+    uint32_t sx, sy, sz;  // byte selectors of the near bounds (blk_node_step)
     float best_t;
     uint32_t best, ni, sp;
 };
 
-// A lane's stack: row r of the wave's LDS array (lane stride 4 B, row stride 4 x `stride`), rows from ROWS on
-// in the lane's private array.  Row 0 holds RT_BLK_DONE, so taking the top entry of an empty stack ends the
-// trace without a test of its own.  The tree's depth bounds the rows (3 per level): the launchers choose
-// this traversal only when they fit RT_STACK.
+// A lane's stack: row r < ROWS in the wave's LDS array (lane stride 4 B, row stride 4 x `stride`), rows from ROWS on
+// in the lane's private array `ovf`, whose entry 0 is row ROWS - 2 (see the pushes).  Row 0 holds RT_BLK_DONE, so
+// taking the top entry of an empty stack ends the trace without a test of its own.  The tree's depth bounds the
+// rows (3 per level): the launchers choose this traversal only when they fit RT_STACK.
+#define RT_BLK_OVF(ROWS) (RT_STACK + 5 - (ROWS))
 template <int ROWS>
 __device__ __forceinline__ uint32_t blk_pop(BlkRay &L, const lds_u32 *stk, const uint32_t *ovf, uint32_t stride) {
     L.sp--;
-    return L.sp < (uint32_t)ROWS ? stk[L.sp * stride] : ovf[L.sp - ROWS];
+    uint32_t v = stk[min(L.sp, (uint32_t)ROWS - 1u) * stride];
+    if (L.sp >= (uint32_t)ROWS) v = ovf[L.sp - (ROWS - 2)];
+    return v;
 }
 
 // Reciprocal of a direction component for the box tests: any value within a few ulps does (a box is padded by
@@ -827,23 +831,61 @@ __device__ __forceinline__ void blk_start(BlkRay &L, lds_u32 *stk) {
     stk[0] = RT_BLK_DONE;
 }
 
-__device__ __forceinline__ float qbyte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xFFu); }
+// The direction's part of a ray: reciprocals and near-bound selectors
+__device__ __forceinline__ void blk_direction(BlkRay &L, float ix, float iy, float iz) {
+    L.ix = ix;
+    L.iy = iy;
+    L.iz = iz;
+    L.sx = ix >= 0.f ? 0x0C020C00u : 0x0C060C04u;
+    L.sy = iy >= 0.f ? 0x0C020C00u : 0x0C060C04u;
+    L.sz = iz >= 0.f ? 0x0C020C00u : 0x0C060C04u;
+}
+
+// Lanes set in a wave-uniform mask, counted on the scalar unit (the compiler compares __popcll()'s 64-bit result in
+// vector registers)
+__device__ __forceinline__ int wave_popc(uint64_t m) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    int r;
+    asm("s_bcnt1_i32_b64 %0, %1" : "=s"(r) : "s"(m) : "scc");
+    return r;
+#else
+    return __popcll(m);
+#endif
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ int max3i(int a, int b, int c) { int r; asm("v_max3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
+__device__ __forceinline__ int min3i(int a, int b, int c) { int r; asm("v_min3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
+__device__ __forceinline__ int med3i(int a, int b, int c) { int r; asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
+#else
 __device__ __forceinline__ int max3i(int a, int b, int c) { return max(max(a, b), c); }
+__device__ __forceinline__ int min3i(int a, int b, int c) { return min(min(a, b), c); }
 __device__ __forceinline__ int med3i(int a, int b, int c) { return max(min(a, b), min(max(a, b), c)); }
+#endif
+// a 16-bit half of w read as a half-precision number, times m plus a (one v_fma_mix_f32)
+__device__ __forceinline__ float fma_lo(uint32_t w, float m, float a) {
+    return fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)w), m, a);
+}
+__device__ __forceinline__ float fma_hi(uint32_t w, float m, float a) {
+    return fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)), m, a);
+}
 
 // Visit the node block L.ni: four child boxes against [0, best_t]; the hit children are pushed farthest first and
 // the nearest (or, with none hit, the stack's top entry) becomes the next link.
 //
-// The traversals are bound by the issue of VALU instructions (a wave's step takes about as many cycles as its
-// instructions need at 8 waves per SIMD), and fma, mul, add and bit operations take about half the cycles of
-// min/max, compares, selects, shifts and conversions here.  So: a child bound q decodes in t-space as
-// q (2^e / dir) + (o - ray origin) / dir, one convert and one fma; one select per axis picks the bound word
-// nearer the origin instead of a min and a max per child; each hit child is one 32-bit key, the bits of its
-// entry distance with the low byte replaced by its link code (v_perm), so the order of four children takes
-// eight min / med / max and no selects of links, and a link is base + (key & 0xC1); pushes need no branches:
-// the three farthest keys are stored above the stack's top whether they are hits or not (a key that is not
-// lies above the new top).  Keys of missed children are 0x80000000: the smallest as int, so last in the
-// descending order, and above every hit as unsigned, so never the nearest.
+// The step is written for the cycles of its vector instructions (see k_diffuse): fma, mul, add and bit operations
+// take about 2.5 cycles of a SIMD here against 4.3 for min/max, compares, selects, shifts, permutes and 4.7 for byte
+// conversions (measured at 8 waves per SIMD).  So:
+// - a child bound q decodes in t-space as q (s / dir) + (o - ray origin) / dir with the axis' step s.  v_perm takes the bounds nearer
+//   the origin of two children from the lower or upper word (the ray's selector says which) as two half-precision
+//   numbers q 2^-24 (a byte under a zero byte is that denormal), and v_fma_mix multiplies and adds with the 2^24
+//   in the stored step: 170 cycles for the 24 bounds against 204 with selects, byte conversions and fma;
+// - each hit child is one 32-bit key, the bits of its entry distance with the low byte replaced by its link code
+//   (v_perm), so the order of four children takes eight min / med / max and no selects of links, and a link is
+//   base + the key's low byte;
+// - pushes need no branches: the three farthest keys are stored above the stack's top whether they are hits or
+//   not (a key that is not lies above the new top).  Keys of missed children are 0x80000000: the smallest as int,
+//   so last in the descending order, and above every hit as unsigned, so never the nearest.
 template <int ROWS>
 __device__ __forceinline__ void blk_node_step(const char *blk, BlkRay &L, lds_u32 *stk, uint32_t *ovf, uint32_t stride) {
     const uint4 *nd = (const uint4 *)(blk + L.ni);
@@ -851,51 +893,56 @@ __device__ __forceinline__ void blk_node_step(const char *blk, BlkRay &L, lds_u3
     // the entry a pop would take, read beside the node
     const uint32_t sp0 = L.sp;
     uint32_t popv = stk[min(sp0 - 1u, (uint32_t)ROWS - 1u) * stride];
-    const float Ax = __uint_as_float(a.w & 0x7F800000u) * L.ix;
-    const float Ay = __uint_as_float((a.w << 8) & 0x7F800000u) * L.iy;
-    const float Az = __uint_as_float((a.w << 16) & 0x7F800000u) * L.iz;
+    // the three steps: the word itself, and its two low bytes shifted to the exponent (rt_types.h)
+    const float Ax = __uint_as_float(a.w) * L.ix, Ay = fabsf(__uint_as_float(a.w << 23)) * L.iy,
+                Az = __uint_as_float(a.w << 15) * L.iz;
     const float Bx = fmaf(__uint_as_float(a.x), L.ix, -L.ox), By = fmaf(__uint_as_float(a.y), L.iy, -L.oy),
                 Bz = fmaf(__uint_as_float(a.z), L.iz, -L.oz);
-    const bool px = L.ix >= 0.f, py = L.iy >= 0.f, pz = L.iz >= 0.f;
-    const uint32_t nwx = px ? b.x : b.y, fwx = px ? b.y : b.x;
-    const uint32_t nwy = py ? b.z : b.w, fwy = py ? b.w : b.z;
-    const uint32_t nwz = pz ? c.x : c.y, fwz = pz ? c.y : c.x;
+    float tn[4], tf[4];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        // children k and k + 2: byte k and k + 2 of the bound words
+        const uint32_t o = 0x00010001u * (uint32_t)k;
+        const uint32_t nx = __builtin_amdgcn_perm(b.y, b.x, L.sx + o), fx = __builtin_amdgcn_perm(b.x, b.y, L.sx + o);
+        const uint32_t ny = __builtin_amdgcn_perm(b.w, b.z, L.sy + o), fy = __builtin_amdgcn_perm(b.z, b.w, L.sy + o);
+        const uint32_t nz = __builtin_amdgcn_perm(c.y, c.x, L.sz + o), fz = __builtin_amdgcn_perm(c.x, c.y, L.sz + o);
+        tn[k] = fmaxf(max3f(fma_lo(nx, Ax, Bx), fma_lo(ny, Ay, By), fma_lo(nz, Az, Bz)), 0.f);
+        tf[k] = fminf(min3f(fma_lo(fx, Ax, Bx), fma_lo(fy, Ay, By), fma_lo(fz, Az, Bz)), L.best_t);
+        tn[k + 2] = fmaxf(max3f(fma_hi(nx, Ax, Bx), fma_hi(ny, Ay, By), fma_hi(nz, Az, Bz)), 0.f);
+        tf[k + 2] = fminf(min3f(fma_hi(fx, Ax, Bx), fma_hi(fy, Ay, By), fma_hi(fz, Az, Bz)), L.best_t);
+    }
     int key[4];
     uint32_t n = sp0 - 1u;  // becomes the rows in use after the step
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const float tn = fmaxf(max3f(fmaf(qbyte(nwx, k), Ax, Bx), fmaf(qbyte(nwy, k), Ay, By), fmaf(qbyte(nwz, k), Az, Bz)), 0.f);
-        const float tf = fminf(min3f(fmaf(qbyte(fwx, k), Ax, Bx), fmaf(qbyte(fwy, k), Ay, By), fmaf(qbyte(fwz, k), Az, Bz)), L.best_t);
-        const bool h = tn <= tf;
+        const bool h = tn[k] <= tf[k];
         // bytes 3..1 of tn over byte k of the codes
-        const uint32_t kb = __builtin_amdgcn_perm(__float_as_uint(tn), c.z, 0x07060500u + (uint32_t)k);
+        const uint32_t kb = __builtin_amdgcn_perm(__float_as_uint(tn[k]), c.z, 0x07060500u + (uint32_t)k);
         key[k] = h ? (int)kb : (int)0x80000000u;
         n += h ? 1u : 0u;
     }
-    const int hi = max3i(key[0], key[1], key[2]), mid = med3i(key[0], key[1], key[2]),
-              lo = min(min(key[0], key[1]), key[2]);
+    const int hi = max3i(key[0], key[1], key[2]), mid = med3i(key[0], key[1], key[2]), lo = min3i(key[0], key[1], key[2]);
     const uint32_t e0 = (uint32_t)max(hi, key[3]), e1 = (uint32_t)med3i(hi, mid, key[3]), e2 = (uint32_t)med3i(mid, lo, key[3]);
     const uint32_t nearest = min(min(min((uint32_t)key[0], (uint32_t)key[1]), (uint32_t)key[2]), (uint32_t)key[3]);
     const uint32_t base = c.w;
+    const uint32_t l0 = base + (e0 & 0xFFu), l1 = base + (e1 & 0xFFu), l2 = base + (e2 & 0xFFu);
     if (sp0 + 3u <= (uint32_t)ROWS) {
         lds_u32 *top = stk + sp0 * stride;
-        top[0] = base + (e0 & 0xC1u);
-        top[stride] = base + (e1 & 0xC1u);
-        top[2 * stride] = base + (e2 & 0xC1u);
+        top[0] = l0;
+        top[stride] = l1;
+        top[2 * stride] = l2;
     } else {
-        // rows beyond the LDS part
-        const uint32_t e[3] = {e0, e1, e2};
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const uint32_t r = sp0 + (uint32_t)k;
-            if (r < n) {
-                if (r < (uint32_t)ROWS) stk[r * stride] = base + (e[k] & 0xC1u);
-                else ovf[r - ROWS] = base + (e[k] & 0xC1u);
-            }
-        }
-        if (sp0 > (uint32_t)ROWS) popv = ovf[sp0 - 1u - ROWS];
+        // near the end of the LDS rows (some lane of a wave in a quarter of the steps): the private array takes the
+        // entries, without branches, and LDS its rows among them
+        uint32_t *o = ovf + (sp0 - (ROWS - 2));
+        o[0] = l0;
+        o[1] = l1;
+        o[2] = l2;
+        if (sp0 < (uint32_t)ROWS) stk[sp0 * stride] = l0;
+        if (sp0 + 1u < (uint32_t)ROWS) stk[(sp0 + 1u) * stride] = l1;
+        if (sp0 > (uint32_t)ROWS) popv = ovf[sp0 - 1u - (ROWS - 2)];
     }
-    L.ni = (int)nearest >= 0 ? base + (nearest & 0xC1u) : popv;
+    L.ni = (int)nearest >= 0 ? base + (nearest & 0xFFu) : popv;
     L.sp = n;
 }
 

@@ -57,8 +57,10 @@ struct DevScene {
 // Block tree: the BVH4 in 64-byte blocks, each a node with 8-bit child boxes or a primitive record.  The root is
 // block 0 and the two to four children of a node are consecutive blocks (nodes in breadth-first order).  A link
 // is the byte offset of a block, with bit 0 set for a record.  A node holds, as uint words:
-//   w0 = bits of o.x, o.y, o.z; e_x + 127 in bits 23-30, e_y + 127 in bits 15-22, e_z + 127 in bits 7-14
-//   w1 = lo.x, hi.x, lo.y, hi.y: byte k = child k's bound in units of 2^e from o
+//   w0 = bits of o.x, o.y, o.z; a word w whose bits are the step s_x 2^24 of the x bounds as a float, those of
+//        |w << 23| s_y 2^24 and those of w << 15 s_z 2^24 (exponents in bits 23-30, 0-7 and 8-15; w's low half is
+//        mantissa of s_x and its low byte of s_z; the 2^24 because the traversal reads a bound q as q 2^-24)
+//   w1 = lo.x, hi.x, lo.y, hi.y: byte k = child k's bound in steps from o
 //   w2 = lo.z, hi.z; byte k = (64 k | record bit) of child k; byte offset of the children
 // An unused child is an empty box (lower bound 255, upper bound 0) with child 0's code: a ray so far away that
 // the two bounds round to one distance would visit child 0 again, which changes no closest hit.
