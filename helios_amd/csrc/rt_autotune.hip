@@ -104,7 +104,7 @@ extern "C" int rt_autotune(rt_ctx *ctx, const rt_scene *scene, const rt_band_req
     DirectJob *dj = (DirectJob *)take(sizeof(DirectJob));
     DiffuseJob *fj = (DiffuseJob *)take(sizeof(DiffuseJob));
     GatherJob *gj = (GatherJob *)take(sizeof(GatherJob));
-    uint32_t *counter = (uint32_t *)take(64);
+    uint32_t *counter = (uint32_t *)take(RT_QUEUE_WORDS * 4);
     int *err = (int *)take(64);
 
     int rc = 0;

@@ -565,8 +565,8 @@ int rt_launch_direct_rays(rt_ctx *ctx, const rt_launch_params *p) {
     uint32_t *dmap = cv.take<uint32_t>(Bl);
     uint8_t *dact = cv.take<uint8_t>(Bl);
     DirectJob *jobs = cv.take<DirectJob>(S);
-    uint32_t *counter = cv.take<uint32_t>(16);
-    int *err = reinterpret_cast<int *>(counter + 8);
+    uint32_t *counter = cv.take<uint32_t>(RT_QUEUE_WORDS + 8);
+    int *err = reinterpret_cast<int *>(counter + RT_QUEUE_WORDS);
     GlassTables gt;
     float *gsum = nullptr;            // [S][P][B_launch][2] strength x cover transmittance per band and face
     GlassDirectJob *gjobs = nullptr;  // [S]
@@ -756,8 +756,8 @@ int rt_launch_diffuse_rays(rt_ctx *ctx, const rt_launch_params *p) {
     DiffuseJob *fjob = cv.take<DiffuseJob>(1);
     GatherJob *gjob = cv.take<GatherJob>(1);
     float *dsky = hsky.empty() ? nullptr : cv.take<float>(hsky.size());
-    uint32_t *counter = cv.take<uint32_t>(16);
-    int *err = reinterpret_cast<int *>(counter + 8);
+    uint32_t *counter = cv.take<uint32_t>(RT_QUEUE_WORDS + 8);
+    int *err = reinterpret_cast<int *>(counter + RT_QUEUE_WORDS);
     GlassTables gt;
     if (glass) {
         gt.cover = cv.take<uint8_t>(P);

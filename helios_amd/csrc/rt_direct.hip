@@ -95,8 +95,8 @@ __global__ __launch_bounds__(WPB * 64, (COUNT || MK) ? 1 : RT_DIRECT_WAVES_PER_E
     const uint32_t lane = threadIdx.x & 63;
     Cnt<COUNT, MK> cnt{};
     uint32_t nray = 0;
-    for (uint32_t first = wave_item(counter, chunk); first < total; first = wave_item(counter, chunk)) {
-        const uint32_t end = min(first + chunk, total);
+    WaveQueue wq(counter, total, chunk);
+    for (uint32_t first, end; wq.take(first, end);) {
         for (uint32_t item = first; item < end; ++item) {
             // job, scene and primitive data are wave-uniform: scalar loads keep them out of VGPRs
             uint32_t j = find_job(jobs, njobs, item);
@@ -238,6 +238,7 @@ __global__ __launch_bounds__(WPB * 64, MK ? 1 : RT_DIRECT_WAVES_PER_EU) void k_d
     const uint32_t lane = threadIdx.x & 63;
     Cnt<false, MK> cnt{};
     // work queue (wave-uniform)
+    WaveQueue wq(counter, total, chunk);
     uint32_t it = 0, it_end = 0;
     bool drained = false;
     // job (wave-uniform): loaded when the wave first takes one of its items
@@ -265,9 +266,7 @@ __global__ __launch_bounds__(WPB * 64, MK ? 1 : RT_DIRECT_WAVES_PER_EU) void k_d
                 // the open primitive has no rays left: open the next item of the queue
                 if (it == it_end) {
                     if (drained) break;
-                    it = wave_item(counter, chunk);
-                    if (it >= total) { drained = true; it = it_end = 0; break; }
-                    it_end = min(it + chunk, total);
+                    if (!wq.take(it, it_end)) { drained = true; it = it_end = 0; break; }
                 }
                 if (jcur == RT_MISS || it < jbegin || it >= jend) {
                     if (__ballot(act) != 0 || (slots & 0xFFu) != 0) { blocked = true; break; }
@@ -401,7 +400,8 @@ __global__ __launch_bounds__(256) void k_direct_src(const DirectJob *__restrict_
     const uint32_t lane = threadIdx.x & 63;
     Cnt<COUNT, MK> cnt{};
     uint32_t nray = 0;
-    for (uint32_t first = wave_item(counter, 1u); first < nitems; first = wave_item(counter, 1u)) {
+    WaveQueue wq(counter, nitems, 1u);
+    for (uint32_t first, end; wq.take(first, end);) {
         const uint32_t item = item_lo + first;
         const DirectJob &J = jobs[find_job(jobs, njobs, item)];
         const DevScene &sc = *J.sc;
@@ -464,7 +464,7 @@ static int launch_direct_t(const DirectJob *jobs, uint32_t njobs, uint32_t total
                            bool grids) {
     if (total == 0) return 0;
     const uint32_t ch = std::max(cfg.chunk, 1u);
-    k_zero_u32<<<1, 1, 0, st>>>(counter);
+    k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
     uint32_t wpb = cfg.waves_per_block;
     uint32_t g = grid_for(cfg, ncu, total, wpb);
     if (RT_DIRECT_QUEUE && grids && !stats) {
@@ -510,7 +510,7 @@ static int launch_direct_src_t(const DirectJob *jobs, uint32_t njobs, uint32_t i
                                uint32_t depth, uint32_t *counter, int *err, unsigned long long *stats, int ncu,
                                hipStream_t st) {
     if (nitems == 0) return 0;
-    k_zero_u32<<<1, 1, 0, st>>>(counter);
+    k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
     uint64_t g64 = std::min<uint64_t>((uint64_t)4 * ncu, ((uint64_t)nitems + 3) / 4);
     uint32_t g = (uint32_t)std::max<uint64_t>(g64, 1);
     if (stats)

@@ -67,7 +67,8 @@ __global__ __launch_bounds__(256) void k_direct_glass(const GlassDirectJob *__re
     const uint32_t lane = threadIdx.x & 63;
     const GlassCtx G = *gp;
     NoCntT<MK> cnt{};
-    for (uint32_t item = wave_item(counter, 1u); item < total; item = wave_item(counter, 1u)) {
+    WaveQueue wq(counter, total, 1u);
+    for (uint32_t item, end; wq.take(item, end);) {
         uint32_t j = 0;
         {
             uint32_t lo = 0, hi = njobs;  // last job with dj.item_begin <= item
@@ -172,7 +173,8 @@ __global__ __launch_bounds__(256) void k_diffuse_glass(const DiffuseJob *__restr
     const uint32_t n = F.n, nn = n * n, seed = F.seed, C = J.C;
     const float strength = rdiv(1.0f, (float)nn);
     NoCntT<MK> cnt{};
-    for (uint32_t item = wave_item(counter, 1u); item < total; item = wave_item(counter, 1u)) {
+    WaveQueue wq(counter, total, 1u);
+    for (uint32_t item, end; wq.take(item, end);) {
         uint32_t i = item - F.item_begin;
         if (F.order) i = F.order[i];
         const uint32_t ty = sc.type[i];
@@ -280,7 +282,7 @@ int launch_direct_glass(const GlassDirectJob *jobs, uint32_t njobs, uint32_t tot
         set_error("BVH depth " + std::to_string(depth) + " exceeds the traversal stack (" + std::to_string(RT_STACK) + ")");
         return -1;
     }
-    k_zero_u32<<<1, 1, 0, st>>>(counter);
+    k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
     const uint32_t grid = (uint32_t)std::min<uint64_t>((uint64_t)4 * ncu, (total + 3) / 4);
     with_flags(flags, [&](auto fl) {
         constexpr int FL = decltype(fl)::value;
@@ -298,7 +300,7 @@ int launch_diffuse_glass(const DiffuseJob *fj, const GatherJob *gj, uint32_t tot
         set_error("BVH depth " + std::to_string(depth) + " exceeds the traversal stack (" + std::to_string(RT_STACK) + ")");
         return -1;
     }
-    k_zero_u32<<<1, 1, 0, st>>>(counter);
+    k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
     const uint32_t grid = (uint32_t)std::min<uint64_t>((uint64_t)4 * ncu, (total + 3) / 4);
     with_flags(flags, [&](auto fl) {
         constexpr int FL = decltype(fl)::value;

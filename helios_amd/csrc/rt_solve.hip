@@ -550,8 +550,8 @@ int run_solve(SolveCtx &sx, const Scene &S, const rt_band_request &q, const SunS
     DiffuseJob *fjobs = cv.take<DiffuseJob>(1 + maxdepth);
     GatherJob *gjobs = cv.take<GatherJob>(1 + maxdepth);
     float *dsky = hsky.empty() ? nullptr : cv.take<float>(hsky.size());
-    uint32_t *counter = cv.take<uint32_t>(16);
-    int *err = reinterpret_cast<int *>(counter + 8);
+    uint32_t *counter = cv.take<uint32_t>(RT_QUEUE_WORDS + 8);
+    int *err = reinterpret_cast<int *>(counter + RT_QUEUE_WORDS);
 
     // ---- uploads (pageable host -> device, stream ordered) ----
     CK(hipMemsetAsync(in, 0, PC * 4, st));
@@ -828,8 +828,8 @@ int debug_diffuse_hits(SolveCtx &sx, const Scene &S, uint32_t n, uint32_t seed, 
     Carve cv{(char *)sx.ws.base};
     uint32_t *hits = cv.take<uint32_t>((size_t)P * 2 * nn);
     DiffuseJob *fjob = cv.take<DiffuseJob>(1);
-    uint32_t *counter = cv.take<uint32_t>(16);
-    int *err = reinterpret_cast<int *>(counter + 8);
+    uint32_t *counter = cv.take<uint32_t>(RT_QUEUE_WORDS + 8);
+    int *err = reinterpret_cast<int *>(counter + RT_QUEUE_WORDS);
     DiffuseJob fj{};
     fj.sc = S.d; fj.n = n; fj.seed = seed; fj.hits = hits; fj.item_begin = 0; fj.P = P;
     CK(hipMemsetAsync(err, 0, 4, st));
@@ -856,8 +856,8 @@ int debug_direct_sums(SolveCtx &sx, const Scene &S, uint32_t d, uint32_t seed, u
     Carve cv{(char *)sx.ws.base};
     float *sums = cv.take<float>((size_t)nsrc * P * 2);
     DirectJob *jobs = cv.take<DirectJob>(nsrc);
-    uint32_t *counter = cv.take<uint32_t>(16);
-    int *err = reinterpret_cast<int *>(counter + 8);
+    uint32_t *counter = cv.take<uint32_t>(RT_QUEUE_WORDS + 8);
+    int *err = reinterpret_cast<int *>(counter + RT_QUEUE_WORDS);
     // collimated sources first (their items precede the others')
     std::vector<DirectJob> hj;
     std::vector<float> coldir;

@@ -90,6 +90,7 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
     const uint32_t max_steps = (uint32_t)min(64ull * (ldu(&sc.nnode4) + 8ull), 0xFFFFFFFFull);
     // work queue, open primitive and its ray queue (wave-uniform); the primitive's frame and transform are
     // reloaded (scalar) whenever rays are generated or taken, so they hold no registers across the traversal
+    WaveQueue wq(counter, total, chunk);
     uint32_t it = 0, it_end = 0;
     bool drained = false;
     uint32_t op_i = 0, op_next = 0, op_cnt = 0, op_base = 0, op_m = RT_MISS;
@@ -141,9 +142,7 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
                     // open the next primitive of the work queue
                     if (it == it_end) {
                         if (drained) break;
-                        it = wave_item(counter, chunk);
-                        if (it >= total) { drained = true; it = it_end = 0; break; }
-                        it_end = min(it + chunk, total);
+                        if (!wq.take(it, it_end)) { drained = true; it = it_end = 0; break; }
                     }
                     uint32_t i = it - item_begin;
                     if (order) i = ldu(order + i);
@@ -286,6 +285,7 @@ __global__ __launch_bounds__(WPB * 64) void k_diffuse_bin(const DiffuseJob *__re
     uint32_t *hits = ldu(&job->hits);
     // work queue and open primitive (wave-uniform); the primitive's frame and transform are reloaded
     // (scalar) whenever rays are generated, so they hold no registers across the traversal
+    WaveQueue wq(counter, total, chunk);
     uint32_t it = 0, it_end = 0;
     bool drained = false;
     uint32_t op_i = 0, op_next = 0, op_cnt = 0, op_base = 0, op_m = RT_MISS;
@@ -328,9 +328,7 @@ __global__ __launch_bounds__(WPB * 64) void k_diffuse_bin(const DiffuseJob *__re
                 // open the next primitive of the queue
                 if (it == it_end) {
                     if (drained) break;
-                    it = wave_item(counter, chunk);
-                    if (it >= total) { drained = true; it = it_end = 0; break; }
-                    it_end = min(it + chunk, total);
+                    if (!wq.take(it, it_end)) { drained = true; it = it_end = 0; break; }
                 }
                 uint32_t i = it - item_begin;
                 if (order) i = ldu(order + i);
@@ -437,8 +435,8 @@ template <int CM, bool ACCT>
 __global__ __launch_bounds__(256) void k_gather_rays(const GatherJob *__restrict__ jobs, uint32_t njobs, uint32_t total,
                                                      uint32_t *counter, uint32_t chunk) {
     const uint32_t lane = threadIdx.x & 63;
-    for (uint32_t first = wave_item(counter, chunk); first < total; first = wave_item(counter, chunk)) {
-        const uint32_t end = min(first + chunk, total);
+    WaveQueue wq(counter, total, chunk);
+    for (uint32_t first, end; wq.take(first, end);) {
         for (uint32_t item = first; item < end; ++item) {
             uint32_t j = find_job(jobs, njobs, item);
             const GatherJob &J = jobs[j];
@@ -547,8 +545,8 @@ template <int CB, bool ACCT>
 __global__ __launch_bounds__(256, RT_GATHER_WAVES_PER_EU) void k_gather_chan(const GatherJob *__restrict__ jobs, uint32_t njobs, uint32_t total,
                                                      uint32_t *counter, uint32_t chunk) {
     const uint32_t lane = threadIdx.x & 63;
-    for (uint32_t first = wave_item(counter, chunk); first < total; first = wave_item(counter, chunk)) {
-        const uint32_t end = min(first + chunk, total);
+    WaveQueue wq(counter, total, chunk);
+    for (uint32_t first, end; wq.take(first, end);) {
         for (uint32_t item = first; item < end; ++item) {
             uint32_t j = find_job(jobs, njobs, item);
             const GatherJob &J = jobs[j];
@@ -657,7 +655,7 @@ int launch_diffuse(const DiffuseJob *job, uint32_t total, uint32_t depth, uint32
         return -1;
     }
     const uint32_t ch = std::max(cfg.chunk, 1u);
-    k_zero_u32<<<1, 1, 0, st>>>(counter);
+    k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
     uint32_t wpb = cfg.waves_per_block;
     uint32_t g = grid_for(cfg, ncu, total, wpb);
     if (stats) {
@@ -707,7 +705,7 @@ int launch_gather(const GatherJob *jobs, uint32_t njobs, uint32_t total, uint32_
                   const LaunchCfg &cfg, int ncu, hipStream_t st, bool acct) {
     if (total == 0) return 0;
     const uint32_t ch = std::max(cfg.chunk, 1u);
-    k_zero_u32<<<1, 1, 0, st>>>(counter);
+    k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
     uint32_t g = grid_for(cfg, ncu, total, 4);
     return acct ? launch_gather_t<true>(jobs, njobs, total, cmax, counter, g, ch, st)
                 : launch_gather_t<false>(jobs, njobs, total, cmax, counter, g, ch, st);

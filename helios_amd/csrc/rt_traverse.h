@@ -632,15 +632,66 @@ __device__ __forceinline__ bool packet_occluded(const DevScene &sc, v3f o, v3f d
     return occl;
 }
 
-// Next work item of this wave.  No lane-divergent branch around the fetch: every lane issues the
-// atomic (lane 0 adds 1, the others 0) and lane 0's old value is broadcast as a scalar.  A
-// `if (lane == 0) atomicAdd` + shuffle lets the compiler split the persistent loop into a lane-0
-// loop and a lanes-1..63 loop that re-processes item 0 forever.
-__device__ __forceinline__ uint32_t wave_item(uint32_t *counter, uint32_t chunk) {
-    uint32_t lane = threadIdx.x & 63;
-    uint32_t item = atomicAdd(counter, lane == 0 ? chunk : 0u);
-    return __builtin_amdgcn_readfirstlane(item);
-}
+// A wave's view of the work queue of a persistent launch: items [0, total) in chunks of `chunk`.  What bounds a
+// queue is its atomics on one address, 5 to 12 ns each and one after the other: as much as a whole item of the
+// direct kernel (225 rays of a primitive over an occlusion grid: 4.6 ns an item, now 1.9) or of a gather.  So
+// - a launch with at most one chunk a wave uses none: wave w takes chunk w (1,601 primitives: four gathers 0.202
+//   to 0.057 ms, direct 0.060 to 0.027);
+// - a launch of RT_QUEUE_SPLIT chunks a wave or more splits the items into RT_QUEUES segments, each with its own
+//   counter in its own line.  A workgroup starts on the segment of its XCD (workgroups go to the XCDs in turn), so
+//   an XCD's L2 holds one range of the leaf order instead of an eighth of every range, and goes on to the other
+//   segments in turn once its own is empty (1 M primitives x 64 directions: direct 297 to 136 ms; five gathers of
+//   1 M primitives 58 to 24).  Larger chunks on one counter did the same for these but cost the diffuse kernel
+//   and small scenes up to half their time.
+// Looking at a counter before adding to it, past the first segment, made the direct kernel 4 % slower.
+// All members are wave-uniform.
+struct WaveQueue {
+    uint32_t *ctr;
+    uint32_t total, chunk, seg, mask, q, left;
+    __device__ __forceinline__ WaveQueue(uint32_t *counter, uint32_t total_, uint32_t chunk_)
+        : ctr(counter), total(total_), chunk(chunk_) {
+        const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x >> 6);
+        const bool split = gridDim.x >= RT_QUEUES && (uint64_t)total >= RT_QUEUE_SPLIT * waves * chunk;
+        mask = split ? RT_QUEUES - 1u : 0u;
+        seg = split ? (total + RT_QUEUES - 1u) / RT_QUEUES : total;
+        q = blockIdx.x & mask;
+        left = mask + 1u;
+        if (waves * chunk >= total) {
+            ctr = nullptr;
+            q = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+        }
+    }
+    // Adds the chunk to counter word w from lane 0 alone and returns its old value: 64 lanes adding to one word are
+    // 64 atomics (114 ns a fetch, one lane's 5 to 12).
+    __device__ __forceinline__ uint32_t fetch(uint32_t *w) const {
+        uint32_t x = 0;
+        if ((threadIdx.x & 63) == 0) x = __hip_atomic_fetch_add(w, chunk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return __builtin_amdgcn_readfirstlane(x);
+    }
+    // The next items [b, e) of this wave; false once all are taken.
+    __device__ __forceinline__ bool take(uint32_t &b, uint32_t &e) {
+        if (!ctr) {
+            const uint64_t x = (uint64_t)q * chunk;
+            if (left == 0u || x >= total) return false;
+            left = 0u;
+            b = (uint32_t)x;
+            e = min(b + chunk, total);
+            return true;
+        }
+        while (left != 0u) {
+            const uint32_t x = fetch(ctr + q * RT_QUEUE_STRIDE);
+            const uint32_t lo = q * seg;
+            if (x < seg && lo + x < total) {
+                b = lo + x;
+                e = min(b + chunk, min(lo + seg, total));
+                return true;
+            }
+            left--;
+            q = (q + 1u) & mask;
+        }
+        return false;
+    }
+};
 
 template <typename J>
 __device__ __forceinline__ uint32_t find_job(const J *jobs, uint32_t njobs, uint32_t item) {
@@ -971,7 +1022,7 @@ __device__ __forceinline__ void blk_leaf(const char *blk, const float4 *recs, ui
 
 static __global__ void k_zero_u64(unsigned long long *p) { *p = 0ull; }
 
-static __global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
+static __global__ void k_zero_queue(uint32_t *p) { p[threadIdx.x] = 0u; }
 
 // ------------------------------------------------------------------------------------------------
 // launchers
