@@ -3,6 +3,10 @@
 
 namespace rt {
 
+// two neighbouring words, two neighbouring list entries in one load
+typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+
 // Occlusion of one shadow ray through the source's grid: test the primitives binned in the cell of the
 // origin's projection with the BVH traversal's predicate (t in (1e-4, 1e30], not the origin primitive) and
 // stop at the first hit.  Non-periodic scenes only (the grid is not built otherwise).
@@ -14,8 +18,9 @@ __device__ __forceinline__ void grid_cell(const SunGrid &G, v3f o, uint32_t &b, 
     const int cx = fx < 0.f ? 0 : (fx > (float)(G.nx - 1) ? (int)(G.nx - 1) : (int)fx);
     const int cy = fy < 0.f ? 0 : (fy > (float)(G.ny - 1) ? (int)(G.ny - 1) : (int)fy);
     const uint32_t c = (uint32_t)cy * G.nx + (uint32_t)cx;
-    b = G.start[c] - G.sbase;
-    e = G.start[c + 1] - G.sbase;
+    const u32x2_a4 be = *(const u32x2_a4 *)(G.start + c);
+    b = be.x - G.sbase;
+    e = be.y - G.sbase;
 }
 
 // Candidates p and p + 1 (when p + 1 < e) of a cell list: is either accepted as an occluder?  Both
@@ -226,17 +231,34 @@ __global__ __launch_bounds__(WPB * 64, (COUNT || MK) ? 1 : RT_DIRECT_WAVES_PER_E
 // LDS that counts its lit rays; the primitive's sums are written once its last ray has ended.  A job change
 // (another direction, grid and output) waits until the rays in flight have ended.  Every ray is tested
 // exactly as in k_direct, and the sums are the same count x strength.
+// The vector ALU bounds it (1 M primitives x 225 rays x 64 directions, 14.4 G rays: 9.1e10 wave instructions in
+// 122 ms, one per SIMD every 3.3 cycles), so lanes must not idle and work that decides nothing must not run:
+// - rays are generated up to 64 at a time with every lane active, into the wave's LDS queue, together with the first
+//   two entries of their cell's list; a ray with nothing above it is counted lit there and never queued;
+// - a lane tests one candidate a step (two a step tested the second in vain whenever the first hit), and the
+//   origin's own entry, known by its leaf slot, is passed over without loading its record;
+// - a cell's start and end are one 8-byte load and a pair of entries one 16-byte load (2.5e9 load instructions
+//   where two candidates a step took 3.8e9).
+// That batch's direct pass took 136 ms with two candidates a step and rays generated by the lanes being refilled,
+// 121 ms so.  Refills start below RT_DQ_REFILL scanning lanes (32 to 56 swept: 40 best by 2 %).
+// The lists are sorted by descending key (SunGrid), which the scan's end relies on.
 #define RT_DQ_SLOTS 8
+#ifndef RT_DQ_REFILL
+#define RT_DQ_REFILL 40
+#endif
 template <int WPB, int MK>
 __global__ __launch_bounds__(WPB * 64, MK ? 1 : RT_DIRECT_WAVES_PER_EU) void k_direct_q(const DirectJob *__restrict__ jobs,
                                                                                         uint32_t njobs, uint32_t total,
                                                                                         uint32_t *counter, uint32_t chunk) {
+    typedef Cnt<false, MK> C;
     __shared__ uint32_t ring_all[3 * RT_DQ_SLOTS * WPB];  // per wave: lit count, primitive, strength of each slot
+    __shared__ float4 qo_all[64 * WPB];                   // queued rays: origin, depth along the source direction,
+    __shared__ uint4 qe_all[64 * WPB];                    // the next two list entries
+    __shared__ uint2 qp_all[64 * WPB];                    // and the list positions after them
     uint32_t *lit = ring_all + (threadIdx.x >> 6) * 3 * RT_DQ_SLOTS;
     uint32_t *sprim = lit + RT_DQ_SLOTS;
     float *sstr = (float *)(lit + 2 * RT_DQ_SLOTS);
-    const uint32_t lane = threadIdx.x & 63;
-    Cnt<false, MK> cnt{};
+    const uint32_t lane = threadIdx.x & 63, qbase = threadIdx.x & ~63u;
     // work queue (wave-uniform)
     WaveQueue wq(counter, total, chunk);
     uint32_t it = 0, it_end = 0;
@@ -246,97 +268,150 @@ __global__ __launch_bounds__(WPB * 64, MK ? 1 : RT_DIRECT_WAVES_PER_EU) void k_d
     const DevScene *scp = nullptr;
     const SunGrid *grid = nullptr;
     const uint32_t *order = nullptr;
+    const uint2 *ents = nullptr;
+    const float4 *recs = nullptr;
+    bool leaf_items = false;
     float *out = nullptr;
     v3f dir = mk3(0.f, 0.f, 0.f);
-    // open primitive (wave-uniform) and the slots in use (bit mask; a slot's bit 8 + k: its sums are lit from
-    // the top)
-    uint32_t op_i = 0, op_next = 0, op_cnt = 0, op_slot = 0, op_mdi = RT_MISS, slots = 0;
+    // open primitive, the batch of its rays in the queue (wave-uniform) and the slots in use (bit mask; a slot's
+    // bit 8 + k: its sums are lit from the top)
+    uint32_t op_i = 0, op_own = RT_MISS, op_next = 0, op_cnt = 0, op_slot = 0, op_mdi = RT_MISS, slots = 0;
+    uint32_t q_next = 0, q_cnt = 0;
     bool op_patch = false;
-    // lane: its ray (origin, depth along the source direction, cell list position), primitive and slot
+    // lane: its ray (origin, depth, current and following list entry, next list position and end), primitive, the
+    // primitive's leaf slot and ring slot
     bool act = false;
     v3f o = mk3(0.f, 0.f, 0.f);
     float depth = 0.f;
-    uint32_t pc = 0, pe = 0, my_i = 0, my_slot = 0;
+    uint32_t ex = RT_MISS, ek = 0, nx = RT_MISS, nk = 0, pn = 0, pe = 0, my_i = 0, my_own = 0, my_slot = 0;
     while (true) {
         bool blocked = false;
         while (true) {
-            const uint64_t idle = __ballot(!act);
+            const uint64_t idle = __builtin_amdgcn_ballot_w64(!act);
             if (idle == 0) break;
-            if (op_next == op_cnt) {
-                // the open primitive has no rays left: open the next item of the queue
-                if (it == it_end) {
-                    if (drained) break;
-                    if (!wq.take(it, it_end)) { drained = true; it = it_end = 0; break; }
-                }
-                if (jcur == RT_MISS || it < jbegin || it >= jend) {
-                    if (__ballot(act) != 0 || (slots & 0xFFu) != 0) { blocked = true; break; }
-                    jcur = find_job(jobs, njobs, it);
-                    const DirectJob &J = jobs[jcur];
-                    jbegin = ldu(&J.item_begin);
-                    jend = jcur + 1 < njobs ? ldu(&jobs[jcur + 1].item_begin) : total;
-                    scp = ldu(&J.sc);
-                    grid = ldu(&J.grid);
-                    order = ldu(&J.order);
-                    out = ldu(&J.out);
-                    d = ldu(&J.d);
-                    Nrays = d * d;
-                    seed = ldu(&J.seed);
-                    dir = nrm3(mk3(ldu(&J.sdir[0]), ldu(&J.sdir[1]), ldu(&J.sdir[2])));
-                    nleaf = ldu(&scp->nleaf);
-                }
-                if ((slots & 0xFFu) == 0xFFu) { blocked = true; break; }
-                uint32_t i = it - jbegin;
-                if (order) i = ldu(order + i);
-                i = __builtin_amdgcn_readfirstlane(i);
-                it++;
-                const uint32_t ty = ldu(ldu(&scp->type) + i);
-                const float4 n4 = ldu(ldu(&scp->nrm) + i);
-                const v3f n = mk3(n4.x, n4.y, n4.z);
-                const uint32_t tw = __float_as_uint(n4.w);
-                const bool top = dot3(dir, n) > 0.0f;
-                if (!traced_type(ty) || tw == 3 || (!top && tw == 0)) {
-                    if (lane == 0) { out[(size_t)i * 2] = 0.f; out[(size_t)i * 2 + 1] = 0.f; }
+            if (q_next == q_cnt) {
+                if (op_next == op_cnt) {
+                    // the open primitive has no rays left: open the next item of the queue
+                    if (it == it_end) {
+                        if (drained) break;
+                        if (!wq.take(it, it_end)) { drained = true; it = it_end = 0; break; }
+                    }
+                    if (jcur == RT_MISS || it < jbegin || it >= jend) {
+                        if (idle != ~0ull || (slots & 0xFFu) != 0) { blocked = true; break; }
+                        jcur = find_job(jobs, njobs, it);
+                        const DirectJob &J = jobs[jcur];
+                        jbegin = ldu(&J.item_begin);
+                        jend = jcur + 1 < njobs ? ldu(&jobs[jcur + 1].item_begin) : total;
+                        scp = ldu(&J.sc);
+                        grid = ldu(&J.grid);
+                        order = ldu(&J.order);
+                        out = ldu(&J.out);
+                        d = ldu(&J.d);
+                        Nrays = d * d;
+                        seed = ldu(&J.seed);
+                        dir = nrm3(mk3(ldu(&J.sdir[0]), ldu(&J.sdir[1]), ldu(&J.sdir[2])));
+                        nleaf = ldu(&scp->nleaf);
+                        ents = ldu(&grid->ents);
+                        recs = ldu(&scp->rec);
+                        leaf_items = order != nullptr && order == ldu(&scp->order);
+                    }
+                    if ((slots & 0xFFu) == 0xFFu) { blocked = true; break; }
+                    uint32_t i = it - jbegin;
+                    op_own = leaf_items && i < nleaf ? i : RT_MISS;
+                    if (order) i = ldu(order + i);
+                    i = __builtin_amdgcn_readfirstlane(i);
+                    it++;
+                    const uint32_t ty = ldu(ldu(&scp->type) + i);
+                    const float4 n4 = ldu(ldu(&scp->nrm) + i);
+                    const v3f n = mk3(n4.x, n4.y, n4.z);
+                    const uint32_t tw = __float_as_uint(n4.w);
+                    const bool top = dot3(dir, n) > 0.0f;
+                    if (!traced_type(ty) || tw == 3 || (!top && tw == 0)) {
+                        if (lane == 0) { out[(size_t)i * 2] = 0.f; out[(size_t)i * 2 + 1] = 0.f; }
+                        continue;
+                    }
+                    const uint32_t sl = (uint32_t)__builtin_ctz(~slots & 0xFFu);
+                    slots |= (1u << sl) | (top ? (0x100u << sl) : 0u);
+                    lit[sl] = 0u;
+                    sprim[sl] = i;
+                    sstr[sl] = rdiv(fabsf(dot3(n, dir)), (float)Nrays);
+                    const uint32_t *mdesc = ldu(&scp->mdesc);
+                    op_mdi = (MK && mdesc) ? ldu(mdesc + i) : RT_MISS;
+                    op_i = i;
+                    op_next = 0;
+                    op_cnt = Nrays;
+                    op_slot = sl;
+                    op_patch = ty == 0 || ty == 3;
                     continue;
                 }
-                const uint32_t sl = (uint32_t)__builtin_ctz(~slots & 0xFFu);
-                slots |= (1u << sl) | (top ? (0x100u << sl) : 0u);
-                lit[sl] = 0u;
-                sprim[sl] = i;
-                sstr[sl] = rdiv(fabsf(dot3(n, dir)), (float)Nrays);
-                const uint32_t *mdesc = ldu(&scp->mdesc);
-                op_mdi = (MK && mdesc) ? ldu(mdesc + i) : RT_MISS;
-                op_i = i;
-                op_next = 0;
-                op_cnt = Nrays;
-                op_slot = sl;
-                op_patch = ty == 0 || ty == 3;
+                // generate the next batch of the open primitive's rays; those whose cell lists nothing above them
+                // are lit, the others enter the queue with their first two entries
+                const uint32_t left = op_cnt - op_next, batches = (left + 63u) >> 6;
+                const uint32_t cnt = (left + batches - 1u) / batches, r = op_next + lane;
+                op_next += cnt;
+                bool islit = false, enter = false;
+                v3f p = mk3(0.f, 0.f, 0.f);
+                float pd = 0.f;
+                uint4 e2 = make_uint4(RT_MISS, 0u, RT_MISS, 0u);
+                uint32_t b = 0, e = 0;
+                if (lane < cnt) {
+                    float spx, spy;
+                    if (direct_origin(recs, op_mdi, op_i, r, d, seed, op_patch, spx, spy)) {
+                        float tm[12];
+                        const float *Tp = ldu(&scp->T) + (size_t)op_i * 16;
+#pragma unroll
+                        for (int q = 0; q < 12; q++) tm[q] = ldu(Tp + q);
+                        p = xform3(tm, spx, spy, 0.0f);
+                        grid_cell(*grid, p, b, e);
+                        pd = p.x * grid->w[0] + p.y * grid->w[1] + p.z * grid->w[2];
+                        if (b < e) {
+                            const u32x4_a8 v = *(const u32x4_a8 *)(ents + b);
+                            e2 = make_uint4(v.x, v.y, v.z, v.w);
+                            enter = __uint_as_float(e2.y) >= pd;
+                            if (b + 1 >= e) e2.z = RT_MISS;
+                        }
+                        islit = !enter;
+                    }
+                }
+                const uint64_t mlit = __builtin_amdgcn_ballot_w64(islit), menter = __builtin_amdgcn_ballot_w64(enter);
+                if (lane == 0 && mlit) atomicAdd(&lit[op_slot], (uint32_t)wave_popc(mlit));
+                if (enter) {
+                    const uint32_t at = qbase + __builtin_amdgcn_mbcnt_hi((uint32_t)(menter >> 32),
+                                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)menter, 0u));
+                    qo_all[at] = make_float4(p.x, p.y, p.z, pd);
+                    qe_all[at] = e2;
+                    qp_all[at] = make_uint2(b + 2, e);
+                }
+                q_next = 0;
+                q_cnt = (uint32_t)wave_popc(menter);
+                __builtin_amdgcn_wave_barrier();
                 continue;
             }
             const uint32_t rank =
                 __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
-            const uint32_t take = min((uint32_t)__popcll(idle), op_cnt - op_next);
+            const uint32_t take = min((uint32_t)wave_popc(idle), q_cnt - q_next);
             if (!act && rank < take) {
-                const uint32_t r = op_next + rank;
-                const float4 *recs = ldu(&scp->rec);
-                float spx, spy;
-                act = direct_origin(recs, op_mdi, op_i, r, d, seed, op_patch, spx, spy);
-                float tm[12];
-                const float *Tp = ldu(&scp->T) + (size_t)op_i * 16;
-#pragma unroll
-                for (int q = 0; q < 12; q++) tm[q] = ldu(Tp + q);
-                o = xform3(tm, spx, spy, 0.0f);
-                grid_cell(*grid, o, pc, pe);
-                depth = o.x * grid->w[0] + o.y * grid->w[1] + o.z * grid->w[2];
+                const uint32_t at = qbase + q_next + rank;
+                const float4 q = qo_all[at];
+                const uint4 e2 = qe_all[at];
+                const uint2 pp = qp_all[at];
+                o = mk3(q.x, q.y, q.z);
+                depth = q.w;
+                ex = e2.x; ek = e2.y; nx = e2.z; nk = e2.w;
+                pn = pp.x;
+                pe = pp.y;
                 my_i = op_i;
+                my_own = op_own;
                 my_slot = op_slot;
+                act = true;
             }
-            op_next += take;
+            q_next += take;
         }
         // write the sums of the primitives none of whose rays remain (the open one once all its rays are out)
         for (uint32_t pend = slots & 0xFFu; pend != 0u; pend &= pend - 1u) {
             const uint32_t sl = (uint32_t)__builtin_ctz(pend);
-            if (sl == op_slot && op_next < op_cnt) continue;
-            if (__ballot(act && my_slot == sl) != 0) continue;
+            if (sl == op_slot && (op_next < op_cnt || q_next < q_cnt)) continue;
+            if (__builtin_amdgcn_ballot_w64(act && my_slot == sl) != 0) continue;
             const uint32_t i = sprim[sl];
             const float sum = lit_sum(lit[sl], sstr[sl]);
             const bool top = (slots >> (8 + sl)) & 1u;
@@ -346,24 +421,48 @@ __global__ __launch_bounds__(WPB * 64, MK ? 1 : RT_DIRECT_WAVES_PER_EU) void k_d
             }
             slots &= ~((1u << sl) | (0x100u << sl));
         }
-        if (__ballot(act) == 0) {
-            if (drained && op_next == op_cnt && (slots & 0xFFu) == 0u) break;
+        if (__builtin_amdgcn_ballot_w64(act) == 0) {
+            if (drained && op_next == op_cnt && q_next == q_cnt && (slots & 0xFFu) == 0u) break;
             continue;
         }
-        // trace until fewer than RT_DIRECT_REFILL lanes scan (all of them when no ray can be handed out)
-        const uint32_t floor_lanes = (blocked || (drained && op_next == op_cnt)) ? 1u : RT_DIRECT_REFILL;
-        const uint2 *ents = grid->ents;
-        const bool sorted = grid->sorted != 0;
-        const float4 *recs = ldu(&scp->rec);
-        while (true) {
+        // trace until fewer than RT_DQ_REFILL lanes scan (all of them when no ray can be handed out)
+        const uint32_t floor_lanes =
+            (blocked || (drained && op_next == op_cnt && q_next == q_cnt)) ? 1u : RT_DQ_REFILL;
+        do {
             if (act) {
-                const int res = pc >= pe ? 2 : grid_pair(ents, sorted, depth, recs, nleaf, pc, pe, o, dir, my_i, cnt);
-                if (res == 2) atomicAdd(&lit[my_slot], 1u);
-                if (res != 0) act = false;
-                else pc += 2;
+                // the entries after this pair, while its last record is on the way
+                u32x4_a8 f = {RT_MISS, 0u, RT_MISS, 0u};
+                const bool fetch = nx == RT_MISS && pn < pe;
+                if (fetch) f = *(const u32x4_a8 *)(ents + pn);
+                const uint32_t k = ex & RT_GRID_SLOT;
+                bool hit = false;
+                if (k != my_own && k < nleaf) {
+                    const float4 *q = recs + (size_t)k * 4;
+                    const float4 a0 = ldc(q), a1 = ldc(q + 1), a2 = ldc(q + 2);
+                    const float4 a3 = (ex & RT_GRID_REC3) ? ldc(q + 3) : make_float4(0.f, 0.f, 0.f, 0.f);
+                    const uint32_t tag = __float_as_uint(a0.w);
+                    float t, ua, ub;
+                    hit = isect_rec_uv<false, C::wt>(a0, a1, a2, a3, (tag & RT_PATCH_BIT) != 0, o, dir, t, ua, ub) &&
+                          (tag & RT_ID_BITS) != my_i && t > 1e-4f && t <= 1e30f;
+                    if (C::mask && hit && (tag & RT_MASK_BIT))
+                        hit = mask_hit_opaque(recs, __float_as_uint(a3.w), (tag & RT_PATCH_BIT) != 0, ua, ub, a1.w, a2.w);
+                }
+                if (fetch) {
+                    ex = f.x; ek = f.y;
+                    nx = pn + 1 < pe ? f.z : RT_MISS;
+                    nk = f.w;
+                    pn += 2;
+                } else {
+                    ex = nx; ek = nk;  // RT_MISS when the list has ended
+                    nx = RT_MISS;
+                }
+                if (hit) act = false;
+                else if (ex == RT_MISS || !(__uint_as_float(ek) >= depth)) {
+                    atomicAdd(&lit[my_slot], 1u);
+                    act = false;
+                }
             }
-            if ((uint32_t)__popcll(__ballot(act)) < floor_lanes) break;
-        }
+        } while ((uint32_t)wave_popc(__builtin_amdgcn_ballot_w64(act)) >= floor_lanes);
     }
 }
 

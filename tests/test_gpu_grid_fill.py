@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from helios_amd import native
+from tests.helpers import small_canopy
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +31,22 @@ def test_mixed_rectangles(ctx, P):
         ctx.set_direct_grids(True)
     assert np.array_equal(sg, sb)
     assert sg.max() > 0
+
+
+@pytest.mark.parametrize("d", [1, 7, 8, 9, 16, 33])
+@pytest.mark.parametrize("predicates", ["reference", "watertight"])
+def test_ray_batches(ctx, d, predicates):
+    """Rays a primitive below, at and above a batch of 64: the grid's decisions are the BVH's, bit for bit."""
+    s = small_canopy(41, 700)
+    g = ctx.scene(s.transforms, s.types, s.twosided)
+    src = [native.sun_direction(z, a) for z, a in ((3, 0), (50, 130), (87, 260))]
+    try:
+        ctx.set_predicates(predicates)
+        ctx.set_direct_grids(True)
+        sg = g.direct_sums(d, 17, src)
+        ctx.set_direct_grids(False)
+        sb = g.direct_sums(d, 17, src)
+    finally:
+        ctx.set_direct_grids(True)
+        ctx.set_predicates("reference")
+    assert np.array_equal(sg, sb)
