@@ -235,7 +235,7 @@ extern "C" int rt_autotune(rt_ctx *ctx, const rt_scene *scene, const rt_band_req
                     default_launch_cfg(1), best[1], best_ms[1], def_ms[1], count);
     if (rc == 0)
         rc = search(st, tm, gather_c,
-                    [&](const LaunchCfg &c) { return launch_gather(gj, 1, sample, C, counter, c, ncu, st); },
+                    [&](const LaunchCfg &c) { return launch_gather(gj, 1, sample, C, counter, c, ncu, st, false, false); },
                     default_launch_cfg(2), best[2], best_ms[2], def_ms[2], count);
     int herr = 0;
     if (rc == 0 && (hipMemcpy(&herr, err, 4, hipMemcpyDeviceToHost) != hipSuccess || herr != 0)) {

@@ -819,7 +819,7 @@ int rt_launch_diffuse_rays(rt_ctx *ctx, const rt_launch_params *p) {
     if (launch_diffuse(fjob, p->launch_count, be.scene.h.depth, counter, err, ctx->sx.stat_ptr(1), ctx->sx.cfg[1],
                        ctx->sx.ncu, st, scene_flags(be.scene, ctx->sx)))
         return -1;
-    if (launch_gather(gjob, 1, p->launch_count, Bl, counter, ctx->sx.cfg[2], ctx->sx.ncu, st)) return -1;
+    if (launch_gather(gjob, 1, p->launch_count, Bl, counter, ctx->sx.cfg[2], ctx->sx.ncu, st, false, gj.sky != nullptr)) return -1;
     return check_err(ctx, err);
 }
 

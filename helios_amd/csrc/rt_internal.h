@@ -88,9 +88,10 @@ int launch_direct_jobs(const DirectJob *hjobs, const DirectJob *jobs_dev, uint32
 // one diffuse job (device pointer) per launch: items [0, total_items) of that job
 int launch_diffuse(const DiffuseJob *job_dev, uint32_t total_items, uint32_t depth, uint32_t *counter, int *err,
                    unsigned long long *stats, const LaunchCfg &cfg, int ncu, hipStream_t st, int flags);
-// acct: the jobs carry energy-bookkeeping outputs (GatherJob.acct / .miss)
+// acct: the jobs carry energy-bookkeeping outputs (GatherJob.acct / .miss); sky: some job has an anisotropic sky
+// (GatherJob.sky); cmax: the jobs' channel count
 int launch_gather(const GatherJob *jobs_dev, uint32_t njobs, uint32_t total_items, uint32_t cmax, uint32_t *counter,
-                  const LaunchCfg &cfg, int ncu, hipStream_t st, bool acct = false);
+                  const LaunchCfg &cfg, int ncu, hipStream_t st, bool acct, bool sky);
 // Solves with translucent covers (GlassCtx g, device): the direct jobs (items ascending by dj.item_begin),
 // one diffuse/scattering pass traced and gathered together, and the covers' pushed shares added to the
 // radiation buffers (PC = P * C).

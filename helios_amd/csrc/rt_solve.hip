@@ -724,7 +724,7 @@ int run_solve(SolveCtx &sx, const Scene &S, const rt_band_request &q, const SunS
         hipEvent_t c2, d2;
         if (ev_pair(sx, c2, d2)) return -1;
         if (c2) CK(hipEventRecord(c2, st));
-        if (launch_gather(gjobs + g, 1, P, C, counter, sx.cfg[2], sx.ncu, st, acct)) return -1;
+        if (launch_gather(gjobs + g, 1, P, C, counter, sx.cfg[2], sx.ncu, st, acct, hg[g].sky != nullptr)) return -1;
         if (d2) { CK(hipEventRecord(d2, st)); tick(sx, 2, c2, d2); }
         if (acct) {
             const uint8_t *act = hg[g].active;

@@ -429,101 +429,124 @@ __device__ __forceinline__ v3f diffuse_dir(const DevScene &sc, uint32_t i, uint3
     return dir;
 }
 
-// ACCT: also record the pass's incident and sky flux densities and the sky-bound ray counts (GatherJob.acct,
-// .miss) for the energy bookkeeping; a separate instance, so the plain gather carries no extra registers.
-template <int CM, bool ACCT>
+// Sums of N lane-private compensated accumulators over the wave (N a power of two up to 64): while more than one
+// accumulator is left, a step hands half of them to the lane's partner and merges the other half, so N accumulators
+// take N - 1 merges and then one per remaining step instead of 6 N.  On return lane l holds the sum of accumulator
+// i whose bits are l's lowest log2(N) bits in reverse order.
+template <int HALF, int OFF, int N>
+__device__ __forceinline__ void reduce_halves(ksum (&v)[N], uint32_t lane) {
+    if constexpr (HALF >= 1) {
+        const bool up = (lane & (uint32_t)OFF) != 0u;
+#pragma unroll
+        for (int j = 0; j < HALF; j++) {
+            const float gs = up ? v[j].s : v[j + HALF].s, gc = up ? v[j].c : v[j + HALF].c;
+            v[j].s = up ? v[j + HALF].s : v[j].s;
+            v[j].c = up ? v[j + HALF].c : v[j].c;
+            v[j].merge(__shfl_xor(gs, OFF, 64), __shfl_xor(gc, OFF, 64));
+        }
+        reduce_halves<HALF / 2, OFF * 2>(v, lane);
+    } else if constexpr (OFF < 64) {
+        v[0].merge(__shfl_xor(v[0].s, OFF, 64), __shfl_xor(v[0].c, OFF, 64));
+        reduce_halves<0, OFF * 2>(v, lane);
+    }
+}
+template <int N>
+__device__ __forceinline__ ksum wave_reduce_many(ksum (&v)[N], uint32_t lane) {
+    reduce_halves<N / 2, 1>(v, lane);
+    return v[0];
+}
+
+constexpr int pow2_up(int n) { int p = 1; while (p < n) p *= 2; return p; }
+
+// One primitive per wave, lanes over its rays, NC channels (the jobs' C).  A lane's row -- the C-vector of a primitive
+// anywhere in the scene -- is loaded whole, in as few instructions as its width needs: such a load costs the vL1D's
+// address path about 0.67 cycles a lane whatever its width up to 16 B.  SKY: the sky is anisotropic.  ACCT: also
+// record the pass's incident and sky flux densities and the sky-bound ray counts (GatherJob.acct, .miss) for the
+// energy bookkeeping.  Both are separate instances, so the plain gather carries no extra registers.
+// The channel count is exact up to 16: a kernel for the next power of two loaded and added channels that are not
+// there.  Five passes of 1 M primitives x 1,024 rays, 3 channels: 24.1 to 11.9 ms; three passes of 200,000 x 100 rays:
+// 4 channels 2.04 to 1.43 ms, 8 channels 3.75 to 1.44.  k_gather_chan (lanes over the channels) takes 5.2 ms for these
+// passes at 9 to 17 channels and this kernel 1.60, 1.62 and 1.81 at 9, 12 and 16; more channels than 16 would not fit
+// the registers.
+template <int NC, bool SKY, bool ACCT>
 __global__ __launch_bounds__(256) void k_gather_rays(const GatherJob *__restrict__ jobs, uint32_t njobs, uint32_t total,
                                                      uint32_t *counter, uint32_t chunk) {
+    constexpr int N = pow2_up(2 * NC);  // accumulators: 2 c + face slot
+    constexpr int NS = ACCT ? pow2_up(NC) : 1;
     const uint32_t lane = threadIdx.x & 63;
     WaveQueue wq(counter, total, chunk);
     for (uint32_t first, end; wq.take(first, end);) {
         for (uint32_t item = first; item < end; ++item) {
-            uint32_t j = find_job(jobs, njobs, item);
-            const GatherJob &J = jobs[j];
-            uint32_t i = item - J.item_begin;
-            if (J.order) i = J.order[i];
-            uint32_t ty = J.sc->type[i];
-            if (!traced_type(ty)) continue;
-            uint32_t nn = J.n * J.n, C = J.C;
-            const uint32_t *w = J.hits + (size_t)i * 2 * nn;
-            ksum acc[2][CM];
-            ksum asky[ACCT ? CM : 1];
+            const GatherJob &J = jobs[find_job(jobs, njobs, item)];
+            uint32_t i = item - ldu(&J.item_begin);
+            const uint32_t *order = ldu(&J.order);
+            if (order) i = ldu(order + i);
+            i = __builtin_amdgcn_readfirstlane(i);
+            const DevScene *sc = ldu(&J.sc);
+            if (!traced_type(ldu(ldu(&sc->type) + i))) continue;
+            const uint32_t n = ldu(&J.n), nn = n * n;
+            const g_u32 *w = (const g_u32 *)(ldu(&J.hits) + (size_t)i * 2 * nn);
+            const g_f32 *otop = (const g_f32 *)ldu(&J.out_top), *obot = (const g_f32 *)ldu(&J.out_bot),
+                        *dfl = (const g_f32 *)ldu(&J.dflux);
+            ksum acc[N], asky[NS];
             uint32_t mt = 0, mb = 0;
 #pragma unroll
+            for (int k = 0; k < N; k++) acc[k].init();
+#pragma unroll
+            for (int k = 0; k < NS; k++) asky[k].init();
+            // one face at a time: an accumulator index that depends on the ray would put the array in memory
+#pragma unroll
             for (int f = 0; f < 2; f++)
+                for (uint32_t r = (uint32_t)f * nn + lane; r < (uint32_t)(f + 1) * nn; r += 64) {
+                    const uint32_t word = w[r];
+                    if (word == RT_NOT_LAUNCHED) continue;
+                    const bool miss = word == RT_MISS;
+                    if (ACCT && miss) { if (f) mb++; else mt++; }
+                    const g_f32 *src = miss ? dfl : ((word & RT_HIT_BOTTOM) ? obot : otop) + (size_t)(word & ~RT_HIT_BOTTOM) * NC;
+                    float row[NC];
 #pragma unroll
-                for (int c = 0; c < CM; c++) acc[f][c].init();
+                    for (int c = 0; c < NC; c++) row[c] = src[c];
+                    if (SKY && miss) {
+                        // anisotropic sky: fd(direction) x diffuse flux (diffuse_raygen.comp:613-625)
+                        const v3f dir = diffuse_dir(*sc, i, r, n, ldu(&J.seed));
+                        const float *sky = ldu(&J.sky);
 #pragma unroll
-            for (int c = 0; c < (ACCT ? CM : 1); c++) asky[c].init();
-            for (uint32_t r = lane; r < 2 * nn; r += 64) {
-                uint32_t word = w[r];
-                if (word == RT_NOT_LAUNCHED) continue;
-                uint32_t slot = r >= nn ? 1u : 0u;
-                if (ACCT && word == RT_MISS) { if (slot) mb++; else mt++; }
-                if (word == RT_MISS && J.sky) {
-                    // anisotropic sky: fd(direction) x diffuse flux (diffuse_raygen.comp:613-625)
-                    const v3f dir = diffuse_dir(*J.sc, i, r, J.n, J.seed);
+                        for (int c = 0; c < NC; c++) row[c] = sky_weight(dir, sky + 9 * c) * row[c];
+                    }
 #pragma unroll
-                    for (int c = 0; c < CM; c++)
-                        if ((uint32_t)c < C) {
-                            float v = sky_weight(dir, J.sky + 9 * c) * J.dflux[c];
-                            if (slot) acc[1][c].add(v); else acc[0][c].add(v);
-                            if (ACCT) asky[ACCT ? c : 0].add(v);
-                        }
-                } else if (word == RT_MISS) {
-#pragma unroll
-                    for (int c = 0; c < CM; c++)
-                        if ((uint32_t)c < C) {
-                            float v = J.dflux[c];
-                            if (slot) acc[1][c].add(v); else acc[0][c].add(v);
-                            if (ACCT) asky[ACCT ? c : 0].add(v);
-                        }
-                } else {
-                    uint32_t h = word & ~RT_HIT_BOTTOM;
-                    const float *src = ((word & RT_HIT_BOTTOM) ? J.out_bot : J.out_top) + (size_t)h * C;
-#pragma unroll
-                    for (int c = 0; c < CM; c++)
-                        if ((uint32_t)c < C) {
-                            float v = src[c];
-                            if (slot) acc[1][c].add(v); else acc[0][c].add(v);
-                        }
+                    for (int c = 0; c < NC; c++) {
+                        acc[2 * c + f].add(row[c]);
+                        if (ACCT && miss) asky[ACCT ? c : 0].add(row[c]);
+                    }
                 }
-            }
-            float strength = rdiv(1.0f, (float)nn);
-#pragma unroll
-            for (int c = 0; c < CM; c++) {
-                wave_reduce(acc[0][c]);
-                wave_reduce(acc[1][c]);
-                if (ACCT) wave_reduce(asky[ACCT ? c : 0]);
-            }
+            const float strength = rdiv(1.0f, (float)nn);
+            // lane l: accumulator k (bits of l reversed) = channel k / 2, face slot k % 2; the two faces of a channel
+            // lie N / 2 lanes apart
+            const ksum mine = wave_reduce_many<N>(acc, lane);
+            const float I1 = mine.value() * strength, I0 = __shfl_xor(I1, N / 2, 64);
+            float Is = 0.f;
             if (ACCT) {
+                // (channel k / 2 lands in the lanes whose lowest bits are that channel's reversed: the same lanes)
+                Is = wave_reduce_many<NS>(asky, lane).value() * strength;
                 for (int off = 32; off > 0; off >>= 1) { mt += __shfl_xor(mt, off); mb += __shfl_xor(mb, off); }
                 if (lane == 0) { J.miss[(size_t)i * 2] = mt; J.miss[(size_t)i * 2 + 1] = mb; }
             }
-            if (lane < C && lane < CM) {
-                float I1 = 0.f, I0 = 0.f, Is = 0.f;
-#pragma unroll
-                for (int c = 0; c < CM; c++)
-                    if ((uint32_t)c == lane) {
-                        I1 = acc[0][c].value(); I0 = acc[1][c].value();
-                        if (ACCT) Is = asky[ACCT ? c : 0].value();
-                    }
-                uint32_t c = lane;
+            const uint32_t k = __brev(lane) >> (32 - __builtin_ctz((unsigned)N));
+            const uint32_t c = k >> 1;
+            if (lane < (uint32_t)(N / 2) && c < (uint32_t)NC) {
                 const bool act = J.active[c] != 0;
-                I1 = I1 * strength;
-                I0 = I0 * strength;
                 if (act) {
-                    uint32_t b = c % J.B;
-                    float rho = J.rho[(size_t)i * J.B + b], tau = J.tau[(size_t)i * J.B + b];
-                    size_t q = (size_t)i * C + c;
+                    const uint32_t B = ldu(&J.B), b = c % B;
+                    float rho = J.rho[(size_t)i * B + b], tau = J.tau[(size_t)i * B + b];
+                    size_t q = (size_t)i * NC + c;
                     J.in[q] += (I1 + I0) * (1.0f - rho - tau);
                     J.st[q] += I1 * rho + I0 * tau;
                     J.sb[q] += I1 * tau + I0 * rho;
                 }
                 if (ACCT) {
-                    const size_t q = ((size_t)i * C + c) * 2;
+                    const size_t q = ((size_t)i * NC + c) * 2;
                     J.acct[q] = act ? I1 + I0 : 0.f;
-                    J.acct[q + 1] = act ? Is * strength : 0.f;
+                    J.acct[q + 1] = act ? Is : 0.f;
                 }
             }
         }
@@ -682,13 +705,29 @@ int launch_diffuse(const DiffuseJob *job, uint32_t total, uint32_t depth, uint32
     return 0;
 }
 
-template <bool ACCT>
+template <bool SKY, bool ACCT>
 static int launch_gather_t(const GatherJob *jobs, uint32_t njobs, uint32_t total, uint32_t cmax, uint32_t *counter,
                            uint32_t g, uint32_t ch, hipStream_t st) {
-    if (cmax <= 1) k_gather_rays<1, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch);
-    else if (cmax <= 2) k_gather_rays<2, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch);
-    else if (cmax <= 4) k_gather_rays<4, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch);
-    else if (cmax <= 8) k_gather_rays<8, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch);
+    if (cmax <= 16)
+        switch (cmax) {
+            case 1: k_gather_rays<1, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 2: k_gather_rays<2, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 3: k_gather_rays<3, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 4: k_gather_rays<4, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 5: k_gather_rays<5, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 6: k_gather_rays<6, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 7: k_gather_rays<7, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 8: k_gather_rays<8, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 9: k_gather_rays<9, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 10: k_gather_rays<10, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 11: k_gather_rays<11, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 12: k_gather_rays<12, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 13: k_gather_rays<13, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 14: k_gather_rays<14, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 15: k_gather_rays<15, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            case 16: k_gather_rays<16, SKY, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch); break;
+            default: break;
+        }
     else if (cmax <= 64) k_gather_chan<1, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch);
     else if (cmax <= 128) k_gather_chan<2, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch);
     else if (cmax <= 192) k_gather_chan<3, ACCT><<<g, 256, 0, st>>>(jobs, njobs, total, counter, ch);
@@ -702,13 +741,16 @@ static int launch_gather_t(const GatherJob *jobs, uint32_t njobs, uint32_t total
 }
 
 int launch_gather(const GatherJob *jobs, uint32_t njobs, uint32_t total, uint32_t cmax, uint32_t *counter,
-                  const LaunchCfg &cfg, int ncu, hipStream_t st, bool acct) {
+                  const LaunchCfg &cfg, int ncu, hipStream_t st, bool acct, bool sky) {
     if (total == 0) return 0;
     const uint32_t ch = std::max(cfg.chunk, 1u);
     k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
     uint32_t g = grid_for(cfg, ncu, total, 4);
-    return acct ? launch_gather_t<true>(jobs, njobs, total, cmax, counter, g, ch, st)
-                : launch_gather_t<false>(jobs, njobs, total, cmax, counter, g, ch, st);
+    if (acct)
+        return sky ? launch_gather_t<true, true>(jobs, njobs, total, cmax, counter, g, ch, st)
+                   : launch_gather_t<false, true>(jobs, njobs, total, cmax, counter, g, ch, st);
+    return sky ? launch_gather_t<true, false>(jobs, njobs, total, cmax, counter, g, ch, st)
+               : launch_gather_t<false, false>(jobs, njobs, total, cmax, counter, g, ch, st);
 }
 
 }  // namespace rt

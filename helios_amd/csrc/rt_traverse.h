@@ -779,9 +779,14 @@ __device__ __forceinline__ bool lane_begin(LaneRay &L, const float4 *recs, uint3
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 typedef __attribute__((address_space(3))) float lds_f32;
+// device-memory values (a pointer read from a job descriptor is generic, and loads through it go the slower flat way)
+typedef __attribute__((address_space(1))) uint32_t g_u32;
+typedef __attribute__((address_space(1))) float g_f32;
 #else
 typedef uint32_t lds_u32;
 typedef float lds_f32;
+typedef uint32_t g_u32;
+typedef float g_f32;
 #endif
 
 // Traversal entries are inner nodes or leaves (RT_LEAF_BIT).  The stack holds its first LSTK entries in
