@@ -231,7 +231,7 @@ __global__ __launch_bounds__(WPB * 64, (COUNT || MK) ? 1 : RT_DIRECT_WAVES_PER_E
 // LDS that counts its lit rays; the primitive's sums are written once its last ray has ended.  A job change
 // (another direction, grid and output) waits until the rays in flight have ended.  Every ray is tested
 // exactly as in k_direct, and the sums are the same count x strength.
-// The vector ALU bounds it (1 M primitives x 225 rays x 64 directions, 14.4 G rays: 9.1e10 wave instructions in
+// The vector ALU bounds it (401,600 primitives x 225 rays x 64 directions, 5.8 G rays: 9.1e10 wave instructions in
 // 122 ms, one per SIMD every 3.3 cycles), so lanes must not idle and work that decides nothing must not run:
 // - rays are generated up to 64 at a time with every lane active, into the wave's LDS queue, together with the first
 //   two entries of their cell's list; a ray with nothing above it is counted lit there and never queued;
@@ -487,15 +487,63 @@ __device__ __forceinline__ bool source_occluded(const DevScene &sc, v3f o, v3f d
     return false;
 }
 
+// The same over the block tree.  Without periodic faces the question is only whether some accepted hit lies before
+// dist0: the trace starts with dist0 as its closest distance and ends at the first hit.
+template <int ROWS, int MK>
+__device__ __forceinline__ bool source_occluded_blk(const DevScene &sc, const char *blk, const float4 *recs, v3f o, v3f d,
+                                                    uint32_t skip, float dist0, lds_u32 *stk, uint32_t *ovf,
+                                                    uint32_t stride, uint32_t max_steps, int *err) {
+    if (!(dist0 > 0.f)) return false;
+    const bool any = sc.nbbox == 0;
+    BlkRay L;
+    L.o = o;
+    L.d = d;
+    blk_direction(L, blk_rcp(d.x), blk_rcp(d.y), blk_rcp(d.z));
+    for (int step = 0; step < 32; ++step) {
+        blk_start(L, stk);
+        if (any) L.best_t = fminf(L.best_t, dist0);
+        uint32_t left = max_steps;
+        while (L.ni != RT_BLK_DONE) {
+            while (!(L.ni & RT_BLK_REC) && left != 0u) {
+                blk_node_step<ROWS>(blk, L, stk, ovf, stride);
+                left--;
+            }
+            if (left == 0u) {
+                atomicOr(err, 2);
+                return false;
+            }
+            if (L.ni == RT_BLK_DONE) break;
+            uint32_t slot_unused;
+            blk_leaf<false, MK>(blk, recs, L.ni, L, 1e-4f, skip, slot_unused);
+            if (any && L.best != RT_MISS) return true;
+            L.ni = blk_pop<ROWS>(L, stk, ovf, stride);
+        }
+        if (any) return false;
+        const float bt = nearest_face(sc, L.o, d, L.best_t);
+        if (!(bt > 0.f)) return L.best != RT_MISS && L.best_t < dist0;
+        L.o = wrap_at(sc, L.o, d, bt);
+    }
+    return false;
+}
+
 // Direct rays towards sphere, sun-sphere, rectangle and disk sources (direct_raygen.comp:482-561): one
 // wave per (job, primitive), d*d stratified origins as k_direct, per-ray direction, strength and lit face,
 // per-lane closest-hit traversal.  Items [item_lo, item_lo + nitems) of jobs whose item_begin ascend.
-template <int STK, bool COUNT, int MK>
+// BLK: over the block tree (every launch that neither counts nor lacks one).  The binary tree's stacks take 32 or
+// 64 KB of LDS a workgroup, two waves a SIMD at 64, and its trace goes on to the closest hit; the block tree's take
+// RT_SRC_ROWS rows, 17 KB (24 rows: the same time), and four waves a SIMD fit.  Three lamps over 20,100 primitives x
+// 256 rays, the whole pass by pass solve: 9.29 to 8.57 ms.  The quadrature of a sphere's strength, 200 divisions a
+// ray, is the larger part of what is left.
+#ifndef RT_SRC_ROWS
+#define RT_SRC_ROWS 17
+#endif
+template <int STK, bool COUNT, int MK, bool BLK>
 __global__ __launch_bounds__(256) void k_direct_src(const DirectJob *__restrict__ jobs, uint32_t njobs, uint32_t item_lo,
                                                     uint32_t nitems, uint32_t *counter, int *err,
                                                     unsigned long long *stats) {
-    __shared__ uint32_t stk_all[STK * 256];
+    __shared__ uint32_t stk_all[(BLK ? RT_SRC_ROWS : STK) * 256];
     uint32_t *stk = stk_all + threadIdx.x;
+    uint32_t ovf[BLK ? RT_BLK_OVF(RT_SRC_ROWS) : 1];
     const uint32_t lane = threadIdx.x & 63;
     Cnt<COUNT, MK> cnt{};
     uint32_t nray = 0;
@@ -539,7 +587,12 @@ __global__ __launch_bounds__(256) void k_direct_src(const DirectJob *__restrict_
                 if (tw == 3 || (!top && tw == 0)) continue;
                 const v3f dv = sub3(sp3, o);
                 const float dist0 = rsqrt_cr(dot3(dv, dv));
-                if (source_occluded<STK>(sc, o, dir, i, dist0, stk, 256u, err, cnt)) continue;
+                if constexpr (BLK) {
+                    if (source_occluded_blk<RT_SRC_ROWS, MK>(sc, (const char *)sc.blk, sc.rec, o, dir, i, dist0,
+                                                             (lds_u32 *)stk_all + threadIdx.x, ovf, 256u,
+                                                             sc.nnode4 + 8u, err))
+                        continue;
+                } else if (source_occluded<STK>(sc, o, dir, i, dist0, stk, 256u, err, cnt)) continue;
                 if (top) top_acc.add(strength);
                 else bot_acc.add(strength);
             }
@@ -607,17 +660,19 @@ int launch_direct(const DirectJob *jobs, uint32_t njobs, uint32_t total, uint32_
 template <int MK>
 static int launch_direct_src_t(const DirectJob *jobs, uint32_t njobs, uint32_t item_lo, uint32_t nitems,
                                uint32_t depth, uint32_t *counter, int *err, unsigned long long *stats, int ncu,
-                               hipStream_t st) {
+                               hipStream_t st, bool blk) {
     if (nitems == 0) return 0;
     k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
-    uint64_t g64 = std::min<uint64_t>((uint64_t)4 * ncu, ((uint64_t)nitems + 3) / 4);
+    blk = blk && !stats;
+    uint64_t g64 = std::min<uint64_t>((uint64_t)(blk ? 8 : 4) * ncu, ((uint64_t)nitems + 3) / 4);
     uint32_t g = (uint32_t)std::max<uint64_t>(g64, 1);
-    if (stats)
-        PICK_STK(depth, (k_direct_src<32, true, MK><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats)),
-                 (k_direct_src<64, true, MK><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats)));
+    if (blk) k_direct_src<1, false, MK, true><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats);
+    else if (stats)
+        PICK_STK(depth, (k_direct_src<32, true, MK, false><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats)),
+                 (k_direct_src<64, true, MK, false><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats)));
     else
-        PICK_STK(depth, (k_direct_src<32, false, MK><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats)),
-                 (k_direct_src<64, false, MK><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats)));
+        PICK_STK(depth, (k_direct_src<32, false, MK, false><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats)),
+                 (k_direct_src<64, false, MK, false><<<g, 256, 0, st>>>(jobs, njobs, item_lo, nitems, counter, err, stats)));
     LCHECK();
     return 0;
 }
@@ -626,7 +681,8 @@ int launch_direct_src(const DirectJob *jobs, uint32_t njobs, uint32_t item_lo, u
                       uint32_t *counter, int *err, unsigned long long *stats, int ncu, hipStream_t st, int flags) {
     int rc = 0;
     with_flags(stats ? counting_flags(flags) : flags, [&](auto fl) {
-        rc = launch_direct_src_t<decltype(fl)::value>(jobs, njobs, item_lo, nitems, depth, counter, err, stats, ncu, st);
+        rc = launch_direct_src_t<decltype(fl)::value>(jobs, njobs, item_lo, nitems, depth, counter, err, stats, ncu, st,
+                                                      (flags & RT_FL_BLK) != 0);
     });
     return rc;
 }
