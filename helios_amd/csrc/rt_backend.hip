@@ -556,7 +556,7 @@ int rt_launch_direct_rays(rt_ctx *ctx, const rt_launch_params *p) {
     hipStream_t st = ctx->sx.stream;
     const uint32_t P = be.P, Bl = be.Bl, S = be.S;
     const uint32_t d = (uint32_t)std::ceil(std::sqrt((double)p->rays_per_primitive));
-    size_t bytes = (size_t)S * P * 2 * 4 + 2 * (size_t)P * Bl * 4 + Bl * 8 + S * sizeof(DirectJob) + 16 * 256;
+    size_t bytes = (size_t)S * P * 2 * 4 + 2 * (size_t)P * Bl * 4 + Bl * 8 + S * sizeof(DirectJob) + RT_QUEUE_WORDS * 4 + 16 * 256;
     if (glass) bytes += glass_bytes(P, Bl) + (size_t)S * P * Bl * 2 * 4 + S * sizeof(GlassDirectJob) + 2 * 256;
     if (be.ws.reserve(bytes)) return -1;
     Carve cv{(char *)be.ws.base};
@@ -745,7 +745,7 @@ int rt_launch_diffuse_rays(rt_ctx *ctx, const rt_launch_params *p) {
     }
     // a launch with covers traces and gathers in one kernel and keeps no hit table
     size_t bytes = (glass ? 0 : (size_t)P * 2 * nn * 4) + 2 * PB * 4 + Bl * 9 + sizeof(DiffuseJob) +
-                   sizeof(GatherJob) + hsky.size() * 4 + 17 * 256 + (glass ? glass_bytes(P, Bl) : 0);
+                   sizeof(GatherJob) + hsky.size() * 4 + RT_QUEUE_WORDS * 4 + 17 * 256 + (glass ? glass_bytes(P, Bl) : 0);
     if (be.ws.reserve(bytes)) return -1;
     Carve cv{(char *)be.ws.base};
     uint32_t *hits = glass ? nullptr : cv.take<uint32_t>((size_t)P * 2 * nn);

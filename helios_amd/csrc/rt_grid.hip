@@ -280,7 +280,7 @@ __global__ __launch_bounds__(256) void k_grid_rank(const SunGrid *__restrict__ g
 // the rectangles' areas: with one lane a rectangle, a ground patch under the whole scene was 4,000 cells filled
 // one after the other by a single lane, latency after latency (1,601 primitives, one direction: the whole solve
 // 1.71 ms, 1.18 ms so).  Neighbouring lanes also take neighbouring cells of a row, whose counts and starts share
-// lines (1 M primitives, 64 directions: that batch 555 to 549 ms).
+// lines (401,600 primitives, 64 directions: that batch 555 to 549 ms).
 __global__ __launch_bounds__(256) void k_grid_fill(uint32_t nleaf, const float4 *__restrict__ rec, float smax,
                                                    const SunGrid *__restrict__ grids,
                                                    const uint32_t *__restrict__ cell_base,

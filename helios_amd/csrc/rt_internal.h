@@ -29,8 +29,9 @@ constexpr uint64_t RT_MAX_PRIMS = (uint64_t)RT_ID_BITS + 1u;
 #define RT_QUEUE_STRIDE 32u
 #define RT_QUEUE_WORDS (RT_QUEUES * RT_QUEUE_STRIDE)
 // Chunks a wave from which a launch splits its queue: every wave ends with RT_QUEUES empty fetches instead of one.
-// Gather of 1 M primitives (122 chunks a wave): 24.1 ms split, 58.4 not; of 200,000 (24 chunks): 1.38 and 2.50; their
-// diffuse passes 417 and 431, 30.2 and 31.1.  2, 4 and 8 measured the same but for the 200,000 (8: not split).
+// Five gathers of 1 M primitives (122 chunks a wave): 24.1 ms split, 58.4 not; three of 60,400 (7 chunks): 1.38 and
+// 2.50; their diffuse passes 417 and 431, 30.2 and 31.1.  From 2, 4 and 8 chunks measured the same but for the 60,400
+// (8: not split).
 #ifndef RT_QUEUE_SPLIT
 #define RT_QUEUE_SPLIT 4u
 #endif

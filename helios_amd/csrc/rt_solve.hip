@@ -410,7 +410,7 @@ size_t solve_workspace_bytes(uint32_t P, const rt_band_request &q, uint32_t K, b
     if (acct)
         bytes += PC * 8 + (size_t)P * 8 + (size_t)ENERGY_BLOCKS * 4 * C * 8 + (size_t)(1 + maxdepth) * 4 * C * 8 +
                  (size_t)C * RT_ENERGY_ROWS * 8;
-    return bytes + 40 * 256;  // carve alignment
+    return bytes + RT_QUEUE_WORDS * 4 + 40 * 256;  // work counters, carve alignment
 }
 
 size_t Workspace::capacity_for(size_t bytes) { return bytes + bytes / 8 + (1u << 20); }

@@ -464,7 +464,7 @@ constexpr int pow2_up(int n) { int p = 1; while (p < n) p *= 2; return p; }
 // record the pass's incident and sky flux densities and the sky-bound ray counts (GatherJob.acct, .miss) for the
 // energy bookkeeping.  Both are separate instances, so the plain gather carries no extra registers.
 // The channel count is exact up to 16: a kernel for the next power of two loaded and added channels that are not
-// there.  Five passes of 1 M primitives x 1,024 rays, 3 channels: 24.1 to 11.9 ms; three passes of 200,000 x 100 rays:
+// there.  Five passes of 1 M primitives x 450 rays, 3 channels: 24.1 to 11.9 ms; three passes of 200,000 x 100 rays:
 // 4 channels 2.04 to 1.43 ms, 8 channels 3.75 to 1.44.  k_gather_chan (lanes over the channels) takes 5.2 ms for these
 // passes at 9 to 17 channels and this kernel 1.60, 1.62 and 1.81 at 9, 12 and 16; more channels than 16 would not fit
 // the registers.

@@ -633,14 +633,14 @@ __device__ __forceinline__ bool packet_occluded(const DevScene &sc, v3f o, v3f d
 }
 
 // A wave's view of the work queue of a persistent launch: items [0, total) in chunks of `chunk`.  What bounds a
-// queue is its atomics on one address, 5 to 12 ns each and one after the other: as much as a whole item of the
-// direct kernel (225 rays of a primitive over an occlusion grid: 4.6 ns an item, now 1.9) or of a gather.  So
+// queue is its atomics on one address, 11.6 ns each and one after the other: more than a whole item of the direct
+// kernel takes the chip (225 rays of a primitive over an occlusion grid, 5 ns) or one of a gather.  So
 // - a launch with at most one chunk a wave uses none: wave w takes chunk w (1,601 primitives: four gathers 0.202
 //   to 0.057 ms, direct 0.060 to 0.027);
 // - a launch of RT_QUEUE_SPLIT chunks a wave or more splits the items into RT_QUEUES segments, each with its own
 //   counter in its own line.  A workgroup starts on the segment of its XCD (workgroups go to the XCDs in turn), so
 //   an XCD's L2 holds one range of the leaf order instead of an eighth of every range, and goes on to the other
-//   segments in turn once its own is empty (1 M primitives x 64 directions: direct 297 to 136 ms; five gathers of
+//   segments in turn once its own is empty (401,600 primitives x 64 directions: direct 297 to 136 ms; five gathers of
 //   1 M primitives 58 to 24).  Larger chunks on one counter did the same for these but cost the diffuse kernel
 //   and small scenes up to half their time.
 // Looking at a counter before adding to it, past the first segment, made the direct kernel 4 % slower.
@@ -662,7 +662,7 @@ struct WaveQueue {
         }
     }
     // Adds the chunk to counter word w from lane 0 alone and returns its old value: 64 lanes adding to one word are
-    // 64 atomics (114 ns a fetch, one lane's 5 to 12).
+    // 64 atomics (114 ns a fetch, one lane's 11.6).
     __device__ __forceinline__ uint32_t fetch(uint32_t *w) const {
         uint32_t x = 0;
         if ((threadIdx.x & 63) == 0) x = __hip_atomic_fetch_add(w, chunk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
