@@ -60,16 +60,19 @@ def pct(a, q):
     return float(np.percentile(np.asarray(a, np.float64), q)) if len(a) else None
 
 
-# position of the COUNT template argument: k_cast<STK, COUNT, FLAGS>, k_camera / k_direct_src<STK, COUNT, FLAGS>,
-# k_direct / k_diffuse<WAVES, STK, COUNT, FLAGS>
-COUNT_ARG = {"k_cast": 1, "k_camera": 1, "k_direct_src": 1, "k_direct": 2, "k_diffuse": 2}
+# position of the COUNT template argument of the kernels that have one: k_cast_bin / k_camera / k_direct_src<STK,
+# COUNT, FLAGS, ...>, k_direct / k_diffuse_bin<WAVES, STK, COUNT, FLAGS>, and in profiles of earlier kernels k_cast<STK,
+# COUNT, FLAGS> and k_diffuse<WAVES, STK, COUNT, FLAGS> (now <WAVES, FLAGS>)
+COUNT_ARG = {"k_cast_bin": 1, "k_camera": 1, "k_direct_src": 1, "k_direct": 2, "k_diffuse_bin": 2, "k_cast": 1,
+             "k_diffuse": 2}
 
 
 def counting_variant(name):
     m = re.search(r"(k_\w+)<([^>]*)>", name)
     if not m or m.group(1) not in COUNT_ARG:
         return False
-    return [a.strip() for a in m.group(2).split(",")][COUNT_ARG[m.group(1)]] == "true"
+    args = [a.strip() for a in m.group(2).split(",")]
+    return len(args) > COUNT_ARG[m.group(1)] and args[COUNT_ARG[m.group(1)]] == "true"
 
 
 def kernel_flags(name):
