@@ -132,10 +132,14 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
                 const unsigned long long r = q_next + rank;
                 L.o = mk3(O[r * 3], O[r * 3 + 1], O[r * 3 + 2]);
                 L.d = mk3(D[r * 3], D[r * 3 + 1], D[r * 3 + 2]);
-                // a cast ray may start far outside the scene, where an ulp of the reciprocal counts: divide
-                blk_direction(L, fabsf(L.d.x) > 1e-18f ? 1.0f / L.d.x : copysignf(1e18f, L.d.x),
-                              fabsf(L.d.y) > 1e-18f ? 1.0f / L.d.y : copysignf(1e18f, L.d.y),
-                              fabsf(L.d.z) > 1e-18f ? 1.0f / L.d.z : copysignf(1e18f, L.d.z));
+                // A cast ray may start far outside the scene, where an ulp of the reciprocal counts: divide.  Its
+                // direction may have any length (distances count in lengths of it), so what makes a component
+                // near 0 is its size against the largest one: its slab then reaches 1e18 times as far as the
+                // ray's own distances (1e30 at most, as ray_pre()).
+                const float lim = fminf(1e18f * __builtin_amdgcn_rcpf(max3f(fabsf(L.d.x), fabsf(L.d.y), fabsf(L.d.z))), 1e30f);
+                blk_direction(L, copysignf(fminf(1.0f / fabsf(L.d.x), lim), L.d.x),
+                              copysignf(fminf(1.0f / fabsf(L.d.y), lim), L.d.y),
+                              copysignf(fminf(1.0f / fabsf(L.d.z), lim), L.d.z));
                 blk_start(L, stk);
                 L.best_t = tstart;
                 my_r = r;
