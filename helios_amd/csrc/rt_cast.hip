@@ -160,7 +160,7 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
                     L.ni = RT_BLK_DONE;
                     break;
                 }
-                if (inner) blk_node_step<ROWS>(blk, L, stk, ovf, stride);
+                if (inner) blk_node_step<ROWS, true>(blk, L, stk, ovf, stride);
             }
             while (true) {
                 const bool leaf = (L.ni & RT_BLK_REC) && L.ni != RT_BLK_DONE;

@@ -929,7 +929,9 @@ __device__ __forceinline__ float fma_hi(uint32_t w, float m, float a) {
 // Keeps the loads of a node together: the offset they share stays in its register until v has been computed from
 // what the last of them returns.  A load into its own address register ends the clause (the compiler puts an s_nop
 // before it); other waves' loads then run between this one and the first two and have often evicted the block from the
-// vL1D: 20 M rays over 5 M primitives take 7.6 ms that way and 6.7 ms with the three loads in one clause.
+// vL1D: 20 M rays over 5 M primitives take 7.6 ms that way and 6.7 ms with the three loads in one clause.  Only k_cast
+// needs it: the other kernels' registers fall so that the loads stay together, and their order of instructions without
+// the hold measured 0.2 % better (k_diffuse).
 __device__ __forceinline__ void keep_until(uint32_t offset, float &v) {
 #if defined(__HIP_DEVICE_COMPILE__)
     asm("" : "+v"(v) : "v"(offset));
@@ -952,7 +954,7 @@ __device__ __forceinline__ void keep_until(uint32_t offset, float &v) {
 // - pushes need no branches: the three farthest keys are stored above the stack's top whether they are hits or
 //   not (a key that is not lies above the new top).  Keys of missed children are 0x80000000: the smallest as int,
 //   so last in the descending order, and above every hit as unsigned, so never the nearest.
-template <int ROWS>
+template <int ROWS, bool HOLD = false>
 __device__ __forceinline__ void blk_node_step(const char *blk, BlkRay &L, lds_u32 *stk, uint32_t *ovf, uint32_t stride) {
     const uint4 *nd = (const uint4 *)(blk + L.ni);
     const uint4 a = nd[0], b = nd[1], c = nd[2];
@@ -964,7 +966,7 @@ __device__ __forceinline__ void blk_node_step(const char *blk, BlkRay &L, lds_u3
                 Az = __uint_as_float(a.w << 15) * L.iz;
     float Bx = fmaf(__uint_as_float(a.x), L.ix, -L.ox);
     const float By = fmaf(__uint_as_float(a.y), L.iy, -L.oy), Bz = fmaf(__uint_as_float(a.z), L.iz, -L.oz);
-    keep_until(L.ni, Bx);
+    if constexpr (HOLD) keep_until(L.ni, Bx);
     float tn[4], tf[4];
 #pragma unroll
     for (int k = 0; k < 2; k++) {
