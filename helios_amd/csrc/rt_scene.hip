@@ -481,7 +481,9 @@ __device__ __forceinline__ void blk_node(uint32_t t, const float4 *__restrict__ 
                 qh = ceil(dh / s);
                 if (ql * s > dl) ql -= 1.0;  // (rounded quotients)
                 if (qh * s < dh) qh += 1.0;
-                if (!(ql >= 0.0 && qh <= 255.0 && ql <= qh)) atomicOr(bad, 1);
+                // 1: a box that is not finite; 2: an extent beyond 255 of the largest step
+                if (!isfinite(lo[k]) || !isfinite(hi[k])) atomicOr(bad, 1);
+                else if (!(ql >= 0.0 && qh <= 255.0 && ql <= qh)) atomicOr(bad, 2);
             }
             wl[a] |= (uint32_t)fmin(fmax(ql, 0.0), 255.0) << (8 * k);
             wh[a] |= (uint32_t)fmin(fmax(qh, 0.0), 255.0) << (8 * k);
@@ -686,6 +688,8 @@ static int build_bvh4(uint32_t n, const uint32_t *child, const float *lbox, cons
 // bytes of the block tree of nn4 nodes over nleaf records and of the build's check word
 static size_t blk_bytes(uint32_t nn4, uint32_t nleaf) { return 64 * ((size_t)nn4 + nleaf) + 64; }
 
+// Returns 0, 1 when the scene is too large for the nodes' steps (extents above 255 x 2^103: the traversals then walk the
+// binary tree), or -1.
 static int write_blocks(uint32_t nn4, uint32_t nleaf, const float4 *node4, const float4 *rec, uint4 *blk, hipStream_t st) {
     int *bad = (int *)(blk + 4 * ((size_t)nn4 + nleaf));
     uint32_t *cnt;
@@ -705,11 +709,11 @@ static int write_blocks(uint32_t nn4, uint32_t nleaf, const float4 *node4, const
     CK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, st));
     CK(hipStreamSynchronize(st));
     CK(hipFree(cnt)); CK(hipFree(tmp));
-    if (hbad) {
-        set_error("block tree: a child box lies outside its node's 8-bit grid");
+    if (hbad & 1) {
+        set_error("block tree: a primitive's box is not finite");
         return -1;
     }
-    return 0;
+    return hbad ? 1 : 0;
 }
 
 int validate_geometry(uint64_t P, const uint32_t *types, const char *who) {
@@ -851,7 +855,13 @@ int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, cons
             if ((uint64_t)nnode4 + nleaf <= RT_BLK_MAX) {
                 CK(hipMalloc(&blk, blk_bytes(nnode4, nleaf)));
                 S.own.push_back(blk);
-                if (write_blocks(nnode4, nleaf, node4, rec, blk, st)) return -1;
+                const int wrote = write_blocks(nnode4, nleaf, node4, rec, blk, st);
+                if (wrote < 0) return -1;
+                if (wrote > 0) {
+                    S.own.pop_back();
+                    CK(hipFree(blk));
+                    blk = nullptr;
+                }
             }
             CK(hipFree(child)); CK(hipFree(ibox));
         } else {

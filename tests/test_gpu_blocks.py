@@ -8,7 +8,7 @@ kilometres away loses the box tests' padding to FP32 rounding in any of the tree
 import numpy as np
 import pytest
 
-from helios_amd import scenes
+from helios_amd import native, scenes
 from oracle.oracle import OracleScene
 
 pytestmark = pytest.mark.gpu
@@ -94,3 +94,27 @@ def test_cast_axis_parallel_and_far_rays(ctx, distance):
     hit = u != 0xFFFFFFFF
     assert hit.any()
     assert np.array_equal(t[hit], to[hit]) and np.array_equal(nrm[hit], no[hit])
+
+
+@pytest.mark.parametrize("far", [1e30, 1e34, 1e37])
+def test_one_primitive_far_away(ctx, far):
+    """Extents beyond the nodes' largest steps: such a scene is traced without a block tree."""
+    s = _cloud(60)
+    s.transforms[7, 3] = far
+    g, o = ctx.scene(s.transforms, s.types, s.twosided), OracleScene.from_arrays(s)
+    rng = np.random.default_rng(4)
+    O, D = rng.uniform(-0.5, 0.5, (500, 3)).astype(np.float32), rng.normal(size=(500, 3))
+    D = (D / np.linalg.norm(D, axis=1, keepdims=True)).astype(np.float32)
+    t, nrm, u = g.cast_rays(O, D)
+    to, no, uo = o.cast_rays(O, D)
+    hit = u != 0xFFFFFFFF
+    assert np.array_equal(u, uo) and hit.sum() > 100
+    assert np.array_equal(t[hit], to[hit]) and np.array_equal(nrm[hit], no[hit])
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf])
+def test_infinite_coordinates_are_refused(ctx, bad):
+    s = _cloud(60)
+    s.transforms[7, 3] = bad
+    with pytest.raises(native.RTError, match="not finite"):
+        ctx.scene(s.transforms, s.types, s.twosided)
