@@ -685,30 +685,33 @@ static int build_bvh4(uint32_t n, const uint32_t *child, const float *lbox, cons
     return 0;
 }
 
+// Device scratch of one call, freed on every way out of it
+struct Scratch {
+    void *p = nullptr;
+    ~Scratch() { if (p) (void)hipFree(p); }
+};
+
 // bytes of the block tree of nn4 nodes over nleaf records and of the build's check word
 static size_t blk_bytes(uint32_t nn4, uint32_t nleaf) { return 64 * ((size_t)nn4 + nleaf) + 64; }
 
-// Returns 0, 1 when the scene is too large for the nodes' steps (extents above 255 x 2^103: the traversals then walk the
-// binary tree), or -1.
-static int write_blocks(uint32_t nn4, uint32_t nleaf, const float4 *node4, const float4 *rec, uint4 *blk, hipStream_t st) {
+int write_blocks(uint32_t nn4, uint32_t nleaf, const float4 *node4, const float4 *rec, uint4 *blk, hipStream_t st) {
     int *bad = (int *)(blk + 4 * ((size_t)nn4 + nleaf));
-    uint32_t *cnt;
-    CK(hipMalloc(&cnt, sizeof(uint32_t) * 2 * (size_t)nn4));
-    uint32_t *base = cnt + nn4;
+    Scratch counts, scan;
+    CK(hipMalloc(&counts.p, sizeof(uint32_t) * 2 * (size_t)nn4));
+    uint32_t *cnt = (uint32_t *)counts.p, *base = cnt + nn4;
     size_t tmp_bytes = 0;
     // child blocks follow the root's
     CK(hipcub::DeviceScan::ExclusiveScan(nullptr, tmp_bytes, cnt, base, hipcub::Sum(), 1u, (int)nn4, st));
-    void *tmp;
-    CK(hipMalloc(&tmp, tmp_bytes + 16));
+    CK(hipMalloc(&scan.p, tmp_bytes + 16));
     CK(hipMemsetAsync(bad, 0, sizeof(int), st));
     k_blk_count<<<blocks(nn4, 256), 256, 0, st>>>(nn4, node4, cnt);
-    CK(hipcub::DeviceScan::ExclusiveScan(tmp, tmp_bytes, cnt, base, hipcub::Sum(), 1u, (int)nn4, st));
+    CK(hipGetLastError());
+    CK(hipcub::DeviceScan::ExclusiveScan(scan.p, tmp_bytes, cnt, base, hipcub::Sum(), 1u, (int)nn4, st));
     k_blocks<<<blocks((size_t)nn4 * 4, 256), 256, 0, st>>>(nn4, node4, rec, base, blk, bad);
     CK(hipGetLastError());
     int hbad = 0;
     CK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, st));
     CK(hipStreamSynchronize(st));
-    CK(hipFree(cnt)); CK(hipFree(tmp));
     if (hbad & 1) {
         set_error("block tree: a primitive's box is not finite");
         return -1;
@@ -974,34 +977,40 @@ int scene_set_masks(Scene &S, uint32_t nmasks, const uint8_t *texels, const uint
     }
     for (size_t j = 0; j < dmask.size(); j++) desc[3 * j].x = bits_f((uint32_t)(tex_base + toff[dmask[j]]));
     if (nleaf == 0) return 0;
-    float4 *R = nullptr;
-    uint32_t *dm = nullptr;
-    CK(hipMalloc(&R, (total + 15) & ~(uint64_t)15));
+    // Until the new records, descriptors and texels are complete the scene is untouched
+    Scratch recs, map;
+    CK(hipMalloc(&recs.p, (total + 15) & ~(uint64_t)15));
+    float4 *R = (float4 *)recs.p;
     CK(hipMemcpyAsync(R, S.h.rec, rec_f4 * sizeof(float4), hipMemcpyDeviceToDevice, st));
     if (!desc.empty()) {
         CK(hipMemcpyAsync(R + rec_f4, desc.data(), desc.size() * sizeof(float4), hipMemcpyHostToDevice, st));
         CK(hipMemcpyAsync((char *)R + tex_base, texels, toff[nmasks], hipMemcpyHostToDevice, st));
-        CK(hipMalloc(&dm, sizeof(uint32_t) * P));
-        CK(hipMemcpyAsync(dm, mdesc.data(), sizeof(uint32_t) * P, hipMemcpyHostToDevice, st));
+        CK(hipMalloc(&map.p, sizeof(uint32_t) * P));
+        CK(hipMemcpyAsync(map.p, mdesc.data(), sizeof(uint32_t) * P, hipMemcpyHostToDevice, st));
     }
+    uint32_t *dm = (uint32_t *)map.p;
     k_mask_tags<<<blocks(nleaf, 256), 256, 0, st>>>(nleaf, R, dm);
     CK(hipGetLastError());
     CK(hipStreamSynchronize(st));
-    // replace the record buffer and the descriptor map
-    auto drop = [&S](const void *p) {
-        for (size_t k = 0; k < S.own.size(); k++)
-            if (S.own[k] == p) { (void)hipFree(S.own[k]); S.own.erase(S.own.begin() + k); return; }
-    };
-    drop(S.h.rec);
-    if (S.h.mdesc) drop(S.h.mdesc);
+    // From here on the scene owns the new buffers, and it keeps the old ones until the device descriptor names the new.
+    // The block tree holds copies of the records; a call that fails before they fit the descriptor leaves the scene
+    // without it (the launches look at the host's copy), traced over the binary tree.
+    DevScene next = S.h;
+    const void *old_rec = S.h.rec, *old_mdesc = S.h.mdesc;
+    next.rec = R;
+    next.mdesc = dm;
     S.own.push_back(R);
+    recs.p = nullptr;
     if (dm) S.own.push_back(dm);
-    S.h.rec = R;
-    S.h.mdesc = dm;
-    // the block tree holds copies of the records
-    if (S.h.blk && write_blocks(S.h.nnode4, nleaf, S.h.node4, R, const_cast<uint4 *>(S.h.blk), st)) return -1;
-    CK(hipMemcpyAsync(S.d, &S.h, sizeof(DevScene), hipMemcpyHostToDevice, st));
+    map.p = nullptr;
+    S.h.blk = nullptr;
+    if (next.blk && write_blocks(next.nnode4, nleaf, next.node4, R, const_cast<uint4 *>(next.blk), st)) return -1;
+    CK(hipMemcpyAsync(S.d, &next, sizeof(DevScene), hipMemcpyHostToDevice, st));
     CK(hipStreamSynchronize(st));
+    S.h = next;
+    for (const void *p : {old_rec, old_mdesc})
+        for (size_t k = 0; p && k < S.own.size(); k++)
+            if (S.own[k] == p) { (void)hipFree(S.own[k]); S.own.erase(S.own.begin() + k); break; }
     return 0;
 }
 

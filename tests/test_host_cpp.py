@@ -10,14 +10,23 @@ BIN = os.path.join(ROOT, "tests", "cpp", "test_radiation_model")
 REF = "/root/reference"
 
 
-def _binary():
-    if not os.path.exists(BIN):
+def _binary(path=BIN):
+    if not os.path.exists(path):
         subprocess.run(["make", "-s", "-C", os.path.join(ROOT, "tests", "cpp")], check=True)
-    return BIN
+    return path
 
 
 def test_cpp_host_cases_cpu():
     r = subprocess.run([_binary(), "--cpu"], capture_output=True, text=True, timeout=120)
+    print(r.stdout)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_scene_update_failures_cpu():
+    """Scene updates whose n-th runtime call fails, for every n, over a test double of the HIP runtime
+    (tests/cpp/test_scene_failures.cpp): no descriptor names a freed buffer and no buffer is lost."""
+    r = subprocess.run([_binary(os.path.join(ROOT, "tests", "cpp", "test_scene_failures"))], capture_output=True,
+                       text=True, timeout=120)
     print(r.stdout)
     assert r.returncode == 0, r.stdout + r.stderr
 
