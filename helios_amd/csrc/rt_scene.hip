@@ -365,7 +365,8 @@ __global__ void k_ploc_emit(uint32_t n, uint32_t node_base, const uint32_t *__re
 // node's two children and repeatedly opens the internal child with the largest surface area until it
 // has four children or only leaves.  Nodes are numbered breadth-first (the root is 0).
 // Node layout (8 float4, 128 B): lo.x[4], hi.x[4], lo.y[4], hi.y[4], lo.z[4], hi.z[4], links[4]
-// (leaf bit 31 | leaf slot, else node index; unused slots 0x7FFFFFFF with a box at +inf), (child count, 0, 0, 0).
+// (leaf bit 31 | leaf slot, else node index; unused slots 0x7FFFFFFF with a box at +inf), (child count, block of the
+// first child in the block tree, 0, 0).
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ const float *box_of(uint32_t c, const float *lbox, const float *ibox) {
     return (c & RT_LEAF_BIT) ? lbox + (size_t)(c & ~RT_LEAF_BIT) * 6 : ibox + (size_t)c * 6;
@@ -510,12 +511,13 @@ __global__ void k_blk_count(uint32_t nn4, const float4 *__restrict__ node4, uint
 }
 
 // one thread per (node, child slot); thread 0 also writes the root
-__global__ void k_blocks(uint32_t nn4, const float4 *__restrict__ node4, const float4 *__restrict__ rec,
+__global__ void k_blocks(uint32_t nn4, float4 *node4, const float4 *__restrict__ rec,
                          const uint32_t *__restrict__ base, uint4 *__restrict__ blk, int *__restrict__ bad) {
     const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t t = g >> 2, k = g & 3u;
     if (t >= nn4) return;
     if (g == 0) blk_node(0u, node4, base, blk, bad);
+    if (k == 0) node4[(size_t)t * 8 + 7].y = __uint_as_float(base[t]);
     if (k >= __float_as_uint(node4[(size_t)t * 8 + 7].x)) return;
     const uint32_t lk = __float_as_uint(((const float *)(node4 + (size_t)t * 8 + 6))[k]);
     uint4 *dst = blk + ((size_t)base[t] + k) * 4;
@@ -525,6 +527,21 @@ __global__ void k_blocks(uint32_t nn4, const float4 *__restrict__ node4, const f
     } else {
         blk_node(lk, node4, base, dst, bad);
     }
+}
+
+// Copies the records into their blocks again, one thread per (node, child slot)
+__global__ void k_blk_records(uint32_t nn4, const float4 *__restrict__ node4, const float4 *__restrict__ rec,
+                              uint4 *__restrict__ blk) {
+    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = g >> 2, k = g & 3u;
+    if (t >= nn4) return;
+    const float4 c = node4[(size_t)t * 8 + 7];
+    if (k >= __float_as_uint(c.x)) return;
+    const uint32_t lk = __float_as_uint(((const float *)(node4 + (size_t)t * 8 + 6))[k]);
+    if (!(lk & RT_LEAF_BIT)) return;
+    const uint4 *r = (const uint4 *)rec + (size_t)(lk & ~RT_LEAF_BIT) * 4;
+    uint4 *dst = blk + ((size_t)__float_as_uint(c.y) + k) * 4;
+    for (int q = 0; q < 4; q++) dst[q] = r[q];
 }
 
 // node layout: (c0.lo.x, c0.hi.x, c0.lo.y, c0.hi.y), (c0.lo.z, c0.hi.z, c1.lo.x, c1.hi.x),
@@ -694,7 +711,7 @@ struct Scratch {
 // bytes of the block tree of nn4 nodes over nleaf records and of the build's check word
 static size_t blk_bytes(uint32_t nn4, uint32_t nleaf) { return 64 * ((size_t)nn4 + nleaf) + 64; }
 
-int write_blocks(uint32_t nn4, uint32_t nleaf, const float4 *node4, const float4 *rec, uint4 *blk, hipStream_t st) {
+int write_blocks(uint32_t nn4, uint32_t nleaf, float4 *node4, const float4 *rec, uint4 *blk, hipStream_t st) {
     int *bad = (int *)(blk + 4 * ((size_t)nn4 + nleaf));
     Scratch counts, scan;
     CK(hipMalloc(&counts.p, sizeof(uint32_t) * 2 * (size_t)nn4));
@@ -1004,7 +1021,11 @@ int scene_set_masks(Scene &S, uint32_t nmasks, const uint8_t *texels, const uint
     if (dm) S.own.push_back(dm);
     map.p = nullptr;
     S.h.blk = nullptr;
-    if (next.blk && write_blocks(next.nnode4, nleaf, next.node4, R, const_cast<uint4 *>(next.blk), st)) return -1;
+    if (next.blk) {
+        k_blk_records<<<blocks((size_t)next.nnode4 * 4, 256), 256, 0, st>>>(next.nnode4, next.node4, R,
+                                                                            const_cast<uint4 *>(next.blk));
+        CK(hipGetLastError());
+    }
     CK(hipMemcpyAsync(S.d, &next, sizeof(DevScene), hipMemcpyHostToDevice, st));
     CK(hipStreamSynchronize(st));
     S.h = next;

@@ -12,7 +12,7 @@
 
 namespace {
 std::map<void *, size_t> live;
-int calls = 0, fail_at = 0, mallocs = 0, launches = 0;  // fail_at 0: none
+int calls = 0, fail_at = 0, mallocs = 0;  // fail_at 0: none
 bool step() { return ++calls == fail_at; }
 bool is_live(const void *p) { return live.count(const_cast<void *>(p)) != 0; }
 void *take(size_t n) {
@@ -45,7 +45,6 @@ hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) {
 hipError_t hipStreamSynchronize(hipStream_t) { return step() ? hipErrorUnknown : hipSuccess; }
 static hipError_t last = hipSuccess;
 hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) {
-    launches++;
     return last = step() ? hipErrorLaunchFailure : hipSuccess;
 }
 hipError_t hipGetLastError() {
@@ -137,12 +136,19 @@ bool run(const char *what, int (*call)(rt::Scene &), bool earlier) {
 
 int main() {
     const auto blocks = [](rt::Scene &S) {
-        return rt::write_blocks(NN4, P, S.h.node4, S.h.rec, const_cast<uint4 *>(S.h.blk), nullptr);
+        return rt::write_blocks(NN4, P, const_cast<float4 *>(S.h.node4), S.h.rec, const_cast<uint4 *>(S.h.blk), nullptr);
     };
     bool ok = true;
     for (bool earlier : {false, true}) {
         ok = run("scene_set_masks", set_masks, earlier) && ok;
         ok = run("write_blocks", blocks, earlier) && ok;
+    }
+    {
+        // records, descriptors and texels are new buffers; the block tree is refreshed in place
+        Fixture f;
+        fail_at = mallocs = 0;
+        ok = set_masks(f.S) == 0 && ok;
+        if (mallocs != 2) { std::printf("scene_set_masks: %d allocations\n", mallocs); ok = false; }
     }
     std::printf(ok ? "all checks passed\n" : "FAILED\n");
     return ok ? 0 : 1;
