@@ -85,7 +85,7 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
                                               unsigned long long *counter, uint32_t chunk, int *err) {
     constexpr int ROWS = RT_CAST_ROWS;
     __shared__ uint32_t stk_all[ROWS * WPB * 64];
-    uint32_t ovf[RT_BLK_OVF(ROWS)];
+    uint32_t ovf[blk_ovf(ROWS, MK)];
     lds_u32 *stk = (lds_u32 *)stk_all + threadIdx.x;
     const uint32_t stride = WPB * 64;
     const DevScene &sc = *scp;
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
     while (true) {
         // finished lanes write their result
         if (busy && L.ni == RT_BLK_DONE) {
-            cast_result(my_r, L.best, L.best_t, (const float4 *)(blk + (slot & ~63u)), L.o, L.d, uuid, T, N, U);
+            cast_result(my_r, L.best, L.best_t, (const float4 *)blk_at<MK>(blk, slot), L.o, L.d, uuid, T, N, U);
             busy = false;
         }
         // idle lanes take the next rays of the wave's chunk
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(WPB * 64, RT_CAST_WAVES_PER_EU) void k_cast(const D
                     L.ni = RT_BLK_DONE;
                     break;
                 }
-                if (inner) blk_node_step<ROWS, true>(blk, L, stk, ovf, stride);
+                if (inner) blk_node_step<ROWS, MK, true>(blk, L, stk, ovf, stride);
             }
             while (true) {
                 const bool leaf = (L.ni & RT_BLK_REC) && L.ni != RT_BLK_DONE;
@@ -729,6 +729,8 @@ int launch_cast(const DevScene *sc, uint32_t depth, uint64_t n, const float *o, 
     with_flags(flags & RT_FL_WT, [&](auto fl) {
         constexpr int FL = decltype(fl)::value & RT_FL_WT;
         if (stats) k_cast_bin<RT_STACK, true, FL><<<g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, err, stats);
+        else if ((flags & RT_FL_BLK) && (flags & RT_FL_WIDE))
+            k_cast<4, FL | RT_FL_WIDE><<<g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, 64u, err);
         else if (flags & RT_FL_BLK) k_cast<4, FL><<<g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, 64u, err);
         else k_cast_bin<RT_STACK, false, FL><<<g, 256, 0, st>>>(sc, n, o, d, maxd, t, nrm, uuid, counter, err, nullptr);
     });

@@ -505,7 +505,7 @@ __device__ __forceinline__ bool source_occluded_blk(const DevScene &sc, const ch
         uint32_t left = max_steps;
         while (L.ni != RT_BLK_DONE) {
             while (!(L.ni & RT_BLK_REC) && left != 0u) {
-                blk_node_step<ROWS>(blk, L, stk, ovf, stride);
+                blk_node_step<ROWS, MK>(blk, L, stk, ovf, stride);
                 left--;
             }
             if (left == 0u) {
@@ -529,7 +529,7 @@ __device__ __forceinline__ bool source_occluded_blk(const DevScene &sc, const ch
 // Direct rays towards sphere, sun-sphere, rectangle and disk sources (direct_raygen.comp:482-561): one
 // wave per (job, primitive), d*d stratified origins as k_direct, per-ray direction, strength and lit face,
 // per-lane closest-hit traversal.  Items [item_lo, item_lo + nitems) of jobs whose item_begin ascend.
-// BLK: over the block tree (every launch that neither counts nor lacks one).  The binary tree's stacks take 32 or
+// BLK: over the block tree (every launch that does not count, unless the scene lacks one or its links are wide).  The binary tree's stacks take 32 or
 // 64 KB of LDS a workgroup, two waves a SIMD at 64, and its trace goes on to the closest hit; the block tree's take
 // RT_SRC_ROWS rows, 17 KB (24 rows: the same time), and four waves a SIMD fit.  Three lamps over 20,100 primitives x
 // 256 rays, the whole pass by pass solve: 9.29 to 8.57 ms.  The quadrature of a sphere's strength, 200 divisions a
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(256) void k_direct_src(const DirectJob *__restrict_
                                                     unsigned long long *stats) {
     __shared__ uint32_t stk_all[(BLK ? RT_SRC_ROWS : STK) * 256];
     uint32_t *stk = stk_all + threadIdx.x;
-    uint32_t ovf[BLK ? RT_BLK_OVF(RT_SRC_ROWS) : 1];
+    uint32_t ovf[BLK ? blk_ovf(RT_SRC_ROWS, MK) : 1];
     const uint32_t lane = threadIdx.x & 63;
     Cnt<COUNT, MK> cnt{};
     uint32_t nray = 0;
@@ -682,7 +682,7 @@ int launch_direct_src(const DirectJob *jobs, uint32_t njobs, uint32_t item_lo, u
     int rc = 0;
     with_flags(stats ? counting_flags(flags) : flags, [&](auto fl) {
         rc = launch_direct_src_t<decltype(fl)::value>(jobs, njobs, item_lo, nitems, depth, counter, err, stats, ncu, st,
-                                                      (flags & RT_FL_BLK) != 0);
+                                                      (flags & RT_FL_BLK) && !(flags & RT_FL_WIDE));
     });
     return rc;
 }

@@ -20,6 +20,7 @@ struct Scene {
     std::vector<void *> own;
     size_t bytes = 0;
     int builder = 0;  // 1 = PLOC, 0 = Karras LBVH
+    bool wide = false;  // the block tree's links are wide
 };
 
 // Largest primitive count of a scene: leaf tags and hit words carry a 30-bit primitive index.
@@ -48,10 +49,11 @@ int check_work_items(uint64_t items, const char *what);
 int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, const uint32_t *uuid,
                 const uint32_t *twos, int px, int py, hipStream_t st);
 void scene_free(Scene &S);
-// Writes the block tree blk (rt_types.h) of nn4 BVH4 nodes over nleaf records, and into each node where its children
+// Writes the block tree blk (rt_types.h; wide: with wide links) of nn4 BVH4 nodes over nleaf records, and into each node where its children
 // lie.  Returns 0, 1 when the scene is too large
 // for the nodes' steps (extents above 255 x 2^103: the traversals then walk the binary tree), or -1.
-int write_blocks(uint32_t nn4, uint32_t nleaf, float4 *node4, const float4 *rec, uint4 *blk, hipStream_t st);
+int write_blocks(uint32_t nn4, uint32_t nleaf, float4 *node4, const float4 *rec, uint4 *blk, bool wide,
+                 hipStream_t st);
 // Texture masks (RayTracingGeometry mask_data / mask_sizes / mask_IDs / uv_data / uv_IDs,
 // R/include/RayTracingTypes.h:72-77): nmasks masks of sizes[m] = (width, height) texels, one byte per texel
 // (0 = transparent) concatenated row-major in texels; mask_id[P] (-1 = none); uv[P][4][2] (null = zeros)

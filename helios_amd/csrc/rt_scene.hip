@@ -455,9 +455,9 @@ __device__ __forceinline__ int q_exponent(double ext, double m) {
     return x < -126 ? -126 : (x > 103 ? 103 : x);
 }
 
-// base[t]: block of node t's first child
+// base[t]: block of node t's first child; shift: log2 of a link's units a block
 __device__ __forceinline__ void blk_node(uint32_t t, const float4 *__restrict__ node4, const uint32_t *__restrict__ base,
-                                         uint4 *__restrict__ dst, int *bad) {
+                                         uint32_t shift, uint4 *__restrict__ dst, int *bad) {
     const float4 *o = node4 + (size_t)t * 8;
     const uint32_t cnt = __float_as_uint(o[7].x);
     uint32_t org[3], wl[3], wh[3], w = 0u;
@@ -497,11 +497,11 @@ __device__ __forceinline__ void blk_node(uint32_t t, const float4 *__restrict__ 
     uint32_t code = 0u;
     for (uint32_t k = 0; k < 4; k++) {
         const uint32_t c = k < cnt ? k : 0u;
-        code |= ((c << 6) | ((lk[c] & RT_LEAF_BIT) ? RT_BLK_REC : 0u)) << (8 * k);
+        code |= ((c << shift) | ((lk[c] & RT_LEAF_BIT) ? RT_BLK_REC : 0u)) << (8 * k);
     }
     dst[0] = make_uint4(org[0], org[1], org[2], w);
     dst[1] = make_uint4(wl[0], wh[0], wl[1], wh[1]);
-    dst[2] = make_uint4(wl[2], wh[2], code, 64u * base[t]);
+    dst[2] = make_uint4(wl[2], wh[2], code, base[t] << shift);
     dst[3] = make_uint4(0u, 0u, 0u, 0u);
 }
 
@@ -512,11 +512,12 @@ __global__ void k_blk_count(uint32_t nn4, const float4 *__restrict__ node4, uint
 
 // one thread per (node, child slot); thread 0 also writes the root
 __global__ void k_blocks(uint32_t nn4, float4 *node4, const float4 *__restrict__ rec,
-                         const uint32_t *__restrict__ base, uint4 *__restrict__ blk, int *__restrict__ bad) {
+                         const uint32_t *__restrict__ base, uint32_t shift, uint4 *__restrict__ blk,
+                         int *__restrict__ bad) {
     const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t t = g >> 2, k = g & 3u;
     if (t >= nn4) return;
-    if (g == 0) blk_node(0u, node4, base, blk, bad);
+    if (g == 0) blk_node(0u, node4, base, shift, blk, bad);
     if (k == 0) node4[(size_t)t * 8 + 7].y = __uint_as_float(base[t]);
     if (k >= __float_as_uint(node4[(size_t)t * 8 + 7].x)) return;
     const uint32_t lk = __float_as_uint(((const float *)(node4 + (size_t)t * 8 + 6))[k]);
@@ -525,7 +526,7 @@ __global__ void k_blocks(uint32_t nn4, float4 *node4, const float4 *__restrict__
         const uint4 *r = (const uint4 *)rec + (size_t)(lk & ~RT_LEAF_BIT) * 4;
         for (int q = 0; q < 4; q++) dst[q] = r[q];
     } else {
-        blk_node(lk, node4, base, dst, bad);
+        blk_node(lk, node4, base, shift, dst, bad);
     }
 }
 
@@ -711,7 +712,8 @@ struct Scratch {
 // bytes of the block tree of nn4 nodes over nleaf records and of the build's check word
 static size_t blk_bytes(uint32_t nn4, uint32_t nleaf) { return 64 * ((size_t)nn4 + nleaf) + 64; }
 
-int write_blocks(uint32_t nn4, uint32_t nleaf, float4 *node4, const float4 *rec, uint4 *blk, hipStream_t st) {
+int write_blocks(uint32_t nn4, uint32_t nleaf, float4 *node4, const float4 *rec, uint4 *blk, bool wide,
+                 hipStream_t st) {
     int *bad = (int *)(blk + 4 * ((size_t)nn4 + nleaf));
     Scratch counts, scan;
     CK(hipMalloc(&counts.p, sizeof(uint32_t) * 2 * (size_t)nn4));
@@ -724,7 +726,7 @@ int write_blocks(uint32_t nn4, uint32_t nleaf, float4 *node4, const float4 *rec,
     k_blk_count<<<blocks(nn4, 256), 256, 0, st>>>(nn4, node4, cnt);
     CK(hipGetLastError());
     CK(hipcub::DeviceScan::ExclusiveScan(scan.p, tmp_bytes, cnt, base, hipcub::Sum(), 1u, (int)nn4, st));
-    k_blocks<<<blocks((size_t)nn4 * 4, 256), 256, 0, st>>>(nn4, node4, rec, base, blk, bad);
+    k_blocks<<<blocks((size_t)nn4 * 4, 256), 256, 0, st>>>(nn4, node4, rec, base, wide ? 2u : 6u, blk, bad);
     CK(hipGetLastError());
     int hbad = 0;
     CK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -872,10 +874,12 @@ int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, cons
             CK(hipMalloc(&node4, sizeof(float4) * 8 * (size_t)(nleaf - 1)));
             S.own.push_back(node4);
             if (build_bvh4(nleaf, child, lbox, ibox, node4, nnode4, depth4, st)) return -1;
-            if ((uint64_t)nnode4 + nleaf <= RT_BLK_MAX) {
+            // wide links where the others do not reach, or with more stack rows (three a level)
+            S.wide = (uint64_t)nnode4 + nleaf > RT_BLK_MAX || 3 * depth4 + 1 > RT_STACK;
+            if (!S.wide || ((uint64_t)nnode4 + nleaf <= RT_BLK_MAX_WIDE && 3 * depth4 + 1 <= RT_STACK_WIDE)) {
                 CK(hipMalloc(&blk, blk_bytes(nnode4, nleaf)));
                 S.own.push_back(blk);
-                const int wrote = write_blocks(nnode4, nleaf, node4, rec, blk, st);
+                const int wrote = write_blocks(nnode4, nleaf, node4, rec, blk, S.wide, st);
                 if (wrote < 0) return -1;
                 if (wrote > 0) {
                     S.own.pop_back();
@@ -907,7 +911,7 @@ int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, cons
     S.h.order = vals2;
     // a BVH4 traversal pushes at most 3 entries per level: use it only when that fits the wave stack (128)
     S.h.node4 = (node4 && 3 * depth4 + 1 <= 128) ? node4 : nullptr;
-    S.h.blk = 3 * depth4 + 1 <= RT_STACK ? blk : nullptr;
+    S.h.blk = blk;
     S.h.nnode4 = nnode4;
     S.h.depth4 = depth4;
     S.h.nleaf = nleaf;
@@ -1042,6 +1046,7 @@ void scene_free(Scene &S) {
     S.d = nullptr;
     S.twos = nullptr;
     S.bytes = 0;
+    S.wide = false;
     memset(&S.h, 0, sizeof(S.h));
 }
 

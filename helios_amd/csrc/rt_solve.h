@@ -75,7 +75,8 @@ struct SolveCtx {
 };
 // traversal flags of launches on scene S from this context (RT_FL_*)
 inline int scene_flags(const Scene &S, const SolveCtx &sx) {
-    return (S.h.mdesc ? RT_FL_MASK : 0) | (sx.watertight ? RT_FL_WT : 0) | (S.h.blk ? RT_FL_BLK : 0);
+    return (S.h.mdesc ? RT_FL_MASK : 0) | (sx.watertight ? RT_FL_WT : 0) |
+           (S.h.blk ? RT_FL_BLK | (S.wide ? RT_FL_WIDE : 0) : 0);
 }
 
 // The per-sun part of a solve (K suns share everything else).

@@ -65,7 +65,7 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
     __shared__ uint32_t stk_all[ROWS * WPB * 64];
     __shared__ float queue_all[5 * WPB * 64];
     // stack rows beyond the LDS part, in private memory
-    uint32_t ovf[RT_BLK_OVF(ROWS)];
+    uint32_t ovf[blk_ovf(ROWS, MK)];
     lds_u32 *stk = (lds_u32 *)stk_all + threadIdx.x;
     const uint32_t stride = WPB * 64;
     const uint32_t lane = threadIdx.x & 63;
@@ -243,7 +243,7 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
                     L.ni = RT_BLK_DONE;
                     break;
                 }
-                if (inner) blk_node_step<ROWS>(blk, L, stk, ovf, stride);
+                if (inner) blk_node_step<ROWS, MK>(blk, L, stk, ovf, stride);
             }
             if (__builtin_amdgcn_inverse_ballot_w64(mpend)) {
                 uint32_t slot_unused;
@@ -691,8 +691,16 @@ int launch_diffuse(const DiffuseJob *job, uint32_t total, uint32_t depth, uint32
     }
     with_flags(flags, [&](auto fl) {
         constexpr int FL = decltype(fl)::value;
+        // the rarer kernels come with two waves a workgroup alone: as many waves a CU as the configuration asks for
+        LaunchCfg two = cfg;
+        two.blocks_per_cu = std::max(1u, cfg.blocks_per_cu * wpb / 2u);
+        const uint32_t g2 = grid_for(two, ncu, total, 2);
         if (!(flags & RT_FL_BLK)) {
-            k_diffuse_bin<2, RT_STACK, false, FL><<<grid_for(cfg, ncu, total, 2), 128, 0, st>>>(job, total, counter, ch, err, stats);
+            k_diffuse_bin<2, RT_STACK, false, FL><<<g2, 128, 0, st>>>(job, total, counter, ch, err, stats);
+            return;
+        }
+        if (flags & RT_FL_WIDE) {
+            k_diffuse<2, FL | RT_FL_WIDE><<<g2, 128, 0, st>>>(job, total, counter, ch, err);
             return;
         }
         switch (wpb) {

@@ -859,8 +859,15 @@ struct BlkRay {
 // A lane's stack: row r < ROWS in the wave's LDS array (lane stride 4 B, row stride 4 x `stride`), rows from ROWS on
 // in the lane's private array `ovf`, whose entry 0 is row ROWS - 2 (see the pushes).  Row 0 holds RT_BLK_DONE, so
 // taking the top entry of an empty stack ends the trace without a test of its own.  The tree's depth bounds the
-// rows (3 per level): the launchers choose this traversal only when they fit RT_STACK.
-#define RT_BLK_OVF(ROWS) (RT_STACK + 5 - (ROWS))
+// rows (3 per level): a tree that needs more than RT_STACK has wide links, one that needs more than RT_STACK_WIDE is
+// not built.
+constexpr int blk_ovf(int rows, int flags) { return ((flags & RT_FL_WIDE) ? RT_STACK_WIDE : RT_STACK) + 5 - rows; }
+// The block at a link (whose low bits may hold RT_BLK_REC)
+template <int FL>
+__device__ __forceinline__ const char *blk_at(const char *blk, uint32_t link) {
+    if constexpr ((FL & RT_FL_WIDE) != 0) return blk + ((uint64_t)(link & ~3u) << 4);
+    else return blk + (link & ~63u);
+}
 template <int ROWS>
 __device__ __forceinline__ uint32_t blk_pop(BlkRay &L, const lds_u32 *stk, const uint32_t *ovf, uint32_t stride) {
     L.sp--;
@@ -954,9 +961,9 @@ __device__ __forceinline__ void keep_until(uint32_t offset, float &v) {
 // - pushes need no branches: the three farthest keys are stored above the stack's top whether they are hits or
 //   not (a key that is not lies above the new top).  Keys of missed children are 0x80000000: the smallest as int,
 //   so last in the descending order, and above every hit as unsigned, so never the nearest.
-template <int ROWS, bool HOLD = false>
+template <int ROWS, int FL, bool HOLD = false>
 __device__ __forceinline__ void blk_node_step(const char *blk, BlkRay &L, lds_u32 *stk, uint32_t *ovf, uint32_t stride) {
-    const uint4 *nd = (const uint4 *)(blk + L.ni);
+    const uint4 *nd = (const uint4 *)((FL & RT_FL_WIDE) ? blk + ((uint64_t)L.ni << 4) : blk + L.ni);
     const uint4 a = nd[0], b = nd[1], c = nd[2];
     // the entry a pop would take, read beside the node
     const uint32_t sp0 = L.sp;
@@ -1021,7 +1028,7 @@ __device__ __forceinline__ void blk_leaf(const char *blk, const float4 *recs, ui
                                          uint32_t skip, uint32_t &slot) {
     uint32_t id;
     float t;
-    const float4 *r = (const float4 *)(blk + (link & ~63u));
+    const float4 *r = (const float4 *)blk_at<MK>(blk, link);
     // castRays takes a patch or triangle beyond 1e-6 and a voxel at 1e-6 or beyond
     // (CD/src/CollisionDetection_RayTracing.cpp:1562, 1595, 1681)
     if (leaf_hit_at<CD, MK>(r, recs, L.o, L.d, skip, id, t) &&

@@ -16,8 +16,10 @@
 #define RT_FL_WT 2
 // host-side launch flag (not a kernel template argument): every job of a direct launch has an occlusion grid
 #define RT_FL_GRIDS 4
-// host-side launch flag: the scene has a block tree whose traversal fits the stack
+// host-side launch flag: the scene has a block tree
 #define RT_FL_BLK 8
+// its links are wide (with RT_FL_BLK; a kernel template argument where the block tree is traversed)
+#define RT_FL_WIDE 16
 #define RT_NOT_LAUNCHED 0xFFFFFFFEu
 #define RT_HIT_BOTTOM 0x80000000u
 
@@ -64,10 +66,15 @@ struct DevScene {
 //   w2 = lo.z, hi.z; byte k = (64 k | record bit) of child k; byte offset of the children
 // An unused child is an empty box (lower bound 255, upper bound 0) with child 0's code: a ray so far away that
 // the two bounds round to one distance would visit child 0 again, which changes no closest hit.
-// 32-bit byte offsets reach 2^26 blocks (about 45 million primitives); a larger scene has no block tree.
+// 32-bit byte offsets reach 2^26 blocks (about 45 million primitives).  Beyond them, and where the tree's depth needs
+// more than RT_STACK stack rows, the links are wide: they count 16 bytes (codes 4 k | record bit), which reaches 2^30
+// blocks, more than RT_MAX_PRIMS records and their nodes make up, and the kernels that walk them are instances of their
+// own with RT_STACK_WIDE rows.
 #define RT_BLK_REC 1u
 #define RT_BLK_DONE 0xFFFFFFFFu
 #define RT_BLK_MAX 0x3FFFFFFull
+#define RT_BLK_MAX_WIDE 0x3FFFFFFFull
+#define RT_STACK_WIDE 128
 
 // Occlusion grid of one collimated-source direction: every traced primitive's padded projection onto the
 // plane perpendicular to the direction, binned into a uniform grid (CSR: start[cell] .. start[cell + 1]

@@ -136,7 +136,7 @@ bool run(const char *what, int (*call)(rt::Scene &), bool earlier) {
 
 int main() {
     const auto blocks = [](rt::Scene &S) {
-        return rt::write_blocks(NN4, P, const_cast<float4 *>(S.h.node4), S.h.rec, const_cast<uint4 *>(S.h.blk), nullptr);
+        return rt::write_blocks(NN4, P, const_cast<float4 *>(S.h.node4), S.h.rec, const_cast<uint4 *>(S.h.blk), false, nullptr);
     };
     bool ok = true;
     for (bool earlier : {false, true}) {
