@@ -27,7 +27,7 @@ namespace rt {
 // - Refills start below RT_BLK_REFILL traversing lanes (40 to 58 swept: 48 best on all scenes).
 // A pass of that orchard took 110 ms over 64-byte nodes with explicit links, 87 ms so (the masked kernel on 140,000
 // texture-masked patches, 1,024 rays: 95 to 65 ms).  LDS per wave: RT_BLK_ROWS stack rows and the queue's five; 17 rows let 28 waves
-// share the CU's 160 KB, and 7 waves per SIMD need no spills.  More than 11 entries lie on one lane in 0.6 % of its
+// share the CU's 160 KB.  More than 11 entries lie on one lane in 0.6 % of its
 // steps and so on some lane of a wave in a quarter of them; 17 rows against 15 with 8 waves: 427 and 431 ms for
 // the orchard's five passes, 21 rows with 6 waves 459, 26 with 5 waves 506.
 #ifndef RT_LEAF_BATCH_PARKED
@@ -39,16 +39,14 @@ namespace rt {
 #ifndef RT_BLK_ROWS
 #define RT_BLK_ROWS 17
 #endif
-// Waves per SIMD the compiler must fit the kernel into.  Watertight predicates: 6 (their larger leaf test would
-// spill).
+// Waves per SIMD the compiler must fit the kernel into.  At 7 the plain kernel spills no registers and the masked one two
+// or three.  Watertight predicates: 6, where their larger leaf test spills three (with masks 7 to 14, at 7 waves 19 to 25:
+// 70,000 texture-masked patches x 400 rays 11.9 ms either way).
 #ifndef RT_DIFFUSE_WAVES_PER_EU
 #define RT_DIFFUSE_WAVES_PER_EU 7
 #endif
 #ifndef RT_DIFFUSE_WAVES_PER_EU_WT
 #define RT_DIFFUSE_WAVES_PER_EU_WT 6
-#endif
-#ifndef RT_DIFFUSE_WAVES_PER_EU_MASKED
-#define RT_DIFFUSE_WAVES_PER_EU_MASKED 7
 #endif
 // rr / n and rr % n of a ray number rr < n * n: a multiply by ceil(2^32 / n) is exact while n^3 < 2^32
 __device__ __forceinline__ void ray_cell(uint32_t rr, uint32_t n, uint32_t inv, uint32_t &lx, uint32_t &ly) {
@@ -57,9 +55,7 @@ __device__ __forceinline__ void ray_cell(uint32_t rr, uint32_t n, uint32_t inv, 
 }
 
 template <int WPB, int MK>
-__global__ __launch_bounds__(WPB * 64, (MK & RT_FL_MASK) ? RT_DIFFUSE_WAVES_PER_EU_MASKED
-                                       : (MK & RT_FL_WT) ? RT_DIFFUSE_WAVES_PER_EU_WT
-                                                         : RT_DIFFUSE_WAVES_PER_EU)
+__global__ __launch_bounds__(WPB * 64, (MK & RT_FL_WT) ? RT_DIFFUSE_WAVES_PER_EU_WT : RT_DIFFUSE_WAVES_PER_EU)
 void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *counter, uint32_t chunk, int *err) {
     constexpr int ROWS = RT_BLK_ROWS;
     __shared__ uint32_t stk_all[ROWS * WPB * 64];
