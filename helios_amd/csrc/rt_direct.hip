@@ -32,12 +32,11 @@ __device__ __forceinline__ void grid_cell(const SunGrid &G, v3f o, uint32_t &b, 
 // by 1e-5 of the scene's largest coordinate) is below the ray origin's depth lies wholly behind the origin:
 // no FP32 hit of it can have t > 1e-4 (the FP32 errors of t, of the key and of the depth are a few ulps of
 // that coordinate), so it is skipped without loading its record.
-// Returns 1 when a candidate occludes the ray, 2 when the list is known to hold no further occluder (a
-// sorted list whose next key is below the origin's depth), else 0.
+// Returns 1 when a candidate occludes the ray, 2 when the list holds no further occluder (its next key is below
+// the origin's depth), else 0.
 template <typename C>
-__device__ __forceinline__ int grid_pair(const uint2 *ents, bool sorted, float depth, const float4 *recs,
-                                         uint32_t nleaf, uint32_t p, uint32_t e, v3f o, v3f d, uint32_t skip,
-                                         C &cnt) {
+__device__ __forceinline__ int grid_pair(const uint2 *ents, float depth, const float4 *recs, uint32_t nleaf,
+                                         uint32_t p, uint32_t e, v3f o, v3f d, uint32_t skip, C &cnt) {
     const bool two = p + 1 < e;
     const uint2 e0 = ents[p];
     const uint2 e1 = two ? ents[p + 1] : make_uint2(RT_MISS, __float_as_uint(-INFINITY));
@@ -63,15 +62,16 @@ __device__ __forceinline__ int grid_pair(const uint2 *ents, bool sorted, float d
         h1 = mask_hit_opaque(recs, __float_as_uint(b3.w), (tb & RT_PATCH_BIT) != 0, ua1, ub1, b1.w, b2.w);
     cnt.prims += (v0 ? 1u : 0u) + ((v1 && !h0) ? 1u : 0u);  // the tests a one-at-a-time scan makes
     if (h0 || h1) return 1;
-    return (sorted && (!(key0 >= depth) || (two && !(key1 >= depth)))) ? 2 : 0;
+    return (!(key0 >= depth) || (two && !(key1 >= depth))) ? 2 : 0;
 }
 
 // ------------------------------------------------------------------------------------------------
 // direct rays
 // ------------------------------------------------------------------------------------------------
-// COUNT: the counting variant (stats != nullptr) traces every ray on its own (per-lane LDS stack) so the
-// counters hold single-ray node visits and primitive tests -- the algorithmic work per ray -- rather than
-// the packet's visits.  Both variants make the same occlusion decision for every ray.
+// COUNT: the counting variant (stats != nullptr) traces every ray on its own (per-lane LDS stack, or the
+// occlusion grid's lists when the job has one) so the counters hold single-ray node visits and primitive
+// tests -- the algorithmic work per ray -- rather than the packet's visits.  The other variant takes the
+// launches without grids and walks the BVH4 in packets.  Both make the same occlusion decision for every ray.
 #ifndef RT_DIRECT_REFILL
 #define RT_DIRECT_REFILL 24
 #endif
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(WPB * 64, (COUNT || MK) ? 1 : RT_DIRECT_WAVES_PER_E
             uint32_t ty = ldu(ldu(&sc.type) + i);
             float sum_out = 0.f;
             bool top = true;
-            const SunGrid *grid = ldu(&J.grid);
+            const SunGrid *grid = COUNT ? ldu(&J.grid) : nullptr;
             const float4 *recs = ldu(&sc.rec);
             const uint32_t *mdesc = ldu(&sc.mdesc);
             const uint32_t mdi = (MK && mdesc) ? ldu(mdesc + i) : RT_MISS;
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(WPB * 64, (COUNT || MK) ? 1 : RT_DIRECT_WAVES_PER_E
                     // sum is count x strength, rounded once (exact up to that rounding)
                     uint32_t lit = 0;
                     const uint32_t seed = ldu(&J.seed);
-                    if (grid) {
+                    if (COUNT && grid) {
                         // Occlusion grid: each lane scans its ray's cell list two candidates per step.  A lane
                         // whose ray ends (occluder found, or list exhausted: lit) takes the primitive's next
                         // ray; idle lanes are refilled together once fewer than RT_DIRECT_REFILL lanes still
@@ -144,7 +144,6 @@ __global__ __launch_bounds__(WPB * 64, (COUNT || MK) ? 1 : RT_DIRECT_WAVES_PER_E
                         // and the summation grouping differ).
                         const SunGrid &G = *grid;
                         const uint2 *ents = G.ents;
-                        const bool sorted = G.sorted != 0;
                         const uint32_t nleaf = ldu(&sc.nleaf);
                         const float gw0 = G.w[0], gw1 = G.w[1], gw2 = G.w[2];
                         uint32_t r = lane, pc = 0, pe = 0;
@@ -166,8 +165,7 @@ __global__ __launch_bounds__(WPB * 64, (COUNT || MK) ? 1 : RT_DIRECT_WAVES_PER_E
                             while (true) {
                                 if (act) {
                                     const int res = pc >= pe ? 2
-                                                             : grid_pair(ents, sorted, depth, recs, nleaf, pc, pe,
-                                                                         o, dir, i, cnt);
+                                                             : grid_pair(ents, depth, recs, nleaf, pc, pe, o, dir, i, cnt);
                                     if (res == 2) lit++;
                                     if (res != 0) act = false;
                                     else pc += 2;
@@ -607,9 +605,6 @@ __global__ __launch_bounds__(256) void k_direct_src(const DirectJob *__restrict_
     add_stats(stats, cnt, nray);
 }
 
-#ifndef RT_DIRECT_QUEUE
-#define RT_DIRECT_QUEUE 1
-#endif
 template <int MK>
 static int launch_direct_t(const DirectJob *jobs, uint32_t njobs, uint32_t total, uint32_t depth, uint32_t *counter,
                            int *err, unsigned long long *stats, const LaunchCfg &cfg, int ncu, hipStream_t st,
@@ -619,7 +614,7 @@ static int launch_direct_t(const DirectJob *jobs, uint32_t njobs, uint32_t total
     k_zero_queue<<<1, RT_QUEUE_WORDS, 0, st>>>(counter);
     uint32_t wpb = cfg.waves_per_block;
     uint32_t g = grid_for(cfg, ncu, total, wpb);
-    if (RT_DIRECT_QUEUE && grids && !stats) {
+    if (grids && !stats) {
         switch (wpb) {
             case 1: k_direct_q<1, MK><<<g, 64, 0, st>>>(jobs, njobs, total, counter, ch); break;
             case 2: k_direct_q<2, MK><<<g, 128, 0, st>>>(jobs, njobs, total, counter, ch); break;

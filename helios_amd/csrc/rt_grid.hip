@@ -422,7 +422,6 @@ int build_sun_grids(GridSet &gs, const Scene &S, const float *dirs, uint32_t n, 
         G.inv_cs = 1.f;
         G.nx = G.ny = 1;
         G.sbase = 0;
-        G.sorted = 0;
         G.start = nullptr;
         G.ents = nullptr;
     }
@@ -523,12 +522,10 @@ int build_sun_grids(GridSet &gs, const Scene &S, const float *dirs, uint32_t n, 
             GK(hipGetLastError());
         }
     }
-    const bool sorted = true;
     for (uint32_t j = 0; j < n; j++) {
         hg[j].start = starts + base[j];
         hg[j].ents = ents + ibase[j];
         hg[j].sbase = (uint32_t)ibase[j];
-        hg[j].sorted = sorted ? 1u : 0u;
     }
     GK(hipMemcpyAsync(dgrids, hg.data(), n * sizeof(SunGrid), hipMemcpyHostToDevice, st));
     GK(hipStreamSynchronize(st));

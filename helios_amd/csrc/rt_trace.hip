@@ -8,8 +8,8 @@ namespace rt {
 // ------------------------------------------------------------------------------------------------
 // A wave keeps 64 rays in flight; a lane whose traversal ends writes its hit word and takes another ray, and
 // the wave opens the next primitive of the work queue when the current one has no rays left, so lanes do not
-// idle for the longest ray of a fixed group of 64.  Every ray is traced exactly as a plain per-ray
-// trace_loop() would trace it; only the assignment of rays to lanes and steps differs.
+// idle for the longest ray of a fixed group of 64.  Every ray is traced exactly as on its own, over up to 32
+// periodic wraps (diffuse_raygen.comp:498-560); only the assignment of rays to lanes and steps differs.
 //
 // k_diffuse walks the block tree.  Two units of a CU bound it together (SQ and TCP counters, 86 ms a pass of the
 // 1,001,600-primitive orchard, 439 M rays): the vector ALU (one instruction per SIMD every 3.1 cycles where the mix
@@ -106,7 +106,7 @@ void k_diffuse(const DiffuseJob *__restrict__ job, uint32_t total, uint32_t *cou
     uint32_t pend = 0u;   // link of the parked record of the lanes in mpend
     uint64_t mpend = 0u;  // lanes with a parked record (none outside the traversal loop)
     while (true) {
-        // finish lanes whose traversal ended: periodic wrap (as trace_loop: at most 32 traces), else write
+        // finish lanes whose traversal ended: periodic wrap (at most 32 traces), else write
         if (busy && L.ni == RT_BLK_DONE) {
             bool done = true;
             if (nbbox) {
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(WPB * 64) void k_diffuse_bin(const DiffuseJob *__re
     lane_start(L, nleaf);
     uint32_t my_i = 0, my_r = 0, wraps = 0;
     while (true) {
-        // finish lanes whose traversal ended: periodic wrap (as trace_loop: at most 32 traces), else write
+        // finish lanes whose traversal ended: periodic wrap (at most 32 traces), else write
         if (busy && !trav) {
             bool done = true;
             if (nbbox) {

@@ -7,15 +7,13 @@
 //   trace_any       occlusion query: any accepted hit with t <= tmax ends the traversal.  The direct
 //                   pass only needs "occluded or not"; with the nearest periodic face as tmax this
 //                   reproduces the reference decision (closest hit vs periodic face) exactly.
-//   k_direct        direct rays (R/shaders/direct_raygen.comp:323-731): one wave per (job, primitive),
-//                   d*d stratified samples, occlusion trace with periodic wrap, compensated sums of
-//                   ray strength split by lit face.
-//   k_diffuse       diffuse/scatter rays (R/shaders/diffuse_raygen.comp:330-560): one wave per
-//                   (pass, primitive), both faces, writes one hit word per ray.
-//   k_gather_*      per-primitive compensated reduction of gathered radiation_out / sky flux over a
-//                   hit table (diffuse_raygen.comp:562-652), deterministic (no atomics).
-//   k_cast          CollisionDetection::castRaysSoA (CD/src/CollisionDetection_RayTracing.cpp:551-680,
-//                   980-1080): one thread per ray, CD predicates, face-forwarded normal.
+//   packet_any4     the same for the 64 rays of a wave over the BVH4 (packet_any: over the BVH2).
+//   WaveQueue       work queue of a persistent launch.
+//   LaneRay, lane_* resumable closest-hit traversal of one lane over the BVH2 (counting kernels, scenes
+//                   without a block tree).
+//   BlkRay, blk_*   the same over the block tree (rt_types.h).
+// The kernels that use them are in rt_trace.hip (diffuse rays and gathers), rt_direct.hip (direct rays),
+// rt_cast.hip (castRays, cameras) and rt_glass.hip (translucent covers).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -56,8 +54,6 @@ struct NoCntT {
     static constexpr bool wt = (MK & RT_FL_WT) != 0;
     static constexpr int flags = MK;
 };
-using TCnt = TCntT<RT_FL_MASK>;
-using NoCnt = NoCntT<RT_FL_MASK>;
 template <bool COUNT, int MK>
 using Cnt = typename std::conditional<COUNT, TCntT<MK>, NoCntT<MK>>::type;
 
@@ -169,12 +165,6 @@ struct NodeTest {
     uint32_t c0, c1;
     bool h0, h1;
 };
-
-__device__ __forceinline__ NodeTest node_test_p(const float4 *nodes, uint32_t ni, const RayPre &rp, float tlim);
-
-__device__ __forceinline__ NodeTest node_test(const DevScene &sc, uint32_t ni, const RayPre &rp, float tlim) {
-    return node_test_p(sc.node, ni, rp, tlim);
-}
 
 __device__ __forceinline__ NodeTest node_test_p(const float4 *nodes, uint32_t ni, const RayPre &rp, float tlim) {
     const float4 *nd = nodes + (size_t)ni * 4;
@@ -568,28 +558,6 @@ __device__ __forceinline__ v3f wrap_at(const DevScene &sc, v3f o, v3f d, float b
     else if (sc.py && fabsf(hp.y - sc.dom[2]) <= eps) w.y += wy - eps;
     else if (sc.py && fabsf(hp.y - sc.dom[3]) <= eps) w.y -= wy - eps;
     return w;
-}
-
-// Closest-hit trace with up to 32 periodic wraps (diffuse_raygen.comp:498-560 without translucent
-// covers).  Returns the last traversal result.
-template <int STK, typename C>
-__device__ __forceinline__ uint32_t trace_loop(const DevScene &sc, v3f o, v3f d, float tmin, uint32_t skip,
-                                               bool &exhausted, uint32_t *stk, uint32_t stride, int *err, C &cnt) {
-    uint32_t hit = RT_MISS;
-    v3f cur = o;
-    exhausted = true;
-    for (int step = 0; step < 32; ++step) {
-        float t;
-        uint32_t slot;
-        hit = trace_closest<false, STK>(sc, cur, d, tmin, skip, 1e30f, t, slot, stk, stride, err, cnt);
-        if (sc.nbbox) {
-            float bt = nearest_face(sc, cur, d, t);
-            if (bt > 0.f) { cur = wrap_at(sc, cur, d, bt); continue; }
-        }
-        exhausted = false;
-        break;
-    }
-    return hit;
 }
 
 // Occlusion towards a collimated source with periodic wraps (direct_raygen.comp:603-672 without

@@ -89,13 +89,12 @@ struct SunGrid {
     float g0u, g0v;        // grid origin
     float inv_cs;          // 1 / cell size
     uint32_t nx, ny;
-    uint32_t sorted;       // 1: each cell's list is in descending key order (a scan may stop at the first
-                           // key below the ray origin's depth)
     uint32_t sbase;        // start[] values count from sbase (modulo 2^32): cell c lists
                            // ents[start[c] - sbase, start[c + 1] - sbase)
     const uint32_t *start; // [nx*ny + 1]
-    const uint2 *ents;     // this direction's list: (slot | flag, key); the key is the primitive's largest
-                           // depth along w (max over its vertices of v.w), padded
+    const uint2 *ents;     // this direction's lists: (slot | flag, key); the key is the primitive's largest
+                           // depth along w (max over its vertices of v.w), padded; each cell's list is in
+                           // descending key order (a scan may stop at the first key below its origin's depth)
 };
 
 // one direct trace job: one scene, one collimated source
