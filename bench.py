@@ -60,29 +60,26 @@ def pct(a, q):
     return float(np.percentile(np.asarray(a, np.float64), q)) if len(a) else None
 
 
-# position of the COUNT template argument of the kernels that have one: k_cast_bin / k_camera / k_direct_src<STK,
-# COUNT, FLAGS, ...>, k_direct / k_diffuse_bin<WAVES, STK, COUNT, FLAGS>, and in profiles of earlier kernels k_cast<STK,
-# COUNT, FLAGS> and k_diffuse<WAVES, STK, COUNT, FLAGS> (now <WAVES, FLAGS>)
-COUNT_ARG = {"k_cast_bin": 1, "k_camera": 1, "k_direct_src": 1, "k_direct": 2, "k_diffuse_bin": 2, "k_cast": 1,
-             "k_diffuse": 2}
+# template arguments of the ray kernels, as their names list them.  A name of another shape is a kernel of another
+# build (an earlier k_cast<STK, COUNT, FLAGS>, say): a profile that holds it says nothing about the launched one.
+TEMPLATE_ARGS = {"k_cast": ("WAVES", "FLAGS"), "k_diffuse": ("WAVES", "FLAGS"), "k_direct_q": ("WAVES", "FLAGS"),
+                 "k_cast_bin": ("STK", "COUNT", "FLAGS"), "k_diffuse_bin": ("WAVES", "STK", "COUNT", "FLAGS"),
+                 "k_direct": ("WAVES", "STK", "COUNT", "FLAGS"), "k_direct_src": ("STK", "COUNT", "FLAGS", "BLK"),
+                 "k_camera": ("STK", "COUNT", "FLAGS", "SPEC")}
 
 
-def counting_variant(name):
+def template_args(name):
+    """{argument: value} of a ray kernel's name, None for other kernels and for names of another shape."""
     m = re.search(r"(k_\w+)<([^>]*)>", name)
-    if not m or m.group(1) not in COUNT_ARG:
-        return False
-    args = [a.strip() for a in m.group(2).split(",")]
-    return len(args) > COUNT_ARG[m.group(1)] and args[COUNT_ARG[m.group(1)]] == "true"
-
-
-def kernel_flags(name):
-    """The traversal-flags template argument of a ray kernel's name (its last integer argument; boolean
-    arguments such as the camera's specular switch may follow it), as an int, else None."""
-    m = re.search(r"(k_\w+)<([^>]*)>", name)
-    if not m:
+    if not m or m.group(1) not in TEMPLATE_ARGS:
         return None
-    nums = [a.strip() for a in m.group(2).split(",") if a.strip().isdigit()]
-    return int(nums[-1]) if nums else None
+    keys, vals = TEMPLATE_ARGS[m.group(1)], [a.strip() for a in m.group(2).split(",")]
+    if len(keys) != len(vals):
+        return None
+    flag = {"COUNT", "BLK", "SPEC"}
+    if any((v in ("true", "false")) != (k in flag) for k, v in zip(keys, vals)):
+        return None
+    return {k: v == "true" if k in flag else int(v) for k, v in zip(keys, vals)}
 
 
 def pmc_profile(kernel, profile="pmc_traffic_config3_diurnal.json", flags=0):
@@ -90,7 +87,8 @@ def pmc_profile(kernel, profile="pmc_traffic_config3_diurnal.json", flags=0):
     its largest timed (non-counting) dispatch with the traversal flags of the timed launch (0: no masks,
     reference predicates; other variants in the same profile, such as the watertight solves of the predicate
     comparison, are different kernels), each scaled by what the counter read for a copy of known size, and
-    that kernel's L2 hit rate when the profile has one.  None without a profile of the kernel."""
+    that kernel's L2 hit rate when the profile has one.  None without a profile of the kernel in its present
+    shape (TEMPLATE_ARGS)."""
     path = os.path.join(ROOT, "profiles", profile)
     if not os.path.exists(path):
         return None
@@ -98,8 +96,9 @@ def pmc_profile(kernel, profile="pmc_traffic_config3_diurnal.json", flags=0):
         d = json.load(f)
     best = None
     for name, cs in d.get("kernels", {}).items():
-        if (re.search(re.escape(kernel) + r"<", name) and not counting_variant(name)
-                and (flags is None or kernel_flags(name) == flags) and "FETCH_SIZE" in cs and "WRITE_SIZE" in cs):
+        args = template_args(name)
+        if (re.search(re.escape(kernel) + r"<", name) and args and not args.get("COUNT")
+                and (flags is None or args["FLAGS"] == flags) and "FETCH_SIZE" in cs and "WRITE_SIZE" in cs):
             b = cs["FETCH_SIZE"]["max_bytes"] + cs["WRITE_SIZE"]["max_bytes"]
             if best is None or b > best["bytes"]:
                 best = {"bytes": b, "fetch": cs["FETCH_SIZE"]["max_bytes"], "write": cs["WRITE_SIZE"]["max_bytes"],
@@ -132,9 +131,9 @@ def roofline(kernel, avg_launch_ms, canonical_bytes, profile, flags=0, **extra):
                           "exceeds_hbm_peak": canon_gbs > HBM_PEAK_GBS, **extra}}
 
 
-# occlusion-grid direct pass: 8 B cell range per lookup ("nodes" counts lookups), 4 B list entry + 48 B
+# occlusion-grid direct pass: 8 B cell range per lookup ("nodes" counts lookups), 8 B list entry + 48 B
 # primitive record per candidate tested ("prims")
-B_CELL, B_CAND = 8, 52
+B_CELL, B_CAND = 8, 56
 
 
 def bytes_per_ray(c, grid=False):

@@ -601,7 +601,7 @@ __device__ __forceinline__ bool packet_occluded(const DevScene &sc, v3f o, v3f d
 }
 
 // A wave's view of the work queue of a persistent launch: items [0, total) in chunks of `chunk`.  What bounds a
-// queue is its atomics on one address, 11.4 ns each and one after the other: more than a whole item of the direct
+// queue is its atomics on one address, 11.3 ns each and one after the other: more than a whole item of the direct
 // kernel takes the chip (225 rays of a primitive over an occlusion grid, 5 ns) or one of a gather.  So
 // - a launch with at most one chunk a wave uses none: wave w takes chunk w (1,601 primitives: four gathers 0.202
 //   to 0.057 ms, direct 0.060 to 0.027);
@@ -630,8 +630,8 @@ struct WaveQueue {
         }
     }
     // Adds the chunk to counter word w from lane 0 alone and returns its old value.  (Where all lanes add, the compiler
-    // sums them first, in a loop of 64 scalar steps, and one lane adds the sum: the counter is as fast, 11.3 ns a fetch
-    // against 11.4, but a wave waits 600 ns for its fetch where lane 0's takes 96.)
+    // sums them first, in a loop of 64 scalar steps, and one lane adds the sum: 11.3 ns a fetch of a busy counter either
+    // way, 12.0 for a 64-bit one, but with four waves on the chip a fetch takes a wave 2.4 us where lane 0's takes 0.4.)
     __device__ __forceinline__ uint32_t fetch(uint32_t *w) const {
         uint32_t x = 0;
         if ((threadIdx.x & 63) == 0) x = __hip_atomic_fetch_add(w, chunk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
