@@ -27,3 +27,13 @@ def test_profile_of_the_launched_kernel(tmp_path, monkeypatch, kernel, name, fla
     monkeypatch.setattr(bench, "ROOT", str(tmp_path))
     got = bench.pmc_profile(kernel, "p.json", flags)
     assert (got["bytes"] if got else None) == (4.0 if taken else None)
+
+
+def test_committed_profiles_hold_kernels_of_known_shapes():
+    """Every committed profile that a roofline reads has its kernel."""
+    for kernel, profile, flags in (("k_diffuse", "pmc_traffic_config3_diurnal.json", 0),
+                                   ("k_diffuse", "pmc_traffic_config2.json", 0),
+                                   ("k_diffuse", "pmc_traffic_homogeneous_canopy.json", 1),
+                                   ("k_cast", "pmc_traffic_config5_castrays.json", 0),
+                                   ("k_camera", "pmc_traffic_config5_camera.json", 0)):
+        assert bench.pmc_profile(kernel, profile, flags), (kernel, profile)
