@@ -229,15 +229,16 @@ __global__ __launch_bounds__(WPB * 64, (COUNT || MK) ? 1 : RT_DIRECT_WAVES_PER_E
 // LDS that counts its lit rays; the primitive's sums are written once its last ray has ended.  A job change
 // (another direction, grid and output) waits until the rays in flight have ended.  Every ray is tested
 // exactly as in k_direct, and the sums are the same count x strength.
-// The vector ALU bounds it (401,600 primitives x 225 rays x 64 directions, 5.8 G rays: 9.1e10 wave instructions in
-// 122 ms, one per SIMD every 3.3 cycles), so lanes must not idle and work that decides nothing must not run:
+// The vector ALU bounds it (1,001,600 primitives x 225 rays x 64 directions, 14.4 G rays: 2.2e11 wave instructions in
+// 302 ms, one per SIMD every 3.4 cycles; 401,600 primitives: 122 ms), so lanes must not idle and work that decides
+// nothing must not run:
 // - rays are generated up to 64 at a time with every lane active, into the wave's LDS queue, together with the first
 //   two entries of their cell's list; a ray with nothing above it is counted lit there and never queued;
 // - a lane tests one candidate a step (two a step tested the second in vain whenever the first hit), and the
 //   origin's own entry, known by its leaf slot, is passed over without loading its record;
 // - a cell's start and end are one 8-byte load and a pair of entries one 16-byte load (2.5e9 load instructions
 //   where two candidates a step took 3.8e9).
-// That batch's direct pass took 136 ms with two candidates a step and rays generated by the lanes being refilled,
+// The smaller batch's direct pass took 136 ms with two candidates a step and rays generated by the lanes being refilled,
 // 121 ms so.  Refills start below RT_DQ_REFILL scanning lanes (32 to 56 swept: 40 best by 2 %).
 // The lists are sorted by descending key (SunGrid), which the scan's end relies on.
 #define RT_DQ_SLOTS 8

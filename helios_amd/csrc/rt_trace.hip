@@ -11,12 +11,12 @@ namespace rt {
 // idle for the longest ray of a fixed group of 64.  Every ray is traced exactly as on its own, over up to 32
 // periodic wraps (diffuse_raygen.comp:498-560); only the assignment of rays to lanes and steps differs.
 //
-// k_diffuse walks the block tree.  Two units of a CU bound it together (SQ and TCP counters, 86 ms a pass of the
-// 1,001,600-primitive orchard, 439 M rays): the vector ALU (one instruction per SIMD every 3.1 cycles where the mix
-// needs about 3.3) and the vL1D's address path (a load instruction whose lanes lie on different lines takes 43
-// cycles for 64 lanes whatever its width, 1.5 lanes a cycle: about 90 % of the pass).  So a node is three 16-byte
-// loads (rt_types.h), its step is short (blk_node_step()), and the rest keeps as many lanes as it can in each
-// instruction:
+// k_diffuse walks the block tree.  Two units of a CU bound it together (SQ and TA counters, 83 ms a pass of the
+// 1,001,600-primitive orchard, 439 M rays): the vector ALU (one instruction per SIMD every 3.3 cycles, where those of
+// a node step take 2.4 to 4.7) and the vL1D's address unit (busy 80 % of the pass; a load instruction whose lanes lie on
+// different lines takes it 45 cycles for 64 lanes whatever its width).  So a node is three 16-byte loads
+// (rt_types.h), its step is short (blk_node_step()), and the rest keeps as many lanes as it can in each instruction
+// (0.66 of them):
 // - Rays are generated up to 64 at a time with every lane active, into the wave's LDS queue (local sample point
 //   and world direction, 20 B a ray): the hashing, square roots and divisions of a ray (about 1,500 cycles a
 //   wave) ran for the 19 lanes being refilled on average when each refill generated its own rays.  A
@@ -25,11 +25,10 @@ namespace rt {
 //   waits only at a second record or with no links left.  Once RT_LEAF_BATCH_PARKED lanes wait, every parked
 //   record is tested, one per lane, and the node phase goes on (6 to 16 lanes swept: 8 best, 16 3 % slower).
 // - Refills start below RT_BLK_REFILL traversing lanes (40 to 58 swept: 48 best on all scenes).
-// A pass of that orchard took 110 ms over 64-byte nodes with explicit links, 87 ms so (the masked kernel on 140,000
-// texture-masked patches, 1,024 rays: 95 to 65 ms).  LDS per wave: RT_BLK_ROWS stack rows and the queue's five; 17 rows let 28 waves
-// share the CU's 160 KB.  More than 11 entries lie on one lane in 0.6 % of its
-// steps and so on some lane of a wave in a quarter of them; 17 rows against 15 with 8 waves: 427 and 431 ms for
-// the orchard's five passes, 21 rows with 6 waves 459, 26 with 5 waves 506.
+// A pass of that orchard took 110 ms over 64-byte nodes with explicit links, 83 ms so (the masked kernel on 140,000
+// texture-masked patches, 1,024 rays: 95 to 65 ms).  LDS per wave: RT_BLK_ROWS stack rows and the queue's five; 17 rows
+// let 28 waves share the CU's 160 KB.  A step that finds 14 entries or more on a lane goes on in private memory; 17 rows
+// against 15 with 8 waves: 427 and 431 ms for the orchard's five passes, 21 rows with 6 waves 459, 26 with 5 waves 506.
 #ifndef RT_LEAF_BATCH_PARKED
 #define RT_LEAF_BATCH_PARKED 8
 #endif
@@ -462,8 +461,8 @@ constexpr int pow2_up(int n) { int p = 1; while (p < n) p *= 2; return p; }
 // The channel count is exact up to 16: a kernel for the next power of two loaded and added channels that are not
 // there.  Five passes of 1 M primitives x 450 rays, 3 channels: 24.1 to 11.9 ms; three passes of 200,000 x 100 rays:
 // 4 channels 2.04 to 1.43 ms, 8 channels 3.75 to 1.44.  k_gather_chan (lanes over the channels) takes 5.2 ms for these
-// passes at 9 to 17 channels and this kernel 1.60, 1.62 and 1.81 at 9, 12 and 16; more channels than 16 would not fit
-// the registers.
+// passes at 9 to 17 channels and this kernel 1.60, 1.62 and 1.81 at 9, 12 and 16 (112 registers, none spilled).  The rule
+// stops at 16 because the instances do; where the other kernel becomes the better one has not been measured.
 template <int NC, bool SKY, bool ACCT>
 __global__ __launch_bounds__(256) void k_gather_rays(const GatherJob *__restrict__ jobs, uint32_t njobs, uint32_t total,
                                                      uint32_t *counter, uint32_t chunk) {
