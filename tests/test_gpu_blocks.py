@@ -182,18 +182,33 @@ def test_more_blocks_than_byte_offsets_reach(ctx):
 
 @pytest.mark.parametrize("far", [1e30, 1e34, 1e37])
 def test_one_primitive_far_away(ctx, far):
-    """Extents beyond the nodes' largest steps: such a scene is traced without a block tree."""
+    """Extents beyond the nodes' largest steps (the last two): such a scene is traced without a block tree, by the
+    kernels over the binary tree."""
     s = _cloud(60)
     s.transforms[7, 3] = far
     g, o = ctx.scene(s.transforms, s.types, s.twosided), OracleScene.from_arrays(s)
     rng = np.random.default_rng(4)
     O, D = rng.uniform(-0.5, 0.5, (500, 3)).astype(np.float32), rng.normal(size=(500, 3))
     D = (D / np.linalg.norm(D, axis=1, keepdims=True)).astype(np.float32)
-    t, nrm, u = g.cast_rays(O, D)
-    to, no, uo = o.cast_rays(O, D)
-    hit = u != 0xFFFFFFFF
-    assert np.array_equal(u, uo) and hit.sum() > 100
-    assert np.array_equal(t[hit], to[hit]) and np.array_equal(nrm[hit], no[hit])
+    mask = (np.indices((8, 8)).sum(0) % 2).astype(np.uint8)
+    masks = ([mask], np.where(np.arange(s.P) % 3 == 0, -1, 0).astype(np.int32))
+    lamp = ([[0.1, 0.2, 0.9]], [native.SOURCE_DISK], [(0.2, 0.2)], [(np.pi, 0.0, 0.0)])
+    for masked in (False, True):
+        if masked:
+            g.set_masks(*masks)
+            o.set_masks(*masks)
+        for mode in ("reference", "watertight"):
+            try:
+                ctx.set_predicates(mode)
+                with predicates(mode):
+                    assert np.array_equal(g.diffuse_hits(6, 3), o.diffuse_hits(6, 3))
+                    (t, nrm, u), (to, no, uo) = g.cast_rays(O, D), o.cast_rays(O, D)
+                    assert np.allclose(g.direct_sums_src(6, 5, *lamp), o.direct_sums_src(6, 5, *lamp), rtol=1e-5, atol=1e-7)
+            finally:
+                ctx.set_predicates("reference")
+            hit = u != 0xFFFFFFFF
+            assert np.array_equal(u, uo) and hit.sum() > 100
+            assert np.array_equal(t[hit], to[hit]) and np.array_equal(nrm[hit], no[hit])
 
 
 @pytest.mark.parametrize("bad", [np.inf, -np.inf])
