@@ -528,11 +528,11 @@ __device__ __forceinline__ bool source_occluded_blk(const DevScene &sc, const ch
 // Direct rays towards sphere, sun-sphere, rectangle and disk sources (direct_raygen.comp:482-561): one
 // wave per (job, primitive), d*d stratified origins as k_direct, per-ray direction, strength and lit face,
 // per-lane closest-hit traversal.  Items [item_lo, item_lo + nitems) of jobs whose item_begin ascend.
-// BLK: over the block tree (every launch that does not count, unless the scene lacks one or its links are wide).  The binary tree's stacks take 32 or
-// 64 KB of LDS a workgroup, two waves a SIMD at 64, and its trace goes on to the closest hit; the block tree's take
-// RT_SRC_ROWS rows, 17 KB (24 rows: the same time), and four waves a SIMD fit.  Three lamps over 20,100 primitives x
-// 256 rays, the whole pass by pass solve: 9.29 to 8.57 ms.  The quadrature of a sphere's strength, 200 divisions a
-// ray, is the larger part of what is left.
+// BLK: over the block tree (every launch that does not count, unless the scene lacks one or its links are wide).  The
+// binary tree's stacks take 32 or 64 KB of LDS a workgroup, two waves a SIMD at 64, and its trace goes on to the closest
+// hit; the block tree's take RT_SRC_ROWS rows, 17 KB (24 rows: the same time), and four waves a SIMD fit.  Three lamps
+// over 20,100 primitives x 256 rays, the whole pass by pass solve: 9.29 to 8.57 ms.  The quadrature of a sphere's
+// strength, 200 divisions a ray, is the larger part of what is left.
 #ifndef RT_SRC_ROWS
 #define RT_SRC_ROWS 17
 #endif

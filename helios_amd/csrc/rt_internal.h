@@ -49,9 +49,9 @@ int check_work_items(uint64_t items, const char *what);
 int scene_build(Scene &S, uint32_t P, const float *T, const uint32_t *type, const uint32_t *uuid,
                 const uint32_t *twos, int px, int py, hipStream_t st);
 void scene_free(Scene &S);
-// Writes the block tree blk (rt_types.h; wide: with wide links) of nn4 BVH4 nodes over nleaf records, and into each node where its children
-// lie.  Returns 0, 1 when the scene is too large
-// for the nodes' steps (extents above 255 x 2^103: the traversals then walk the binary tree), or -1.
+// Writes the block tree blk (rt_types.h; wide: with wide links) of nn4 BVH4 nodes over nleaf records, and into each
+// node where its children lie.  Returns 0, 1 when the scene is too large for the nodes' steps (extents above
+// 255 x 2^103: the traversals then walk the binary tree), or -1.
 int write_blocks(uint32_t nn4, uint32_t nleaf, float4 *node4, const float4 *rec, uint4 *blk, bool wide,
                  hipStream_t st);
 // Texture masks (RayTracingGeometry mask_data / mask_sizes / mask_IDs / uv_data / uv_IDs,

@@ -920,11 +920,11 @@ __device__ __forceinline__ void keep_until(uint32_t offset, float &v) {
 // The step is written for the cycles of its vector instructions (see k_diffuse): fma, mul, add and bit operations
 // take 2.4 to 3.0 cycles of a SIMD here against 4.1 to 4.5 for min/max, compares, selects, shifts, permutes and
 // v_fma_mix and 4.7 for byte conversions (measured at 8 waves per SIMD).  So:
-// - a child bound q decodes in t-space as q (s / dir) + (o - ray origin) / dir with the axis' step s.  v_perm takes the bounds nearer
-//   the origin of two children from the lower or upper word (the ray's selector says which) as two half-precision
-//   numbers q 2^-24 (a byte under a zero byte is that denormal), and v_fma_mix multiplies and adds with the 2^24
-//   in the stored step: 36 instructions, 160 cycles, for the 24 bounds against 54 and 210 with selects, byte conversions and
-//   fma;
+// - a child bound q decodes in t-space as q (s / dir) + (o - ray origin) / dir with the axis' step s.  v_perm takes the
+//   bounds nearer the origin of two children from the lower or upper word (the ray's selector says which) as two
+//   half-precision numbers q 2^-24 (a byte under a zero byte is that denormal), and v_fma_mix multiplies and adds with
+//   the 2^24 in the stored step: 36 instructions, 160 cycles, for the 24 bounds against 54 and 210 with selects, byte
+//   conversions and fma;
 // - each hit child is one 32-bit key, the bits of its entry distance with the low byte replaced by its link code
 //   (v_perm), so the order of four children takes eight min / med / max and no selects of links, and a link is
 //   base + the key's low byte;
